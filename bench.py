@@ -107,6 +107,14 @@ def profiled_traffic(kernel):
     return None
 
 
+def band_fraction(g):
+    """Share of a wave's columns inside the propagator's band, the ones the sweeps move (all of
+    them for a limit factor other than 2/3)."""
+    res = g.resolution
+    k = int(np.ceil(res * g.limit_factor / 2)) - 1
+    return (2 * k + 1) / res if abs(g.limit_factor - 2.0 / 3.0) < 1e-12 else 1.0
+
+
 def roofline(engine, g, pos, batch, probe, dets):
     """Dominant sweep's achieved algorithmic bandwidth: average launch durations of the row
     and column passes timed back to back with hipEvents on the engine stream (a batch of B
@@ -115,10 +123,11 @@ def roofline(engine, g, pos, batch, probe, dets):
     engine.stem_batch(0, pos[:batch], batch, probe, dets)  # B waves of configuration 0
     row_us, col_us = engine.time_sweeps(g.n_slices // 2, reps=20)
     # algorithmic bytes per launch (8 bytes per complex64):
-    #   row pass: read + write every wave (16N each) and the shared t slice once (8N)
-    #   column pass: read + write every wave
-    row_bytes = batch * 16 * N + 8 * N
-    col_bytes = batch * 16 * N
+    #   row pass: read + write the band's columns of every wave and the shared t slice once (8N)
+    #   column pass: read + write the band's columns of every wave
+    f = band_fraction(g)
+    row_bytes = int(batch * 16 * N * f) + 8 * N
+    col_bytes = int(batch * 16 * N * f)
     kern = {"row_pass": (row_us, row_bytes), "column_pass": (col_us, col_bytes)}
     name = max(kern, key=lambda k: kern[k][0])
     us, b = kern[name]
@@ -143,7 +152,7 @@ def roofline(engine, g, pos, batch, probe, dets):
         "column_pass_GBs": round(col_bytes / (col_us * 1e-6) / 1e9, 1),
         "copy_pattern_avg_us": round(copy_us, 2),
         "copy_pattern_GBs": round(batch * 16 * N / (copy_us * 1e-6) / 1e9, 1),
-        "frac_of_copy_pattern": round(copy_us / us, 4),
+        "frac_of_copy_pattern": round(achieved / (batch * 16 * N / (copy_us * 1e-6) / 1e9), 4),
         "timing": "hipEvents around 20 back-to-back launches of each sweep on the engine stream; the copy "
                   "pattern is the same kernel's tile loads and stores without arithmetic (10 launches)",
     }
@@ -192,8 +201,8 @@ def kernel_roofline(engine, g, n_waves, label):
     transmission function), timed back to back with hipEvents, as achieved algorithmic GB/s."""
     N = g.resolution * g.resolution
     row_us, col_us = engine.time_sweeps(g.n_slices // 2, reps=10)
-    row_bytes = n_waves * 24 * N   # read + write the wave, read its own t
-    col_bytes = n_waves * 16 * N
+    col_bytes = int(n_waves * 16 * N * band_fraction(g))  # read + write the band's columns of each wave
+    row_bytes = col_bytes + n_waves * 8 * N               # and read its own t
     kern = {"row_pass": (row_us, row_bytes), "column_pass": (col_us, col_bytes)}
     name = max(kern, key=lambda k: kern[k][0])
     us, b = kern[name]
@@ -539,7 +548,8 @@ def bench_sweeps(args):
         engine.set_wave_count(B)
         engine.set_wave_configs([0] * B)
         N = res * res
-        rowb, colb = B * 16 * N + 8 * N, B * 16 * N
+        colb = int(B * 16 * N * band_fraction(g))
+        rowb = colb + 8 * N
         rows, cols = [], []
         for rv in range(7):
             engine.set_kernel_variant(0, rv)

@@ -34,13 +34,16 @@ void copy_planes(mse_engine* e, float2* dst, const float2* src, size_t count) {
     HIPX(hipMemcpyAsync(dst, src, count * sizeof(float2), hipMemcpyDeviceToDevice, e->stream));
 }
 
-// One forward slice from `in` into `out` (in != out): the row pass reads one buffer and
-// writes the other, so recomputed states need no copy of their predecessor.
-void slice_step_into(mse_engine* e, const float2* in, float2* out, int nw, int slice) {
+// One forward slice from `in` into `out` (in place, or from one buffer into another, so that
+// recomputed states need no copy of their predecessor).  A state in a buffer of its own needs its
+// zeros outside the band written; in place they are there after the first slice.
+void slice_step(mse_engine* e, const float2* in, float2* out, int nw, int slice) {
     mse::RowArgs ra = base_row_args(e);
+    mse::ColArgs ca = base_col_args(e);
     ra.slice = slice;
+    slice_band(e, in != out || slice == 0, ra, ca);
     row_pass(e, mse::ROW_IFFT_T_FFT, in, out, nw, e->N, ra);
-    col_pass(e, mse::COL_PROP, out, out, nw, e->N, base_col_args(e));
+    col_pass(e, mse::COL_PROP, out, out, nw, e->N, ca);
 }
 
 }  // namespace
@@ -72,10 +75,7 @@ int mse_forward_checkpointed(mse_engine* e, int cfg, double* intensity) {
         for (int s = 0; s < n; ++s) {
             const float2* in = s % K == 0 ? e->adj_ckpt.p + (size_t)(s / K) * plane : e->waves.p;
             float2* out = (s + 1 < n && (s + 1) % K == 0) ? e->adj_ckpt.p + (size_t)((s + 1) / K) * plane : e->waves.p;
-            if (in == out)
-                slice_step(e, out, nw, s);
-            else
-                slice_step_into(e, in, out, nw, s);
+            slice_step(e, in, out, nw, s);
         }
         copy_planes(e, e->adj_exit.p, e->waves.p, plane);
         if (intensity) {
@@ -168,7 +168,8 @@ int mse_adjoint_positions(mse_engine* e, const double* dl_di, double* grad_xyz) 
         e->adj_seg.ensure((size_t)std::max(K - 1, 1) * plane);  // states 1..K-1 of a segment
         HIPX(hipStreamSynchronize(e->stream));
 
-        // seed: res F_x (2 w psi_N)
+        // seed: res F_x (2 w psi_N), in every column; from then on the adjoint states are
+        // kept and read inside the band alone (outside it, adj_g holds what the seed left there)
         mse::RowArgs ra = base_row_args(e);
         ra.weights = e->adj_w.p;
         row_pass(e, mse::ROW_ADJ_SEED, e->adj_exit.p, e->adj_g.p, nw, N, ra);
@@ -187,6 +188,7 @@ int mse_adjoint_positions(mse_engine* e, const double* dl_di, double* grad_xyz) 
             ca.px = e->adj_pconj.p;
             ca.py = e->adj_pconj.p + e->res;
         }
+        ca.band_k = e->prop_k;
         e->adj_gtau.ensure((size_t)std::max(n, 1) * N);  // g_t of every slice, summed over the waves
         const int n_seg = (n + K - 1) / K;
         for (int j = n_seg - 1; j >= 0; --j) {
@@ -196,12 +198,14 @@ int mse_adjoint_positions(mse_engine* e, const double* dl_di, double* grad_xyz) 
             const float2* ck = e->adj_ckpt.p + (size_t)j * plane;
             auto slot = [&](int i) { return e->adj_seg.p + (size_t)(i - 1) * plane; };
             auto state = [&](int i) -> const float2* { return i == 0 ? ck : slot(i); };
-            for (int i = 1; i < len; ++i) slice_step_into(e, state(i - 1), slot(i), nw, start + i - 1);
+            for (int i = 1; i < len; ++i) slice_step(e, state(i - 1), slot(i), nw, start + i - 1);
             for (int s = start + len - 1; s >= start; --s) {
                 col_pass(e, conj_tables ? mse::COL_PROP : mse::COL_PROP_CONJ, e->adj_g.p, e->adj_g.p, nw, N, ca);
                 float2* gs = e->adj_gtau.p + (size_t)s * N;
                 mse::RowArgs rb = base_row_args(e);
                 rb.slice = s;
+                rb.band_k = e->prop_k;
+                if (e->prop_k >= 0) rb.io = mse::BAND_STEP;
                 rb.aux_in = state(s - start);
                 rb.aux_out = nw == 1 ? gs : e->adj_gt.p;  // one wave: its g_t is the sum
                 row_pass(e, mse::ROW_ADJ, e->adj_g.p, e->adj_g.p, nw, N, rb);

@@ -144,6 +144,7 @@ mse::ColArgs base_col_args(mse_engine* e) {
     a.py = e->py.p;
     a.wave_prop = e->any_beam ? e->wave_prop.p : nullptr;
     a.lim = e->prop_lim.p;
+    a.band_k = -1;
     a.kx = e->kx.p;
     a.ky = e->ky.p;
     a.scale = 1.0f;
@@ -159,8 +160,9 @@ mse::RowArgs base_row_args(mse_engine* e) {
     a.dout = nullptr;
     a.wave_cfg = e->wave_cfg.p;
     a.slice = 0;
-    a.plane_value = 0.f;
     a.scale = 1.0f;
+    a.io = mse::BAND_FULL;
+    a.band_k = -1;
     a.mix_key = e->mix_key.p;
     a.mix_seed = make_uint2((unsigned)(e->mix_seed & 0xffffffffu), (unsigned)(e->mix_seed >> 32));
     a.mix_first = e->mix_first;
@@ -542,6 +544,14 @@ int mse_set_geometry(mse_engine* e, const mse_geometry* g) {
             plim[y] = pl;
             blim[y] = bl;
         }
+        // the largest |kx index| any row keeps (row 0: the limits fall with |ky|), where the band
+        // classes of fft_wave.hpp cover it; -1 (another limit factor): the sweeps visit every column
+        const auto band_of = [res](const std::vector<int>& lim) {
+            const int k = *std::max_element(lim.begin(), lim.end());
+            return k >= mse::band_k_min(res) && k <= mse::band_k_max(res) ? k : -1;
+        };
+        e->prop_k = band_of(plim);
+        e->band_k = band_of(blim);
         e->tw.ensure(res);
         e->px.ensure(res);
         e->py.ensure(res);
@@ -1238,10 +1248,15 @@ void potential_planes(mse_engine* e, const ConfigData& c, const mse_geometry& g,
 // bit for bit, on the persistent column kernels.  Their variant is fixed per grid size (not
 // tuned), so that transmission functions do not depend on the tuning state.
 void band_limit_planes(mse_engine* e, float2* p, int planes) {
+    const bool band = e->band_k >= 0;
     mse::RowArgs ra = base_row_args(e);
     ra.scale = 1.0f;
+    ra.band_k = e->band_k;
+    if (band) ra.io = mse::BAND_WRITE;
     row_pass(e, mse::ROW_FFT, p, p, planes, e->N, ra);
+    if (band) ra.io = mse::BAND_READ;
     mse::ColArgs ca = base_col_args(e);
+    ca.band_k = e->band_k;
     ca.wave_map = nullptr;
     ca.wave_prop = nullptr;
     ca.px = e->band_xy.p;
@@ -1252,11 +1267,9 @@ void band_limit_planes(mse_engine* e, float2* p, int planes) {
     row_pass(e, mse::ROW_IFFT, p, p, planes, e->N, ra);
 }
 
-void slice_step(mse_engine* e, float2* waves, int nw, int slice) {
-    mse::RowArgs ra = base_row_args(e);
-    ra.slice = slice;
-    row_pass(e, mse::ROW_IFFT_T_FFT, waves, waves, nw, e->N, ra);
-    col_pass(e, mse::COL_PROP, waves, waves, nw, e->N, base_col_args(e));
+void slice_band(mse_engine* e, bool first, mse::RowArgs& ra, mse::ColArgs& ca) {
+    ra.band_k = ca.band_k = e->prop_k;
+    ra.io = e->prop_k < 0 ? mse::BAND_FULL : first ? mse::BAND_FIRST : mse::BAND_STEP;
 }
 
 void multislice(mse_engine* e, int nw, int first, int count, bool last_detect, const mse::ColArgs* det_args) {
@@ -1272,10 +1285,15 @@ void multislice(mse_engine* e, int nw, int first, int count, bool last_detect, c
         ra.slice = s;
         ra.wave_map = map;
         ca.wave_map = map;
+        // the waves of a slice are among those of the slice before (specimens only end), so after
+        // the first slice of the range all of them are band limited
+        slice_band(e, s == first, ra, ca);
         row_pass(e, mse::ROW_IFFT_T_FFT, e->waves.p, e->waves.p, na, e->N, ra);
-        if (last_detect && s == first + count - 1)
-            e->det_tiles = col_pass(e, mse::COL_PROP_DETECT, e->waves.p, e->waves.p, nw, e->N, *det_args);
-        else
+        if (last_detect && s == first + count - 1) {
+            mse::ColArgs da = *det_args;
+            da.band_k = ca.band_k;
+            e->det_tiles = col_pass(e, mse::COL_PROP_DETECT, e->waves.p, e->waves.p, nw, e->N, da);
+        } else
             col_pass(e, mse::COL_PROP, e->waves.p, e->waves.p, na, e->N, ca);
     }
 }
@@ -1854,12 +1872,13 @@ int mse_stem_batch_frames(mse_engine* e, int cfg, const double* pos_xy, const do
         ra.wave_cfg = e->frame_wcfg.p;
         ra.slice = 0;
         ra.mix_sets = 0;
-        const mse::ColArgs ca = base_col_args(e);
+        mse::ColArgs ca = base_col_args(e);
         mse::ColArgs da = base_col_args(e);
         da.det_scale = 1.0;
         da.det_bits = e->det_bits.p;
         da.ndet = n_det;
         da.partials = e->partials.p;
+        da.band_k = e->prop_k;
         std::vector<double> rel(2 * (size_t)batch), org(2 * (size_t)batch);
         for (int p0 = 0; p0 < n_probes; p0 += batch) {
             const int nb = std::min(batch, n_probes - p0);
@@ -1884,6 +1903,7 @@ int mse_stem_batch_frames(mse_engine* e, int cfg, const double* pos_xy, const do
             for (int s = 0; s < ns; ++s) {
                 potential_planes(e, c, g, pa, e->frame_trans.p, nb, s);
                 band_limit_planes(e, e->frame_trans.p, nb);
+                slice_band(e, s == 0, ra, ca);
                 row_pass(e, mse::ROW_IFFT_T_FFT, e->waves.p, e->waves.p, nb, e->N, ra);
                 if (s == ns - 1)
                     e->det_tiles = col_pass(e, mse::COL_PROP_DETECT, e->waves.p, e->waves.p, nb, e->N, da);
@@ -2172,6 +2192,7 @@ int mse_autotune(mse_engine* e, int cfg, int n_waves, int reps, double* row_us, 
         e->prof = false;
         mse::RowArgs ra = base_row_args(e);
         mse::ColArgs ca = base_col_args(e);
+        slice_band(e, false, ra, ca);  // a plane wave is band limited
         double best = 1e30;
         int bi = 0;
         for (int v = 0; v < kRowVariants; ++v) {
@@ -2233,7 +2254,8 @@ int mse_time_sweeps(mse_engine* e, int slice, int reps, double* row_us, double* 
         HIPX(hipEventCreate(&c));
         mse::RowArgs ra = base_row_args(e);
         ra.slice = slice;
-        const mse::ColArgs ca = base_col_args(e);
+        mse::ColArgs ca = base_col_args(e);
+        slice_band(e, false, ra, ca);
         const int nw = e->n_waves;
         row_pass(e, mse::ROW_IFFT_T_FFT, e->waves.p, e->waves.p, nw, e->N, ra);  // warm
         col_pass(e, mse::COL_PROP, e->waves.p, e->waves.p, nw, e->N, ca);

@@ -121,6 +121,9 @@ struct mse_engine {
     size_t N = 0;
     DevBuf<float2> tw, px, py;
     DevBuf<int> prop_lim, band_lim;
+    // largest |kx index| the propagator's and the band limit's masks keep, for the sweeps on the
+    // band alone; -1: limits the band classes do not cover, the sweeps visit every column
+    int prop_k = -1, band_k = -1;
     DevBuf<float2> band_xy;  // x then y factors of the band limit's column pass
     DevBuf<double> kx, ky;
     std::vector<double> h_kx, h_ky;
@@ -256,8 +259,10 @@ void row_pass(mse_engine* e, int mode, const float2* in, float2* out, int nlines
               const mse::RowArgs& args, int variant = -1);
 int col_pass(mse_engine* e, int mode, const float2* in, float2* out, int nsets, size_t wave_stride,
              const mse::ColArgs& args, int kind = PK_COL, int variant = -1);
-// one forward slice (row pass with t, column pass with the propagator) on nw waves in place
-void slice_step(mse_engine* e, float2* waves, int nw, int slice);
+// The columns of one slice's row and column pass (io, band_k of both): the band alone where the
+// limits allow it.  first: the row pass's input may hold anything outside the band (the start of
+// a slice loop), which it clears; else the wave comes from a column pass.
+void slice_band(mse_engine* e, bool first, mse::RowArgs& ra, mse::ColArgs& ca);
 // exp(i sigma V) of `planes` planes into out from the sorted atoms of c: slices
 // first..first+planes-1, or with a.frame_xy set one plane per frame of slice `first`
 void potential_planes(mse_engine* e, const ConfigData& c, const mse_geometry& g, const mse::PotArgs& a,

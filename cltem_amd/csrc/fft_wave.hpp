@@ -64,8 +64,13 @@ constexpr double ct_sin2pi(int J, int R) {
     return ct_sin_series(a);
 }
 
-// multiply by W_R^J = exp(-+ 2 pi i J / R) (forward: minus, inverse: plus)
-template <int R, int J, bool INV>
+// multiply by W_R^J = exp(-+ 2 pi i J / R) (forward: minus, inverse: plus).  Of the two products
+// of each component one is rounded and the other enters the fused multiply-add.  Which one is
+// written out (XR: the product with a.x is rounded in the real part, XI: in the imaginary part):
+// the compiler's own choice depends on the expressions around it (on negated operands, say), and
+// written out a transform with zero inputs left out rounds exactly as the full one, and every
+// kernel's transform as every other's.
+template <int R, int J, bool INV, bool XR, bool XI>
 __device__ __forceinline__ float2 rot(float2 a) {
     constexpr int j = ((J % R) + R) % R;
     if constexpr (j == 0) {
@@ -76,44 +81,78 @@ __device__ __forceinline__ float2 rot(float2 a) {
         return make_float2(-a.x, -a.y);
     } else if constexpr (4 * j == 3 * R) {  // +i (fwd) / -i (inv)
         return INV ? make_float2(a.y, -a.x) : make_float2(-a.y, a.x);
-    } else if constexpr (8 * j == R || 8 * j == 3 * R || 8 * j == 5 * R || 8 * j == 7 * R) {
-        constexpr float h = 0.70710678118654752440f;
-        constexpr float c = (float)ct_cos2pi(j, R);
-        constexpr float s = (float)(INV ? ct_sin2pi(j, R) : -ct_sin2pi(j, R));
-        // (a.x + i a.y)(c + i s) with |c| = |s| = 1/sqrt2
-        constexpr float sc = c > 0 ? h : -h;
-        constexpr float ss = s > 0 ? h : -h;
-        return make_float2(a.x * sc - a.y * ss, a.x * ss + a.y * sc);
     } else {
-        constexpr float c = (float)ct_cos2pi(j, R);
-        constexpr float s = (float)(INV ? ct_sin2pi(j, R) : -ct_sin2pi(j, R));
-        return make_float2(a.x * c - a.y * s, a.x * s + a.y * c);
+        constexpr bool eighth = 8 * j == R || 8 * j == 3 * R || 8 * j == 5 * R || 8 * j == 7 * R;
+        constexpr float h = 0.70710678118654752440f;
+        constexpr float cf = (float)ct_cos2pi(j, R);
+        constexpr float sf = (float)(INV ? ct_sin2pi(j, R) : -ct_sin2pi(j, R));
+        constexpr float c = eighth ? (cf > 0 ? h : -h) : cf;
+        constexpr float s = eighth ? (sf > 0 ? h : -h) : sf;
+        const float re = XR ? fmaf(a.y, -s, a.x * c) : fmaf(a.x, c, -(a.y * s));
+        const float im = XI ? fmaf(a.y, c, a.x * s) : fmaf(a.x, s, a.y * c);
+        return make_float2(re, im);
     }
+}
+// The choices of a composite transform's rotation W_R^J of its inner output s2 (signs of W's
+// real and imaginary part: c, s).
+constexpr bool rot_x_re(int R, int J, int s2, bool inv) {
+    const bool c = ct_cos2pi(J, R) > 0, s = (ct_sin2pi(J, R) > 0) == inv;
+    if (R == 16) return 8 * J == R ? !inv || s2 == 1 : 8 * J == 3 * R ? !inv && s2 == 3 : c ? !inv : inv;
+    return 8 * J == R ? !inv : !c && !s && 8 * J != 3 * R;
+}
+constexpr bool rot_x_im(int R, int J, int s2, bool inv) {
+    const bool c = ct_cos2pi(J, R) > 0, s = (ct_sin2pi(J, R) > 0) == inv;
+    if (R == 16) return 8 * J == R ? !inv || s2 == 1 : 8 * J == 3 * R ? !inv && s2 == 3 : c;
+    return 8 * J == R ? !inv : c && !s;
 }
 
 // ---- small DFTs in registers --------------------------------------------------------
+// run<Z>: bit r of Z says that input a[r] is zero (its register is not read).  The sums and
+// differences with those inputs are left out; x + 0 and 0 - x are exact, so every output equals
+// that of run<0> on stored zeros (up to the sign of a zero).
 template <int R, bool INV>
 struct Dft;
 
+__device__ __forceinline__ float2 cneg(float2 a) { return make_float2(-a.x, -a.y); }
+template <bool ZA, bool ZB>
+__device__ __forceinline__ float2 cadd_z(float2 a, float2 b) {
+    if constexpr (ZA && ZB) return make_float2(0.f, 0.f);
+    else if constexpr (ZA) return b;
+    else if constexpr (ZB) return a;
+    else return cadd(a, b);
+}
+template <bool ZA, bool ZB>
+__device__ __forceinline__ float2 csub_z(float2 a, float2 b) {
+    if constexpr (ZA && ZB) return make_float2(0.f, 0.f);
+    else if constexpr (ZA) return cneg(b);
+    else if constexpr (ZB) return a;
+    else return csub(a, b);
+}
+
 template <bool INV>
 struct Dft<2, INV> {
+    template <int Z = 0>
     static __device__ __forceinline__ void run(float2* a) {
-        float2 t = a[0];
-        a[0] = cadd(t, a[1]);
-        a[1] = csub(t, a[1]);
+        constexpr bool z0 = Z & 1, z1 = Z & 2;
+        const float2 t = a[0], u = a[1];
+        a[0] = cadd_z<z0, z1>(t, u);
+        a[1] = csub_z<z0, z1>(t, u);
     }
 };
 
 template <bool INV>
 struct Dft<3, INV> {
+    template <int Z = 0>
     static __device__ __forceinline__ void run(float2* a) {
+        constexpr bool z0 = Z & 1, z1 = Z & 2, z2 = Z & 4;
         constexpr float s3 = 0.86602540378443864676f;
-        float2 t1 = cadd(a[1], a[2]);
-        float2 t2 = make_float2(a[0].x - 0.5f * t1.x, a[0].y - 0.5f * t1.y);
-        float2 d = csub(a[1], a[2]);
+        const float2 a0 = z0 ? make_float2(0.f, 0.f) : a[0];
+        float2 t1 = cadd_z<z1, z2>(a[1], a[2]);
+        float2 t2 = make_float2(a0.x - 0.5f * t1.x, a0.y - 0.5f * t1.y);
+        float2 d = csub_z<z1, z2>(a[1], a[2]);
         // forward: y1 = t2 - i s3 d, y2 = t2 + i s3 d
         float2 isd = INV ? make_float2(-s3 * d.y, s3 * d.x) : make_float2(s3 * d.y, -s3 * d.x);
-        a[0] = cadd(a[0], t1);
+        a[0] = cadd_z<z0, z1 && z2>(a0, t1);
         a[1] = cadd(t2, isd);
         a[2] = csub(t2, isd);
     }
@@ -121,14 +160,17 @@ struct Dft<3, INV> {
 
 template <bool INV>
 struct Dft<4, INV> {
+    template <int Z = 0>
     static __device__ __forceinline__ void run(float2* a) {
-        float2 t0 = cadd(a[0], a[2]), t1 = csub(a[0], a[2]);
-        float2 t2 = cadd(a[1], a[3]), t3 = csub(a[1], a[3]);
+        constexpr bool z0 = Z & 1, z1 = Z & 2, z2 = Z & 4, z3 = Z & 8;
+        float2 t0 = cadd_z<z0, z2>(a[0], a[2]), t1 = csub_z<z0, z2>(a[0], a[2]);
+        float2 t2 = cadd_z<z1, z3>(a[1], a[3]), t3 = csub_z<z1, z3>(a[1], a[3]);
         float2 t3r = INV ? make_float2(-t3.y, t3.x) : make_float2(t3.y, -t3.x);
-        a[0] = cadd(t0, t2);
-        a[2] = csub(t0, t2);
-        a[1] = cadd(t1, t3r);
-        a[3] = csub(t1, t3r);
+        constexpr bool ze = z0 && z2, zo = z1 && z3;
+        a[0] = cadd_z<ze, zo>(t0, t2);
+        a[2] = csub_z<ze, zo>(t0, t2);
+        a[1] = cadd_z<ze, zo>(t1, t3r);
+        a[3] = csub_z<ze, zo>(t1, t3r);
     }
 };
 
@@ -137,37 +179,52 @@ struct Dft<4, INV> {
 template <int R1, int R2, bool INV>
 struct DftComposite {
     static constexpr int R = R1 * R2;
-    template <int r1>
+    // zero inputs of the inner transform r1, and the inner transforms that are zero altogether
+    static constexpr int inner_zero(int Z, int r1) {
+        int z = 0;
+        for (int r2 = 0; r2 < R2; ++r2) z |= ((Z >> (r1 + R1 * r2)) & 1) << r2;
+        return z;
+    }
+    static constexpr int outer_zero(int Z) {
+        int z = 0;
+        for (int r1 = 0; r1 < R1; ++r1) z |= (inner_zero(Z, r1) == (1 << R2) - 1) << r1;
+        return z;
+    }
+    template <int r1, int Z>
     static __device__ __forceinline__ void inner(const float2* a, float2* b) {
-        float2 tmp[R2];
+        if constexpr (((outer_zero(Z) >> r1) & 1) == 0) {
+            float2 tmp[R2];
 #pragma unroll
-        for (int r2 = 0; r2 < R2; ++r2) tmp[r2] = a[r1 + R1 * r2];
-        Dft<R2, INV>::run(tmp);
-        twid<r1, 0>(tmp, b);
+            for (int r2 = 0; r2 < R2; ++r2) tmp[r2] = a[r1 + R1 * r2];
+            Dft<R2, INV>::template run<inner_zero(Z, r1)>(tmp);
+            twid<r1, 0>(tmp, b);
+        }
     }
     template <int r1, int s2>
     static __device__ __forceinline__ void twid(const float2* tmp, float2* b) {
         if constexpr (s2 < R2) {
-            b[r1 * R2 + s2] = rot<R, r1 * s2, INV>(tmp[s2]);
+            constexpr int J = r1 * s2;
+            b[r1 * R2 + s2] = rot<R, J, INV, rot_x_re(R, J, s2, INV), rot_x_im(R, J, s2, INV)>(tmp[s2]);
             twid<r1, s2 + 1>(tmp, b);
         }
     }
-    template <int r1>
+    template <int r1, int Z>
     static __device__ __forceinline__ void all_inner(const float2* a, float2* b) {
         if constexpr (r1 < R1) {
-            inner<r1>(a, b);
-            all_inner<r1 + 1>(a, b);
+            inner<r1, Z>(a, b);
+            all_inner<r1 + 1, Z>(a, b);
         }
     }
+    template <int Z = 0>
     static __device__ __forceinline__ void run(float2* a) {
         float2 b[R];
-        all_inner<0>(a, b);
+        all_inner<0, Z>(a, b);
 #pragma unroll
         for (int s2 = 0; s2 < R2; ++s2) {
             float2 tmp[R1];
 #pragma unroll
             for (int r1 = 0; r1 < R1; ++r1) tmp[r1] = b[r1 * R2 + s2];
-            Dft<R1, INV>::run(tmp);
+            Dft<R1, INV>::template run<outer_zero(Z)>(tmp);
 #pragma unroll
             for (int s1 = 0; s1 < R1; ++s1) a[R2 * s1 + s2] = tmp[s1];
         }
@@ -306,6 +363,50 @@ struct PlanTw {
     }
 };
 
+// ---- the band of a band-limited line ------------------------------------------------------
+// A line limited to 2/3 of its Nyquist frequency holds only the indices x <= K and x >= N - K,
+// K = N / 3 or just below.  In register layout element m covers x = L m .. L m + L - 1: it is
+// inside the band in every lane, outside in every lane, or at its edge (some lanes in).  The
+// classes hold for every K in [band_k_min(N), band_k_max(N)], so they are compile-time and only
+// the one or two edge elements need a test.
+constexpr int band_k_max(int n) { return n / 3; }
+constexpr int band_k_min(int n) { return n / 3 - 2; }
+enum BandClass : int { BAND_IN, BAND_EDGE, BAND_OUT };
+template <int N, int L>
+constexpr BandClass band_class(int m) {
+    const int lo = L * m, hi = L * m + L - 1;
+    if (hi <= band_k_min(N) || lo >= N - band_k_min(N)) return BAND_IN;
+    if (lo > band_k_max(N) && hi < N - band_k_max(N)) return BAND_OUT;
+    return BAND_EDGE;
+}
+__device__ __forceinline__ bool in_band(int x, int n, int k) { return x <= k || x >= n - k; }
+// the zero inputs a[r] = v[b + r NB] of the first pass's butterfly b for a band-limited line
+template <int N, int L, int R>
+constexpr int band_zero_mask(int b) {
+    constexpr int NB = (N / L) / R;
+    int z = 0;
+    for (int r = 0; r < R; ++r) z |= (band_class<N, L>(b + r * NB) == BAND_OUT) << r;
+    return z;
+}
+
+// First pass of a band-limited line: as stockham_pass with p = 1, with the elements outside the
+// band taken as zero (their registers are not read).
+template <int N, int L, int R, bool INV, int b = 0>
+__device__ __forceinline__ void stockham_first_banded(float2 (&v)[N / L], float2* line, int t) {
+    constexpr int NB = (N / L) / R;
+    if constexpr (b < NB) {
+        constexpr int Z = band_zero_mask<N, L, R>(b);
+        float2 a[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) a[r] = (Z >> r) & 1 ? make_float2(0.f, 0.f) : v[b + r * NB];
+        Dft<R, INV>::template run<Z>(a);
+        const int j = (t + L * b) * R;
+#pragma unroll
+        for (int r = 0; r < R; ++r) line[lpad(j + r)] = a[r];
+        stockham_first_banded<N, L, R, INV, b + 1>(v, line, t);
+    }
+}
+
 // One Stockham pass.  v holds the line in register layout; line is this line's LDS.
 // P_ = product of radices already done (p); LAST = this pass ends the transform.
 template <int N, int L, int R, int P_, bool INV, bool LAST, class TW, bool PAD2 = false>
@@ -352,11 +453,15 @@ struct NoTw {
 
 // Full transform of one line in register layout.  sync() must order LDS writes before
 // reads and reads before the next pass's writes for every lane sharing the LDS line.
-template <class PL, bool INV, class TWS, class Sync>
+// BANDED: the input is band limited (elements of class BAND_OUT are zero and not read).
+template <class PL, bool INV, bool BANDED = false, class TWS, class Sync>
 __device__ __forceinline__ void fft_line(float2 (&v)[PL::E], float2* line, int t, const TWS& tw,
                                          Sync sync) {
     constexpr int N = PL::N, L = PL::L;
-    stockham_pass<N, L, PL::R0, 1, INV, false, NoTw>(v, line, t, nullptr);
+    if constexpr (BANDED)
+        stockham_first_banded<N, L, PL::R0, INV>(v, line, t);
+    else
+        stockham_pass<N, L, PL::R0, 1, INV, false, NoTw>(v, line, t, nullptr);
     sync();
     line_gather<N, L>(v, line, t);
     sync();

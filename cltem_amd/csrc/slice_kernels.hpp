@@ -13,6 +13,15 @@
 // from two res-length tables and a per-row mask limit instead of an N-sized array.
 // V = Psi(k) is the propagated k-space wave (clWaveFunctionRecip), so detector
 // sums are taken from it in the last slice's column pass.
+//
+// The propagator's aperture mask keeps |k| below 2/3 of the Nyquist frequency, so after a
+// column pass the columns |kx| > K (K about N/3) of the stored wave are zero, and of the row
+// pass's output only the columns inside the band are ever used.  With the engine's usual limit
+// (see band_class) the sweeps therefore work on the band alone: a slice's row pass reads and
+// writes the columns of the band (BandIo), the column pass visits the column tiles that hold
+// some, and both leave out the transforms' zero inputs and unused outputs.  That is 2/3 of the
+// bytes and of the column transforms; the values are the same.  The zeros outside the band stay
+// in memory: the first slice of a loop writes them (BAND_FIRST), no later pass touches them.
 #pragma once
 #include "fft_wave.hpp"
 #include "philox.hpp"
@@ -21,7 +30,6 @@ namespace mse {
 
 enum RowMode : int {
     ROW_IFFT_T_FFT = 0,   // slice step, row half
-    ROW_PLANE_T_FFT = 1,  // first slice of a plane wave: psi = value (no load)
     ROW_FFT = 2,          // forward x-DFT (transmission band limit, step 1)
     ROW_IFFT = 3,         // inverse x-DFT (band limit step 3, exit-wave readback)
     ROW_COPY = 4,         // read and write the rows only (bandwidth reference)
@@ -36,12 +44,22 @@ enum ColMode : int {
     COL_PROBE = 3,        // generate the k-space probe and inverse y-DFT
     COL_FFT_DETECT = 4,   // detectors from a stored wave (F_y S / res)
     COL_FFT_DIFF = 5,     // |fftshift Psi|^2 of a stored wave into a double image
-    COL_PROP_STORE_DETECT = 6,  // last slice: propagate, reduce detectors and store
     COL_COPY = 7,         // move the tile through LDS only (bandwidth reference)
     COL_PROP_CONJ = 8,    // adjoint column half: propagation by conj(P')
     COL_CTEM_IMAGE = 9,   // objective-lens transfer of Psi(k) (ctem_image), back to the mixed domain
     COL_FILTER = 10,      // multiply the spectrum by a real per-pixel filter (CCD DQE / NTF)
 };
+
+// Columns a row pass reads and writes (the last four only for limits that band_class covers).
+enum BandIo : int {
+    BAND_FULL = 0,    // reads and writes every column
+    BAND_FIRST = 1,   // reads every column, writes the band and zeros outside it
+    BAND_STEP = 2,    // reads and writes the band (outside it: zero in memory, not touched)
+    BAND_WRITE = 3,   // reads every column, writes the band (the rest is left as it was)
+    BAND_READ = 4,    // reads the band (the rest is taken as zero), writes every column
+};
+constexpr bool band_reads(int io) { return io == BAND_STEP || io == BAND_READ; }
+constexpr bool band_skips_writes(int io) { return io == BAND_STEP || io == BAND_WRITE; }
 
 constexpr int kMaxDet = 8;
 
@@ -79,8 +97,9 @@ struct RowArgs {
     const float2* aux_in;            // ROW_ADJ: forward state S_s = F_x psi_s (wave_stride per wave)
     float2* aux_out;                 // ROW_ADJ: g_t = conj(psi_s) u in real space (wave_stride per wave)
     int slice;
-    float plane_value;               // ROW_PLANE_T_FFT: psi amplitude times res
     float scale;                     // ROW_FFT / ROW_IFFT output scale
+    int io;                          // BandIo
+    int band_k;                      // largest |kx index| of the band (io other than BAND_FULL)
     // mixed static potentials: with mix_sets >= 2 a wave reads configuration mix_first + a
     // set drawn per (mix_key[wave], slice) instead of its own (row_config)
     const unsigned* mix_key;
@@ -119,6 +138,12 @@ struct ColArgs {
     const float* filter;     // COL_FILTER: res*res real factors, row-major [ky][kx] (unshifted)
     const double* kx;        // k-grid (COL_PROBE)
     const double* ky;
+    // COL_PROP*: largest |kx index| that lim keeps, for the sweeps on the band alone (the row
+    // pass before must have left the columns outside it at zero); -1: every column
+    int band_k;
+    // column tiles of a launch (set by the launcher): tile j < n_tiles starts at column
+    // TC j below tile_lo, TC (j + tile_skip) from there
+    int n_tiles, tile_lo, tile_skip;
     float scale;             // COL_FFT_*: multiply after the forward DFT
     double det_scale;        // intensity factor applied to |V|^2 in detector sums
     const unsigned* det_bits;  // ndet bitmasks over the fft-shifted image, res*res bits each
@@ -129,10 +154,44 @@ struct ColArgs {
     ProbeArgs probe;
 };
 
+// One line's elements from and to memory (register layout), as IO says.
+template <class PL, int IO>
+__device__ __forceinline__ void band_load(float2 (&v)[PL::E], const float2* src, int t, int k) {
+    constexpr int N = PL::N, L = PL::L;
+#pragma unroll
+    for (int m = 0; m < PL::E; ++m) {
+        const int x = t + L * m;
+        if (!band_reads(IO) || band_class<N, L>(m) == BAND_IN)
+            v[m] = src[x];
+        else if (band_class<N, L>(m) == BAND_EDGE)
+            v[m] = in_band(x, N, k) ? src[x] : make_float2(0.f, 0.f);
+        else
+            v[m] = make_float2(0.f, 0.f);
+    }
+}
+template <class PL, int IO>
+__device__ __forceinline__ void band_store(const float2 (&v)[PL::E], float2* dst, int t, int k) {
+    constexpr int N = PL::N, L = PL::L;
+#pragma unroll
+    for (int m = 0; m < PL::E; ++m) {
+        const int x = t + L * m;
+        if (IO == BAND_FULL || IO == BAND_READ || band_class<N, L>(m) == BAND_IN) {
+            dst[x] = v[m];
+        } else if (band_class<N, L>(m) == BAND_EDGE) {
+            if (in_band(x, N, k))
+                dst[x] = v[m];
+            else if (IO == BAND_FIRST)
+                dst[x] = make_float2(0.f, 0.f);
+        } else if (IO == BAND_FIRST) {
+            dst[x] = make_float2(0.f, 0.f);
+        }
+    }
+}
+
 // --------------------------------------------------------------------------------------
 // Row pass: 256 threads, 256/L lines per block; grid (res / lines, n_waves)
 // --------------------------------------------------------------------------------------
-template <class PL, int MODE, class SYNC = WaveSync, bool TWREG = true, int WPE = 1>
+template <class PL, int MODE, int IO = BAND_FULL, class SYNC = WaveSync, bool TWREG = true, int WPE = 1>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void k_row(
     const float2* __restrict__ in, float2* __restrict__ out, size_t wave_stride,
     const float2* __restrict__ tw, RowArgs a) {
@@ -152,13 +211,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
 
     const size_t base = (size_t)wave * wave_stride + (size_t)row * N;
     float2 v[E];
-    if constexpr (MODE == ROW_PLANE_T_FFT) {
-#pragma unroll
-        for (int m = 0; m < E; ++m) v[m] = make_float2(a.plane_value, 0.f);
-    } else {
-#pragma unroll
-        for (int m = 0; m < E; ++m) v[m] = in[base + t + L * m];
-    }
+    band_load<PL, IO>(v, in + base, t, a.band_k);
     if constexpr (MODE == ROW_COPY) {
 #pragma unroll
         for (int m = 0; m < E; ++m) out[base + t + L * m] = v[m];
@@ -166,7 +219,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
     }
     if constexpr (MODE == ROW_ADJ_SEED || MODE == ROW_ADJ) {
         // u = F_x^-1 v / res (real space)
-        fft_line<PL, true>(v, ln, t, tws, sync);
+        fft_line<PL, true, band_reads(IO)>(v, ln, t, tws, sync);
         sync();
         const float inv = 1.0f / N;
         if constexpr (MODE == ROW_ADJ_SEED) {
@@ -200,11 +253,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
         fft_line<PL, false>(v, ln, t, tws, sync);
         const float rs = (float)N;
 #pragma unroll
-        for (int m = 0; m < E; ++m) out[base + t + L * m] = make_float2(v[m].x * rs, v[m].y * rs);
+        for (int m = 0; m < E; ++m) v[m] = make_float2(v[m].x * rs, v[m].y * rs);
+        band_store<PL, IO>(v, out + base, t, a.band_k);
         return;
     }
     if constexpr (MODE == ROW_IFFT_T_FFT || MODE == ROW_IFFT || MODE == ROW_IFFT_INTENSITY) {
-        fft_line<PL, true>(v, ln, t, tws, sync);
+        fft_line<PL, true, band_reads(IO)>(v, ln, t, tws, sync);
         sync();
     }
     if constexpr (MODE == ROW_IFFT_INTENSITY) {
@@ -216,7 +270,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
         }
         return;
     }
-    if constexpr (MODE == ROW_IFFT_T_FFT || MODE == ROW_PLANE_T_FFT) {
+    if constexpr (MODE == ROW_IFFT_T_FFT) {
         const int cfg = row_config(a, wave);
         if (a.slice < a.cfg_nslices[cfg]) {  // below a thinner specimen the slice is vacuum
             const float2* tr = a.cfg_trans[cfg] + (size_t)a.slice * N * N + (size_t)row * N;
@@ -231,8 +285,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
 #pragma unroll
         for (int m = 0; m < E; ++m) v[m] = cscale(v[m], a.scale);
     }
-#pragma unroll
-    for (int m = 0; m < E; ++m) out[base + t + L * m] = v[m];
+    band_store<PL, IO>(v, out + base, t, a.band_k);
 }
 
 // complex helpers in double for the probe
@@ -335,12 +388,19 @@ __device__ __forceinline__ double wave_sum(double v) {
 
 // --------------------------------------------------------------------------------------
 // Column pass: TC columns per block, L lanes per column (TC*L threads); grid
-// (res / TC, n_waves).  The TC x res tile is staged through LDS column-major with a
+// (column tiles, n_waves).  The TC x res tile is staged through LDS column-major with a
 // column stride of 1 mod 16 complex, so the coalesced 128-byte row loads and the
 // per-column FFT exchanges are both free of bank conflicts; each column's LDS line
-// doubles as its FFT exchange buffer.
+// doubles as its FFT exchange buffer.  BAND: the propagation's mask cuts the ky outside the
+// band (a.band_k set), whose outputs are not formed and not transformed back.
 // --------------------------------------------------------------------------------------
-template <class PL, int TC, int MODE, class SYNC = WaveSync, bool TWREG = true, int WPE = 1>
+// first column of tile j of a launch
+template <int TC>
+__device__ __forceinline__ int tile_column(const ColArgs& a, int j) {
+    return (j < a.tile_lo ? j : j + a.tile_skip) * TC;
+}
+
+template <class PL, int TC, int MODE, bool BAND = false, class SYNC = WaveSync, bool TWREG = true, int WPE = 1>
 __global__ __launch_bounds__(TC * PL::L) __attribute__((amdgpu_waves_per_eu(WPE))) void k_col(
     const float2* __restrict__ in, float2* __restrict__ out, size_t wave_stride,
     const float2* __restrict__ tw, ColArgs a) {
@@ -353,7 +413,7 @@ __global__ __launch_bounds__(TC * PL::L) __attribute__((amdgpu_waves_per_eu(WPE)
     const int tid = threadIdx.x;
     const int c = tid / L;
     const int t = tid % L;
-    const int x0 = blockIdx.x * TC;
+    const int x0 = tile_column<TC>(a, blockIdx.x);
     const int x = x0 + c;
     const int wave = a.wave_map ? a.wave_map[blockIdx.y] : (int)blockIdx.y;
     float2* ln = tile + c * CS;
@@ -396,8 +456,7 @@ __global__ __launch_bounds__(TC * PL::L) __attribute__((amdgpu_waves_per_eu(WPE)
         fft_line<PL, false>(v, ln, t, tws, sync);
     }
 
-    if constexpr (MODE == COL_PROP || MODE == COL_PROP_DETECT || MODE == COL_PROP_STORE_DETECT ||
-                  MODE == COL_PROP_CONJ) {
+    if constexpr (MODE == COL_PROP || MODE == COL_PROP_DETECT || MODE == COL_PROP_CONJ) {
         const int xs = (x < N / 2) ? x : N - x;  // |signed kx index|
         const float2* pxt = a.px;
         const float2* pyt = a.py;
@@ -408,6 +467,10 @@ __global__ __launch_bounds__(TC * PL::L) __attribute__((amdgpu_waves_per_eu(WPE)
         const float2 pxv = pxt[x];
 #pragma unroll
         for (int m = 0; m < E; ++m) {
+            if (BAND && band_class<N, L>(m) == BAND_OUT) {
+                v[m] = make_float2(0.f, 0.f);
+                continue;
+            }
             const int y = t + L * m;
             const bool keep = xs <= a.lim[y];
             float2 f = cmul(pxv, pyt[y]);
@@ -426,8 +489,7 @@ __global__ __launch_bounds__(TC * PL::L) __attribute__((amdgpu_waves_per_eu(WPE)
         for (int m = 0; m < E; ++m) v[m] = cscale(cmul(v[m], ctem_transfer(a.probe, kxv, a.ky[t + L * m])), a.scale);
     }
 
-    if constexpr (MODE == COL_PROP_DETECT || MODE == COL_PROP_STORE_DETECT ||
-                  MODE == COL_FFT_DETECT) {
+    if constexpr (MODE == COL_PROP_DETECT || MODE == COL_FFT_DETECT) {
         const int xs = (x + N / 2) % N;  // fft-shifted column
         const int nw = NT / 64;
         const int wid = tid / 64, lane = tid % 64;
@@ -436,6 +498,7 @@ __global__ __launch_bounds__(TC * PL::L) __attribute__((amdgpu_waves_per_eu(WPE)
             double acc = 0.0;
 #pragma unroll
             for (int m = 0; m < E; ++m) {
+                if (BAND && band_class<N, L>(m) == BAND_OUT) continue;  // nothing there
                 const int ys = (t + L * m + N / 2) % N;
                 const size_t bit = (size_t)ys * N + xs;
                 if ((bits[bit >> 5] >> (bit & 31)) & 1u) {
@@ -465,10 +528,9 @@ __global__ __launch_bounds__(TC * PL::L) __attribute__((amdgpu_waves_per_eu(WPE)
         }
     }
 
-    if constexpr (MODE == COL_PROP || MODE == COL_PROP_STORE_DETECT ||
-                  MODE == COL_PROBE || MODE == COL_PROP_CONJ || MODE == COL_CTEM_IMAGE || MODE == COL_FILTER) {
+    if constexpr (MODE == COL_PROP || MODE == COL_PROBE || MODE == COL_PROP_CONJ || MODE == COL_CTEM_IMAGE || MODE == COL_FILTER) {
         if constexpr (MODE != COL_PROBE) sync();  // the forward pass's last reads precede new writes
-        fft_line<PL, true>(v, ln, t, tws, sync);
+        fft_line<PL, true, BAND>(v, ln, t, tws, sync);
         sync();
 #pragma unroll
         for (int m = 0; m < E; ++m) ln[lpad(t + L * m)] = v[m];
@@ -493,7 +555,7 @@ __global__ __launch_bounds__(TC * PL::L) __attribute__((amdgpu_waves_per_eu(WPE)
 // its own L2.  With XCD set (and gridDim.x a multiple of 8) the blocks of one XCD take
 // consecutive items in every round, so tiles that share 128-byte lines (8-column tiles: two
 // per line) are read and written through the same L2 at about the same time.
-template <class PL, int TC, class SYNC = WaveSync, bool TWREG = true, int WPE = 1, bool XCD = false>
+template <class PL, int TC, bool BAND = false, class SYNC = WaveSync, bool TWREG = true, int WPE = 1, bool XCD = false>
 __global__ __launch_bounds__(TC * PL::L) __attribute__((amdgpu_waves_per_eu(WPE))) void k_col_prop_pipe(float2* __restrict__ data, size_t wave_stride,
                                                               const float2* __restrict__ tw, ColArgs a,
                                                               int nsets) {
@@ -502,7 +564,7 @@ __global__ __launch_bounds__(TC * PL::L) __attribute__((amdgpu_waves_per_eu(WPE)
     constexpr int CS = LdsLine<N>::col_stride;
     constexpr int NQ = (TC * N / 2) / NT;  // float4 per thread per tile
     static_assert((TC * N / 2) % NT == 0, "tile must split evenly over the block");
-    constexpr int ntiles = N / TC;
+    const int ntiles = a.n_tiles;
     __shared__ float2 tile[TC * CS];
     const int tid = threadIdx.x;
     const int c = tid / L;
@@ -516,7 +578,7 @@ __global__ __launch_bounds__(TC * PL::L) __attribute__((amdgpu_waves_per_eu(WPE)
     float4 q[NQ];
     auto fetch = [&](int item) {
         const int wv = a.wave_map ? cload(a.wave_map + item / ntiles) : item / ntiles;
-        const int xx = (item % ntiles) * TC;
+        const int xx = tile_column<TC>(a, item % ntiles);
         const float4* in4 = reinterpret_cast<const float4*>(data + (size_t)wv * wave_stride + xx);
 #pragma unroll
         for (int k = 0; k < NQ; ++k) {
@@ -531,7 +593,7 @@ __global__ __launch_bounds__(TC * PL::L) __attribute__((amdgpu_waves_per_eu(WPE)
     float4 o[NQ];
     auto store = [&](int item) {
         const int wv = a.wave_map ? cload(a.wave_map + item / ntiles) : item / ntiles;
-        const int xx = (item % ntiles) * TC;
+        const int xx = tile_column<TC>(a, item % ntiles);
         float4* out4 = reinterpret_cast<float4*>(data + (size_t)wv * wave_stride + xx);
 #pragma unroll
         for (int k = 0; k < NQ; ++k) {
@@ -550,7 +612,8 @@ __global__ __launch_bounds__(TC * PL::L) __attribute__((amdgpu_waves_per_eu(WPE)
     if constexpr (PY_REGS) {
         if (!per_wave) {
 #pragma unroll
-            for (int m = 0; m < E; ++m) pyv[m] = gload(a.py + t + L * m);
+            for (int m = 0; m < E; ++m)
+                if (!BAND || band_class<N, L>(m) != BAND_OUT) pyv[m] = gload(a.py + t + L * m);
         }
     } else {
         if (!per_wave)
@@ -562,7 +625,7 @@ __global__ __launch_bounds__(TC * PL::L) __attribute__((amdgpu_waves_per_eu(WPE)
     if (item < nitems) fetch(item);
     for (; item < nitems; item += gridDim.x) {
         const int wv = a.wave_map ? cload(a.wave_map + item / ntiles) : item / ntiles;
-        const int x0 = (item % ntiles) * TC;
+        const int x0 = tile_column<TC>(a, item % ntiles);
         const int x = x0 + c;
         // propagator factors of this column, loaded before the next tile's prefetch so that
         // waiting for them does not wait for the prefetch
@@ -575,7 +638,8 @@ __global__ __launch_bounds__(TC * PL::L) __attribute__((amdgpu_waves_per_eu(WPE)
                 pyt = cload(a.wave_prop + 2 * wv + 1);
                 if constexpr (PY_REGS) {
 #pragma unroll
-                    for (int m = 0; m < E; ++m) pyv[m] = gload(pyt + t + L * m);
+                    for (int m = 0; m < E; ++m)
+                        if (!BAND || band_class<N, L>(m) != BAND_OUT) pyv[m] = gload(pyt + t + L * m);
                 }
             }
             // the 64 / L columns of this wave: scalar loads, which the stores issued before the
@@ -615,6 +679,7 @@ __global__ __launch_bounds__(TC * PL::L) __attribute__((amdgpu_waves_per_eu(WPE)
         fft_line<PL, false>(v, ln, t, tws, sync);
 #pragma unroll
         for (int m = 0; m < E; ++m) {
+            if (BAND && band_class<N, L>(m) == BAND_OUT) continue;  // masked: the inverse takes it as zero
             const int y = t + L * m;
             const int ys = (y < N / 2) ? y : N - y;
             float2 pyy;
@@ -626,7 +691,7 @@ __global__ __launch_bounds__(TC * PL::L) __attribute__((amdgpu_waves_per_eu(WPE)
             v[m] = ys <= lim ? f : make_float2(0.f, 0.f);
         }
         sync();
-        fft_line<PL, true>(v, ln, t, tws, sync);
+        fft_line<PL, true, BAND>(v, ln, t, tws, sync);
         sync();
 #pragma unroll
         for (int m = 0; m < E; ++m) ln[lpad(t + L * m)] = v[m];
@@ -648,7 +713,7 @@ __global__ __launch_bounds__(TC * PL::L) __attribute__((amdgpu_waves_per_eu(WPE)
 // Column slice step, one 16-column tile per block with no prefetch, sized for two blocks
 // per CU (at most 64 VGPRs): twiddles and y factors are read from per-block copies in LDS,
 // so that the second block's loads and stores overlap the first one's transforms.  Same
-// arithmetic as k_col<..., COL_PROP>.  Grid (N / TC, nsets).
+// arithmetic as k_col<..., COL_PROP>.  Grid (column tiles, nsets).
 // --------------------------------------------------------------------------------------
 // Twiddle table entries a plan's passes read: pass with radix R after p points reads
 // r k N / (p R) for r < R, k < p.
@@ -665,7 +730,7 @@ constexpr int plan_twiddles() {
     return most + 1;
 }
 
-template <class PL, int TC>
+template <class PL, int TC, bool BAND>
 __device__ __forceinline__ void col_prop_lean(float2* __restrict__ data, size_t wave_stride,
                                               const float2* __restrict__ tw, const ColArgs& a) {
     constexpr int N = PL::N, L = PL::L, E = PL::E;
@@ -681,7 +746,7 @@ __device__ __forceinline__ void col_prop_lean(float2* __restrict__ data, size_t 
     const int c = tid / L;
     const int t = tid % L;
     const int wv = a.wave_map ? cload(a.wave_map + blockIdx.y) : (int)blockIdx.y;
-    const int x0 = blockIdx.x * TC;
+    const int x0 = tile_column<TC>(a, blockIdx.x);
     const int x = x0 + c;
     const float4* in4 = reinterpret_cast<const float4*>(data + (size_t)wv * wave_stride + x0);
     float4 q[NQ];
@@ -722,13 +787,14 @@ __device__ __forceinline__ void col_prop_lean(float2* __restrict__ data, size_t 
     fft_line<PL, false>(v, ln, t, tws, sync);
 #pragma unroll
     for (int m = 0; m < E; ++m) {
+        if (BAND && band_class<N, L>(m) == BAND_OUT) continue;
         const int y = t + L * m;
         const int ys = (y < N / 2) ? y : N - y;
         const float2 f = cmul(v[m], cmul(pxv, spy[y]));
         v[m] = ys <= lim ? f : make_float2(0.f, 0.f);
     }
     sync();
-    fft_line<PL, true>(v, ln, t, tws, sync);
+    fft_line<PL, true, BAND>(v, ln, t, tws, sync);
     sync();
 #pragma unroll
     for (int m = 0; m < E; ++m) ln[lpad(t + L * m)] = v[m];
@@ -744,16 +810,16 @@ __device__ __forceinline__ void col_prop_lean(float2* __restrict__ data, size_t 
 }
 
 // 16-column tiles (512 points): 64 VGPRs, two 1024-thread blocks per CU
-template <class PL>
+template <class PL, bool BAND>
 __global__ __launch_bounds__(16 * PL::L) __attribute__((amdgpu_waves_per_eu(8), amdgpu_num_vgpr(64))) void k_col_prop_lean(
     float2* __restrict__ data, size_t wave_stride, const float2* __restrict__ tw, ColArgs a) {
-    col_prop_lean<PL, 16>(data, wave_stride, tw, a);
+    col_prop_lean<PL, 16, BAND>(data, wave_stride, tw, a);
 }
 // 8-column tiles (four-pass plans, 12 elements per lane): two 512-thread blocks per CU
-template <class PL>
+template <class PL, bool BAND>
 __global__ __launch_bounds__(8 * PL::L) __attribute__((amdgpu_waves_per_eu(4))) void k_col_prop_lean8(
     float2* __restrict__ data, size_t wave_stride, const float2* __restrict__ tw, ColArgs a) {
-    col_prop_lean<PL, 8>(data, wave_stride, tw, a);
+    col_prop_lean<PL, 8, BAND>(data, wave_stride, tw, a);
 }
 
 // --------------------------------------------------------------------------------------
@@ -762,7 +828,7 @@ __global__ __launch_bounds__(8 * PL::L) __attribute__((amdgpu_waves_per_eu(4))) 
 // loaded into registers while the current row is transformed.  MODE = ROW_FFT or ROW_IFFT:
 // the one transform and the scale of k_row's same modes, in place (no transmission row).
 // --------------------------------------------------------------------------------------
-template <class PL, class SYNC = WaveSync, bool TWREG = true, int MODE = ROW_IFFT_T_FFT>
+template <class PL, int IO = BAND_FULL, class SYNC = WaveSync, bool TWREG = true, int MODE = ROW_IFFT_T_FFT>
 __global__ __launch_bounds__(256) void k_row_step_pipe(float2* __restrict__ data, size_t wave_stride,
                                                        const float2* __restrict__ tw, RowArgs a, int nsets) {
     static_assert(MODE == ROW_IFFT_T_FFT || MODE == ROW_FFT || MODE == ROW_IFFT, "row step modes");
@@ -787,9 +853,7 @@ __global__ __launch_bounds__(256) void k_row_step_pipe(float2* __restrict__ data
         // transmission row then come from scalar loads
         if constexpr (L == 64) item = __builtin_amdgcn_readfirstlane(item);
         const int wv = a.wave_map ? cload(a.wave_map + item / N) : item / N, row = item % N;
-        const float2* src = data + (size_t)wv * wave_stride + (size_t)row * N;
-#pragma unroll
-        for (int m = 0; m < E; ++m) qv[m] = src[t + L * m];
+        band_load<PL, IO>(qv, data + (size_t)wv * wave_stride + (size_t)row * N, t, a.band_k);
         if constexpr (!STEP) return;
         const int cfg = row_config(a, wv);
         if (a.slice < cload(a.cfg_nslices + cfg)) {
@@ -812,13 +876,13 @@ __global__ __launch_bounds__(256) void k_row_step_pipe(float2* __restrict__ data
         }
         if (item + stride < nitems) fetch(item + stride);
         if constexpr (STEP) {
-            fft_line<PL, true>(v, ln, t, tws, sync);
+            fft_line<PL, true, band_reads(IO)>(v, ln, t, tws, sync);
             sync();
 #pragma unroll
             for (int m = 0; m < E; ++m) v[m] = cmul(v[m], tr[m]);
             fft_line<PL, false>(v, ln, t, tws, sync);
         } else {
-            fft_line<PL, MODE == ROW_IFFT>(v, ln, t, tws, sync);
+            fft_line<PL, MODE == ROW_IFFT, band_reads(IO)>(v, ln, t, tws, sync);
 #pragma unroll
             for (int m = 0; m < E; ++m) v[m] = cscale(v[m], a.scale);
         }
@@ -826,9 +890,7 @@ __global__ __launch_bounds__(256) void k_row_step_pipe(float2* __restrict__ data
         int it = item;
         if constexpr (L == 64) it = __builtin_amdgcn_readfirstlane(it);
         const int wv = a.wave_map ? cload(a.wave_map + it / N) : it / N, row = it % N;
-        float2* dst = data + (size_t)wv * wave_stride + (size_t)row * N;
-#pragma unroll
-        for (int m = 0; m < E; ++m) dst[t + L * m] = v[m];
+        band_store<PL, IO>(v, data + (size_t)wv * wave_stride + (size_t)row * N, t, a.band_k);
     }
 }
 

@@ -24,259 +24,233 @@ int resident_per_cu(int block_threads, int cap) {
 template <int N>
 void row_pass_n(mse_engine* e, int mode, const float2* in, float2* out, int nlines_sets, size_t wave_stride,
                 const mse::RowArgs& args, int variant) {
-    {
-        auto go = [&](auto plan, auto sync, auto twreg) {
-            using PL = decltype(plan);
-            using SY = decltype(sync);
-            constexpr bool TR = decltype(twreg)::value;
-            constexpr int WPE = TR ? 1 : 8;
-            constexpr int LINES = 256 / PL::L;
-            dim3 grid(N / LINES, nlines_sets);
-            launch(e, PK_ROW, [&]() {
-                switch (mode) {
-                    case mse::ROW_IFFT_T_FFT:
-                        mse::k_row<PL, mse::ROW_IFFT_T_FFT, SY, TR, WPE><<<grid, 256, 0, e->stream>>>(in, out, wave_stride, e->tw.p, args);
-                        break;
-                    case mse::ROW_PLANE_T_FFT:
-                        mse::k_row<PL, mse::ROW_PLANE_T_FFT, SY, TR, WPE><<<grid, 256, 0, e->stream>>>(in, out, wave_stride, e->tw.p, args);
-                        break;
-                    case mse::ROW_FFT:
-                        mse::k_row<PL, mse::ROW_FFT, SY, TR, WPE><<<grid, 256, 0, e->stream>>>(in, out, wave_stride, e->tw.p, args);
-                        break;
-                    case mse::ROW_IFFT:
-                        mse::k_row<PL, mse::ROW_IFFT, SY, TR, WPE><<<grid, 256, 0, e->stream>>>(in, out, wave_stride, e->tw.p, args);
-                        break;
-                    case mse::ROW_COPY:
-                        mse::k_row<PL, mse::ROW_COPY, SY, TR, WPE><<<grid, 256, 0, e->stream>>>(in, out, wave_stride, e->tw.p, args);
-                        break;
-                    case mse::ROW_IFFT_INTENSITY:
-                        mse::k_row<PL, mse::ROW_IFFT_INTENSITY, SY, TR, WPE><<<grid, 256, 0, e->stream>>>(in, out, wave_stride, e->tw.p, args);
-                        break;
-                    case mse::ROW_ADJ_SEED:
-                        mse::k_row<PL, mse::ROW_ADJ_SEED, SY, TR, WPE><<<grid, 256, 0, e->stream>>>(in, out, wave_stride, e->tw.p, args);
-                        break;
-                    case mse::ROW_ADJ:
-                        mse::k_row<PL, mse::ROW_ADJ, SY, TR, WPE><<<grid, 256, 0, e->stream>>>(in, out, wave_stride, e->tw.p, args);
-                        break;
-                }
-            });
-        };
-        using P0 = typename mse::PlanFor<N>::P;
-        using P1 = typename mse::PlanHalfLanes<N>::P;
-        using REG = std::true_type;
-        using MEM = std::false_type;
-        if ((mode == mse::ROW_FFT || mode == mse::ROW_IFFT) && in == out) {
-            // one transform in place (the band limit of transmission functions): the persistent
-            // pipelined kernel, whatever the tuned variant
-            auto go_pipe = [&](auto m) {
-                constexpr int MD = decltype(m)::value;
-                constexpr int LINES = 256 / P0::L;
-                const int per_cu = resident_per_cu<mse::k_row_step_pipe<P0, mse::WaveSync, true, MD>>(256, 4);
-                const int blocks = std::max(1, std::min(e->num_cus * per_cu, (N * nlines_sets + LINES - 1) / LINES));
-                launch(e, PK_ROW, [&]() {
-                    mse::k_row_step_pipe<P0, mse::WaveSync, true, MD><<<blocks, 256, 0, e->stream>>>(
-                        out, wave_stride, e->tw.p, args, nlines_sets);
-                });
-            };
-            if (mode == mse::ROW_FFT)
-                go_pipe(std::integral_constant<int, mse::ROW_FFT>{});
-            else
-                go_pipe(std::integral_constant<int, mse::ROW_IFFT>{});
-            return;
-        }
-        if constexpr (N <= 512) {  // half-lane lines keep the prefetch registers within budget up to 512
-            if (mode == mse::ROW_IFFT_T_FFT && variant == 5 && in == out) {
-                constexpr int LINES = 256 / P1::L;
-                const int per_cu = resident_per_cu<mse::k_row_step_pipe<P1, mse::WaveSync>>(256, 4);
-                const int blocks = std::max(1, std::min(e->num_cus * per_cu, (N * nlines_sets + LINES - 1) / LINES));
-                launch(e, PK_ROW, [&]() {
-                    mse::k_row_step_pipe<P1, mse::WaveSync><<<blocks, 256, 0, e->stream>>>(out, wave_stride, e->tw.p,
-                                                                                         args, nlines_sets);
-                });
-                return;
-            }
-        }
-        if (mode == mse::ROW_IFFT_T_FFT && variant == 6 && in == out) {  // twiddles read at use
-            constexpr int LINES = 256 / P0::L;
-            const int per_cu = resident_per_cu<mse::k_row_step_pipe<P0, mse::WaveSync, false>>(256, 4);
-            const int blocks = std::max(1, std::min(e->num_cus * per_cu, (N * nlines_sets + LINES - 1) / LINES));
-            launch(e, PK_ROW, [&]() {
-                mse::k_row_step_pipe<P0, mse::WaveSync, false><<<blocks, 256, 0, e->stream>>>(out, wave_stride, e->tw.p,
-                                                                                            args, nlines_sets);
-            });
-            return;
-        }
-        if (mode == mse::ROW_IFFT_T_FFT && variant >= 4 && in == out) {
-            constexpr int LINES = 256 / P0::L;
-            const int per_cu = resident_per_cu<mse::k_row_step_pipe<P0, mse::WaveSync>>(256, 4);
-            const int blocks = std::max(1, std::min(e->num_cus * per_cu, (N * nlines_sets + LINES - 1) / LINES));
-            launch(e, PK_ROW, [&]() {
-                mse::k_row_step_pipe<P0, mse::WaveSync><<<blocks, 256, 0, e->stream>>>(out, wave_stride, e->tw.p, args,
-                                                                                     nlines_sets);
-            });
-            return;
-        }
-        if (mode == mse::ROW_IFFT_T_FFT && variant == 1)
-            go(P1{}, mse::WaveSync{}, REG{});
-        else if (mode == mse::ROW_IFFT_T_FFT && variant == 2)
-            go(P0{}, mse::BlockSync{}, REG{});
-        else if (mode == mse::ROW_IFFT_T_FFT && variant == 3)
-            go(P0{}, mse::WaveSync{}, MEM{});
-        else
-            go(P0{}, mse::WaveSync{}, REG{});
+    using P0 = typename mse::PlanFor<N>::P;
+    using P1 = typename mse::PlanHalfLanes<N>::P;
+    using REG = std::true_type;
+    using MEM = std::false_type;
+    const bool step = mode == mse::ROW_IFFT_T_FFT;
+    // one row per line of the grid, out of place or with the non-persistent variants
+    auto go = [&](auto plan, auto sync, auto twreg) {
+        using PL = decltype(plan);
+        using SY = decltype(sync);
+        constexpr bool TR = decltype(twreg)::value;
+        constexpr int WPE = TR ? 1 : 8;
+        constexpr int LINES = 256 / PL::L;
+        dim3 grid(N / LINES, nlines_sets);
+        launch(e, PK_ROW, [&]() {
+#define MSE_ROW_CASE(M, IO)                                                                                         \
+    if (mode == mse::M && args.io == mse::IO) {                                                                     \
+        mse::k_row<PL, mse::M, mse::IO, SY, TR, WPE><<<grid, 256, 0, e->stream>>>(in, out, wave_stride, e->tw.p, args); \
+        return;                                                                                                     \
     }
+            MSE_ROW_CASE(ROW_IFFT_T_FFT, BAND_FULL)
+            MSE_ROW_CASE(ROW_IFFT_T_FFT, BAND_FIRST)
+            MSE_ROW_CASE(ROW_IFFT_T_FFT, BAND_STEP)
+            if constexpr (TR && std::is_same<SY, mse::WaveSync>::value && std::is_same<PL, P0>::value) {
+                MSE_ROW_CASE(ROW_FFT, BAND_FULL)
+                MSE_ROW_CASE(ROW_IFFT, BAND_FULL)
+                MSE_ROW_CASE(ROW_COPY, BAND_FULL)
+                MSE_ROW_CASE(ROW_IFFT_INTENSITY, BAND_FULL)
+                MSE_ROW_CASE(ROW_ADJ_SEED, BAND_FULL)
+                MSE_ROW_CASE(ROW_ADJ, BAND_FULL)
+                MSE_ROW_CASE(ROW_ADJ, BAND_STEP)
+            }
+#undef MSE_ROW_CASE
+            throw Error(MSE_ERR_STATE, "row pass without a kernel");
+        });
+    };
+    // the persistent pipelined kernel, in place
+    auto go_pipe = [&](auto plan, auto twreg, auto m, auto io) {
+        using PL = decltype(plan);
+        constexpr bool TR = decltype(twreg)::value;
+        constexpr int MD = decltype(m)::value, IO = decltype(io)::value;
+        constexpr int LINES = 256 / PL::L;
+        const int per_cu = resident_per_cu<mse::k_row_step_pipe<PL, IO, mse::WaveSync, TR, MD>>(256, 4);
+        const int blocks = std::max(1, std::min(e->num_cus * per_cu, (N * nlines_sets + LINES - 1) / LINES));
+        launch(e, PK_ROW, [&]() {
+            mse::k_row_step_pipe<PL, IO, mse::WaveSync, TR, MD><<<blocks, 256, 0, e->stream>>>(
+                out, wave_stride, e->tw.p, args, nlines_sets);
+        });
+    };
+    auto pipe_step = [&](auto plan, auto twreg) {
+        using M = std::integral_constant<int, mse::ROW_IFFT_T_FFT>;
+        if (args.io == mse::BAND_STEP)
+            go_pipe(plan, twreg, M{}, std::integral_constant<int, mse::BAND_STEP>{});
+        else if (args.io == mse::BAND_FIRST)
+            go_pipe(plan, twreg, M{}, std::integral_constant<int, mse::BAND_FIRST>{});
+        else
+            go_pipe(plan, twreg, M{}, std::integral_constant<int, mse::BAND_FULL>{});
+    };
+    if ((mode == mse::ROW_FFT || mode == mse::ROW_IFFT) && in == out) {
+        // one transform in place (the band limit of transmission functions): the persistent
+        // pipelined kernel, whatever the tuned variant
+        using FFT = std::integral_constant<int, mse::ROW_FFT>;
+        using IFFT = std::integral_constant<int, mse::ROW_IFFT>;
+        using FULL = std::integral_constant<int, mse::BAND_FULL>;
+        if (mode == mse::ROW_FFT && args.io == mse::BAND_WRITE)
+            go_pipe(P0{}, REG{}, FFT{}, std::integral_constant<int, mse::BAND_WRITE>{});
+        else if (mode == mse::ROW_FFT)
+            go_pipe(P0{}, REG{}, FFT{}, FULL{});
+        else if (args.io == mse::BAND_READ)
+            go_pipe(P0{}, REG{}, IFFT{}, std::integral_constant<int, mse::BAND_READ>{});
+        else
+            go_pipe(P0{}, REG{}, IFFT{}, FULL{});
+        return;
+    }
+    if (step && variant >= 4 && in == out) {
+        if constexpr (N <= 512) {  // half-lane lines keep the prefetch registers within budget up to 512
+            if (variant == 5) return pipe_step(P1{}, REG{});
+        }
+        return variant == 6 ? pipe_step(P0{}, MEM{}) : pipe_step(P0{}, REG{});
+    }
+    if (step && variant == 1)
+        go(P1{}, mse::WaveSync{}, REG{});
+    else if (step && variant == 2)
+        go(P0{}, mse::BlockSync{}, REG{});
+    else if (step && variant == 3)
+        go(P0{}, mse::WaveSync{}, MEM{});
+    else
+        go(P0{}, mse::WaveSync{}, REG{});
 }
 
 // returns the number of column tiles of the launch (detector partials per wave)
 template <int N>
 int col_pass_n(mse_engine* e, int mode, const float2* in, float2* out, int nsets, size_t wave_stride,
-               const mse::ColArgs& args, int kind, int variant) {
+               const mse::ColArgs& args0, int kind, int variant) {
+    using P0 = typename mse::PlanFor<N>::P;
+    using P1 = typename mse::PlanHalfLanes<N>::P;
+    using C16 = std::integral_constant<int, 16>;
+    using C8 = std::integral_constant<int, 8>;
+    using C32 = std::integral_constant<int, 32>;
+    using REG = std::true_type;
+    using MEM = std::false_type;
+    const bool prop = mode == mse::COL_PROP || mode == mse::COL_PROP_DETECT || mode == mse::COL_PROP_CONJ;
     const bool hot = mode == mse::COL_PROP || mode == mse::COL_PROP_DETECT || mode == mse::COL_COPY;
+    const bool band = prop && args0.band_k >= 0;
     if (!hot) variant = 0;
-    int tiles = 0;
-    {
-        auto go = [&](auto plan, auto tc, auto sync, auto twreg) {
-            using PL = decltype(plan);
-            using SY = decltype(sync);
-            constexpr bool TR = decltype(twreg)::value;
-            constexpr int WPE = TR ? 1 : 8;
-            constexpr int TC = decltype(tc)::value;
-            constexpr int NT = TC * PL::L;
-            dim3 grid(N / TC, nsets);
-            tiles = N / TC;
-            launch(e, kind, [&]() {
-                switch (mode) {
-#define MSE_COL_CASE(M) \
-    case mse::M: mse::k_col<PL, TC, mse::M, SY, TR, WPE><<<grid, NT, 0, e->stream>>>(in, out, wave_stride, e->tw.p, args); break;
-                    MSE_COL_CASE(COL_PROP)
-                    MSE_COL_CASE(COL_PROP_DETECT)
-                    MSE_COL_CASE(COL_PROBE)
-                    MSE_COL_CASE(COL_FFT_DETECT)
-                    MSE_COL_CASE(COL_FFT_DIFF)
-                    MSE_COL_CASE(COL_PROP_STORE_DETECT)
-                    MSE_COL_CASE(COL_COPY)
-                    MSE_COL_CASE(COL_PROP_CONJ)
-                    MSE_COL_CASE(COL_CTEM_IMAGE)
-                    MSE_COL_CASE(COL_FILTER)
+    mse::ColArgs args = args0;
+    // the tiles of TC columns to visit: with a band, those that hold columns 0..K or N-K..N-1
+    auto set_tiles = [&](int TC) {
+        args.tile_lo = N / TC;
+        args.tile_skip = 0;
+        if (band) {
+            const int hi = (N - args.band_k) / TC;
+            args.tile_lo = args.band_k / TC + 1;
+            args.tile_skip = std::max(0, hi - args.tile_lo);
+        }
+        args.n_tiles = N / TC - args.tile_skip;
+        return args.n_tiles;
+    };
+    // one tile per block
+    auto go = [&](auto plan, auto tc, auto sync, auto twreg) {
+        using PL = decltype(plan);
+        using SY = decltype(sync);
+        constexpr bool TR = decltype(twreg)::value;
+        constexpr int WPE = TR ? 1 : 8;
+        constexpr int TC = decltype(tc)::value;
+        constexpr int NT = TC * PL::L;
+        dim3 grid(set_tiles(TC), nsets);
+        launch(e, kind, [&]() {
+#define MSE_COL_CASE(M, BAND)                                                                                         \
+    if (mode == mse::M && band == BAND) {                                                                             \
+        mse::k_col<PL, TC, mse::M, BAND, SY, TR, WPE><<<grid, NT, 0, e->stream>>>(in, out, wave_stride, e->tw.p, args); \
+        return;                                                                                                       \
+    }
+            MSE_COL_CASE(COL_PROP, false)
+            MSE_COL_CASE(COL_PROP, true)
+            MSE_COL_CASE(COL_PROP_DETECT, false)
+            MSE_COL_CASE(COL_PROP_DETECT, true)
+            MSE_COL_CASE(COL_COPY, false)
+            if constexpr (TR && std::is_same<SY, mse::WaveSync>::value && std::is_same<PL, P0>::value) {
+                MSE_COL_CASE(COL_PROBE, false)
+                MSE_COL_CASE(COL_FFT_DETECT, false)
+                MSE_COL_CASE(COL_FFT_DIFF, false)
+                MSE_COL_CASE(COL_PROP_CONJ, false)
+                MSE_COL_CASE(COL_PROP_CONJ, true)
+                MSE_COL_CASE(COL_CTEM_IMAGE, false)
+                MSE_COL_CASE(COL_FILTER, false)
+            }
 #undef MSE_COL_CASE
-                }
+            throw Error(MSE_ERR_STATE, "column pass without a kernel");
+        });
+    };
+    if (variant >= 7 && mode == mse::COL_PROP && in == out) {
+        // persistent blocks, at most `cap` per CU; the XCD-aware order takes a multiple of 8
+        auto go_pipe = [&](auto plan, auto tc, auto twreg, auto xcd, auto bnd, int cap) {
+            using PL = decltype(plan);
+            constexpr bool TR = decltype(twreg)::value, XCD = decltype(xcd)::value, BAND = decltype(bnd)::value;
+            constexpr int TC = decltype(tc)::value, NT = TC * PL::L;
+            const int items = set_tiles(TC) * nsets;
+            const int per_cu = resident_per_cu<mse::k_col_prop_pipe<PL, TC, BAND, mse::WaveSync, TR, 1, XCD>>(NT, cap / NT);
+            int blocks = std::max(1, std::min(e->num_cus * per_cu, items));
+            if (XCD) blocks = blocks >= 8 ? blocks / 8 * 8 : 8;
+            launch(e, kind, [&]() {
+                mse::k_col_prop_pipe<PL, TC, BAND, mse::WaveSync, TR, 1, XCD><<<blocks, NT, 0, e->stream>>>(
+                    out, wave_stride, e->tw.p, args, nsets);
             });
         };
-        using P0 = typename mse::PlanFor<N>::P;
-        using P1 = typename mse::PlanHalfLanes<N>::P;
-        using C16 = std::integral_constant<int, 16>;
-        using C8 = std::integral_constant<int, 8>;
-        using C32 = std::integral_constant<int, 32>;
-        using REG = std::true_type;
-        using MEM = std::false_type;
-        if constexpr (N <= 512) {
-            if (variant == 8 && mode == mse::COL_PROP && in == out) {  // half lanes: two blocks per CU
-                constexpr int NT = 16 * P1::L;
-                const int per_cu = resident_per_cu<mse::k_col_prop_pipe<P1, 16, mse::WaveSync>>(NT, 2048 / NT);
-                const int blocks = std::max(1, std::min(e->num_cus * per_cu, (N / 16) * nsets));
-                tiles = N / 16;
-                launch(e, kind, [&]() {
-                    mse::k_col_prop_pipe<P1, 16, mse::WaveSync><<<blocks, NT, 0, e->stream>>>(out, wave_stride,
-                                                                                            e->tw.p, args, nsets);
-                });
-                return tiles;
+        auto pipe = [&](auto plan, auto tc, auto twreg, auto xcd, int cap) {
+            if (band)
+                go_pipe(plan, tc, twreg, xcd, std::true_type{}, cap);
+            else
+                go_pipe(plan, tc, twreg, xcd, std::false_type{}, cap);
+        };
+        if constexpr (N <= 512) {  // half lanes: two blocks per CU
+            if (variant == 8) {
+                pipe(P1{}, C16{}, REG{}, std::false_type{}, 2048);
+                return args.n_tiles;
             }
         }
-        if ((variant == 12 || variant == 13) && mode == mse::COL_PROP && in == out) {
-            // persistent tiles of 8 (12) or 16 (13) columns with XCD-aware item order; the grid
-            // is a multiple of the 8 XCDs
-            auto go_xcd = [&](auto tc) {
-                constexpr int TCX = decltype(tc)::value;
-                constexpr int NT = TCX * P0::L;
-                const int per_cu = resident_per_cu<mse::k_col_prop_pipe<P0, TCX, mse::WaveSync, true, 1, true>>(
-                    NT, 2048 / NT);
-                int blocks = std::min(e->num_cus * per_cu, (N / TCX) * nsets);
-                blocks = blocks >= 8 ? blocks / 8 * 8 : 8;
-                tiles = N / TCX;
-                launch(e, kind, [&]() {
-                    mse::k_col_prop_pipe<P0, TCX, mse::WaveSync, true, 1, true><<<blocks, NT, 0, e->stream>>>(
-                        out, wave_stride, e->tw.p, args, nsets);
-                });
+        if (variant == 11) {  // lean: two blocks per CU
+            auto lean = [&](auto bnd) {
+                constexpr bool BAND = decltype(bnd)::value;
+                if constexpr (P0::L == 64 && N <= 512) {  // 16-column tiles, 64 VGPRs
+                    dim3 grid(set_tiles(16), nsets);
+                    launch(e, kind, [&]() {
+                        mse::k_col_prop_lean<P0, BAND><<<grid, 16 * P0::L, 0, e->stream>>>(out, wave_stride, e->tw.p, args);
+                    });
+                    return true;
+                } else if constexpr (P0::L == 64 && P0::R3 > 1) {  // four-pass plans: 8-column tiles, 128 VGPRs
+                    dim3 grid(set_tiles(8), nsets);
+                    launch(e, kind, [&]() {
+                        mse::k_col_prop_lean8<P0, BAND><<<grid, 8 * P0::L, 0, e->stream>>>(out, wave_stride, e->tw.p, args);
+                    });
+                    return true;
+                }
+                return false;
             };
-            if (variant == 12)
-                go_xcd(C8{});
-            else
-                go_xcd(C16{});
-            return tiles;
+            if (band ? lean(std::true_type{}) : lean(std::false_type{})) return args.n_tiles;
         }
-        if (variant == 10 && mode == mse::COL_PROP && in == out) {  // 8-column tiles (no spills at 1024)
-            constexpr int NT = 8 * P0::L;
-            const int per_cu = resident_per_cu<mse::k_col_prop_pipe<P0, 8, mse::WaveSync>>(NT, 1024 / NT);
-            const int blocks = std::max(1, std::min(e->num_cus * per_cu, (N / 8) * nsets));
-            tiles = N / 8;
-            launch(e, kind, [&]() {
-                mse::k_col_prop_pipe<P0, 8, mse::WaveSync><<<blocks, NT, 0, e->stream>>>(out, wave_stride, e->tw.p,
-                                                                                        args, nsets);
-            });
-            return tiles;
+        switch (variant) {
+            case 12: pipe(P0{}, C8{}, REG{}, std::true_type{}, 2048); break;
+            case 13: pipe(P0{}, C16{}, REG{}, std::true_type{}, 2048); break;
+            case 10: pipe(P0{}, C8{}, REG{}, std::false_type{}, 1024); break;  // no spills at 1024
+            case 9: pipe(P0{}, C16{}, MEM{}, std::false_type{}, 1024); break;  // twiddles read at use
+            default: pipe(P0{}, C16{}, REG{}, std::false_type{}, 1024); break;
         }
-        if (variant == 9 && mode == mse::COL_PROP && in == out) {  // twiddles read at use
-            constexpr int NT = 16 * P0::L;
-            const int per_cu = resident_per_cu<mse::k_col_prop_pipe<P0, 16, mse::WaveSync, false>>(NT, 1024 / NT);
-            const int blocks = std::max(1, std::min(e->num_cus * per_cu, (N / 16) * nsets));
-            tiles = N / 16;
-            launch(e, kind, [&]() {
-                mse::k_col_prop_pipe<P0, 16, mse::WaveSync, false><<<blocks, NT, 0, e->stream>>>(out, wave_stride,
-                                                                                                e->tw.p, args, nsets);
-            });
-            return tiles;
-        }
-        if (variant == 11 && mode == mse::COL_PROP && in == out) {  // lean: two blocks per CU
-            if constexpr (P0::L == 64 && N <= 512) {  // 16-column tiles, 64 VGPRs
-                dim3 grid(N / 16, nsets);
-                tiles = N / 16;
-                launch(e, kind, [&]() {
-                    mse::k_col_prop_lean<P0><<<grid, 16 * P0::L, 0, e->stream>>>(out, wave_stride, e->tw.p, args);
-                });
-                return tiles;
-            } else if constexpr (P0::L == 64 && P0::R3 > 1) {  // four-pass plans: 8-column tiles, 128 VGPRs
-                dim3 grid(N / 8, nsets);
-                tiles = N / 8;
-                launch(e, kind, [&]() {
-                    mse::k_col_prop_lean8<P0><<<grid, 8 * P0::L, 0, e->stream>>>(out, wave_stride, e->tw.p, args);
-                });
-                return tiles;
-            }
-        }
-        if (variant >= 7 && mode == mse::COL_PROP && in == out) {
-            constexpr int NT = 16 * P0::L;
-            const int per_cu = resident_per_cu<mse::k_col_prop_pipe<P0, 16, mse::WaveSync>>(NT, 1024 / NT);
-            const int blocks = std::max(1, std::min(e->num_cus * per_cu, (N / 16) * nsets));
-            tiles = N / 16;
-            launch(e, kind, [&]() {
-                mse::k_col_prop_pipe<P0, 16, mse::WaveSync><<<blocks, NT, 0, e->stream>>>(out, wave_stride, e->tw.p, args,
-                                                                                          nsets);
-            });
-            return tiles;
-        }
-        if (variant >= 7) variant = 0;
-        if (variant == 1)
-            go(P1{}, C16{}, mse::WaveSync{}, REG{});
-        else if (variant == 2)
-            go(P0{}, C8{}, mse::WaveSync{}, REG{});
-        else if (variant == 3)
-            go(P0{}, C16{}, mse::BlockSync{}, REG{});
-        else if (variant == 4)
-            go(P0{}, C16{}, mse::WaveSync{}, MEM{});
-        else if (variant == 5)
-            go(P0{}, C8{}, mse::WaveSync{}, MEM{});
-        else if (variant == 6) {
-            if constexpr (N <= 512)  // 32 columns exceed the 160 KiB LDS above 512 points
-                go(P1{}, C32{}, mse::WaveSync{}, REG{});
-            else
-                go(P0{}, C16{}, mse::WaveSync{}, REG{});
-        }
-        else if (!hot && P0::L == 64 && P0::E > 8)  // 16-column tiles of 1024 threads spill here
-            go(P0{}, C8{}, mse::WaveSync{}, REG{});
+        return args.n_tiles;
+    }
+    if (variant >= 7) variant = 0;
+    if (variant == 1)
+        go(P1{}, C16{}, mse::WaveSync{}, REG{});
+    else if (variant == 2)
+        go(P0{}, C8{}, mse::WaveSync{}, REG{});
+    else if (variant == 3)
+        go(P0{}, C16{}, mse::BlockSync{}, REG{});
+    else if (variant == 4)
+        go(P0{}, C16{}, mse::WaveSync{}, MEM{});
+    else if (variant == 5)
+        go(P0{}, C8{}, mse::WaveSync{}, MEM{});
+    else if (variant == 6) {
+        if constexpr (N <= 512)  // 32 columns exceed the 160 KiB LDS above 512 points
+            go(P1{}, C32{}, mse::WaveSync{}, REG{});
         else
             go(P0{}, C16{}, mse::WaveSync{}, REG{});
-    }
-    return tiles;
+    } else if (!hot && P0::L == 64 && P0::E > 8)  // 16-column tiles of 1024 threads spill here
+        go(P0{}, C8{}, mse::WaveSync{}, REG{});
+    else
+        go(P0{}, C16{}, mse::WaveSync{}, REG{});
+    return args.n_tiles;
 }
 
 }  // namespace mse_rt
