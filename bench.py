@@ -568,7 +568,8 @@ def bench_sweeps(args):
             "best_row": br, "best_col": bc,
             "row_GBs": round(rowb / rows[br] / 1e3, 1), "col_GBs": round(colb / cols[bc][0] / 1e3, 1),
             "row_frac": round(rowb / rows[br] / 8e6, 4), "col_frac": round(colb / cols[bc][0] / 8e6, 4),
-            "row_copy_GBs": round(rowb / copy_row / 1e3, 1), "col_copy_GBs": round(colb / cols[bc][1] / 1e3, 1)}
+            "row_copy_GBs": round(B * 16 * N / copy_row / 1e3, 1),
+            "col_copy_GBs": round(B * 16 * N / cols[bc][1] / 1e3, 1)}
         log(f"{res}^2, B = {B}: row variant {br} {out[str(res)]['row_GBs']} GB/s "
             f"(copy pattern {out[str(res)]['row_copy_GBs']}), column variant {bc} {out[str(res)]['col_GBs']} GB/s "
             f"(copy pattern {out[str(res)]['col_copy_GBs']})")

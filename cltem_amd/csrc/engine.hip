@@ -103,7 +103,8 @@ void dispatch_res(int res, F&& f) {
 }
 
 // ---- sweeps: dispatch on the resolution to the per-size launchers ---------------------------
-// the variant of a sweep over nsets waves: the one tuned for that wave count, else the default
+// the variant of a sweep over nsets waves: the one tuned for that wave count, else the one set
+// (negative: none, the sweeps' rule)
 int tuned_variant(const mse_engine* e, int nsets, bool column) {
     for (const auto& t : e->tuned)
         if (t.first == nsets) return column ? t.second.second : t.second.first;
@@ -112,7 +113,7 @@ int tuned_variant(const mse_engine* e, int nsets, bool column) {
 
 void row_pass(mse_engine* e, int mode, const float2* in, float2* out, int nlines_sets,
               size_t wave_stride, const mse::RowArgs& args, int variant) {
-    if (variant < 0) variant = tuned_variant(e, nlines_sets, false);
+    if (variant == kEngineChoice) variant = tuned_variant(e, nlines_sets, false);
     switch (e->res) {
         case 256: row_pass_n<256>(e, mode, in, out, nlines_sets, wave_stride, args, variant); break;
         case 384: row_pass_n<384>(e, mode, in, out, nlines_sets, wave_stride, args, variant); break;
@@ -126,7 +127,7 @@ void row_pass(mse_engine* e, int mode, const float2* in, float2* out, int nlines
 // returns the number of column tiles of the launch (detector partials per wave)
 int col_pass(mse_engine* e, int mode, const float2* in, float2* out, int nsets, size_t wave_stride,
              const mse::ColArgs& args, int kind, int variant) {
-    if (variant < 0) variant = tuned_variant(e, nsets, true);
+    if (variant == kEngineChoice) variant = tuned_variant(e, nsets, true);
     switch (e->res) {
         case 256: return col_pass_n<256>(e, mode, in, out, nsets, wave_stride, args, kind, variant);
         case 384: return col_pass_n<384>(e, mode, in, out, nsets, wave_stride, args, kind, variant);
@@ -1245,8 +1246,11 @@ void potential_planes(mse_engine* e, const ConfigData& c, const mse_geometry& g,
 // band limit: FFT -> keep |k| <= kmax*2/3 -> IFFT (simulationgeneral.cpp:596-602).  The
 // column pass is a propagation step whose factors are the constant scale (x) and one (y),
 // with the band's per-row limits as the mask: cmul(v, cmul((s, 0), (1, 0))) = cmul(v, (s, 0))
-// bit for bit, on the persistent column kernels.  Their variant is fixed per grid size (not
-// tuned), so that transmission functions do not depend on the tuning state.
+// bit for bit, on the persistent column kernels.  Their variant goes by the rule on the grid size
+// and the number of planes, so that transmission functions do not depend on the tuning state: the
+// kernels the rule takes round alike, whatever the number of planes.  (At 768^2 the lean kernel,
+// which has always limited that size's functions: its twiddle products round otherwise, 118
+// against 103 us for 64 planes.)
 void band_limit_planes(mse_engine* e, float2* p, int planes) {
     const bool band = e->band_k >= 0;
     mse::RowArgs ra = base_row_args(e);
@@ -1262,8 +1266,7 @@ void band_limit_planes(mse_engine* e, float2* p, int planes) {
     ca.px = e->band_xy.p;
     ca.py = e->band_xy.p + e->res;
     ca.lim = e->band_lim.p;
-    const int variant = e->res == 1024 ? 12 : e->res == 768 ? 11 : 7;
-    col_pass(e, mse::COL_PROP, p, p, planes, e->N, ca, PK_COL, variant);
+    col_pass(e, mse::COL_PROP, p, p, planes, e->N, ca, PK_COL, e->res == 768 ? 11 : kRule);
     row_pass(e, mse::ROW_IFFT, p, p, planes, e->N, ra);
 }
 
@@ -2207,7 +2210,7 @@ int mse_autotune(mse_engine* e, int cfg, int n_waves, int reps, double* row_us, 
             if (row_us) row_us[v] = us;
             if (us < best) { best = us; bi = v; }
         }
-        e->row_var = bi;
+        const int row_best = bi;
         best = 1e30;
         bi = 0;
         for (int v = 0; v < kColVariants; ++v) {
@@ -2222,21 +2225,21 @@ int mse_autotune(mse_engine* e, int cfg, int n_waves, int reps, double* row_us, 
             if (col_us) col_us[v] = us;
             if (us < best) { best = us; bi = v; }
         }
-        e->col_var = bi;
-        // remembered for this wave count; other wave counts use the latest choice
+        const int col_best = bi;
+        // remembered for this wave count
         bool found = false;
         for (auto& t : e->tuned)
             if (t.first == n_waves) {
-                t.second = {e->row_var, e->col_var};
+                t.second = {row_best, col_best};
                 found = true;
             }
-        if (!found) e->tuned.push_back({n_waves, {e->row_var, e->col_var}});
+        if (!found) e->tuned.push_back({n_waves, {row_best, col_best}});
         ++e->tune_version;
         e->prof = prof;
         (void)hipEventDestroy(a);
         (void)hipEventDestroy(b);
-        if (best_row) *best_row = e->row_var;
-        if (best_col) *best_col = e->col_var;
+        if (best_row) *best_row = row_best;
+        if (best_col) *best_col = col_best;
     });
 }
 

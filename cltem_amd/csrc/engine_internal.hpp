@@ -175,9 +175,11 @@ struct mse_engine {
     DevBuf<int> tmp_Z, tmp_bid, tmp_zid;
     DevBuf<unsigned> keys, keys_sorted, idx, idx_sorted;
     DevBuf<unsigned char> cub_tmp;
-    int row_var = 4, col_var = 7;  // kernel variants (see row_pass / col_pass); pipelined by default
+    // kernel variants set by mse_set_kernel_variant, for every wave count; -1: by the sweeps'
+    // own rule on the grid size and the wave count
+    int row_var = -1, col_var = -1;
     // per wave count: the (row, column) variants mse_autotune found fastest for that many waves;
-    // sweeps over a tuned wave count use them, any other count the defaults above
+    // sweeps over a tuned wave count use them, any other count the ones above
     std::vector<std::pair<int, std::pair<int, int>>> tuned;
     unsigned tune_version = 0;     // bumped by every change of variants (captured graphs depend on them)
     hipGraphExec_t stem_exec = nullptr;
@@ -244,6 +246,10 @@ inline void launch(mse_engine* e, int kind, F&& f) {
     }
 }
 
+// variant arguments of row_pass / col_pass: the engine's choice (tuned, else set, else by rule), or
+// the sweeps' rule whatever was tuned or set
+constexpr int kEngineChoice = -1, kRule = -2;
+
 // ---- helpers defined in engine.hip ---------------------------------------------------------
 // potential-kernel arguments for a configuration's geometry
 mse::PotArgs pot_args(mse_engine* e, const ConfigData& c);
@@ -256,9 +262,9 @@ int run_guarded(const char* fn, mse_engine* e, const std::function<void()>& body
 mse::ColArgs base_col_args(mse_engine* e);
 mse::RowArgs base_row_args(mse_engine* e);
 void row_pass(mse_engine* e, int mode, const float2* in, float2* out, int nlines_sets, size_t wave_stride,
-              const mse::RowArgs& args, int variant = -1);
+              const mse::RowArgs& args, int variant = kEngineChoice);
 int col_pass(mse_engine* e, int mode, const float2* in, float2* out, int nsets, size_t wave_stride,
-             const mse::ColArgs& args, int kind = PK_COL, int variant = -1);
+             const mse::ColArgs& args, int kind = PK_COL, int variant = kEngineChoice);
 // The columns of one slice's row and column pass (io, band_k of both): the band alone where the
 // limits allow it.  first: the row pass's input may hold anything outside the band (the start of
 // a slice loop), which it clears; else the wave comes from a column pass.
@@ -284,7 +290,7 @@ void sync_wave_prop(mse_engine* e);
 //   column 0: default plan, 16 columns per block  1: half lanes per column
 //          2: 8 columns per block                 3: block barriers
 //          4: 16 columns, twiddles read at use, >= 8 waves per SIMD (2 blocks per CU)
-//          5: 8 columns, twiddles read at use, >= 8 waves per SIMD (4 blocks per CU)
+//          5: as 12 with 4-column tiles (few waves: the launch covers more CUs)
 //          6: 32 columns (256-byte row runs), half lanes per column
 //   row    4: persistent lines with the next row prefetched into registers
 //          5: as 4 with half lanes per line (res <= 512; otherwise as 4)

@@ -823,10 +823,12 @@ __global__ __launch_bounds__(8 * PL::L) __attribute__((amdgpu_waves_per_eu(4))) 
 }
 
 // --------------------------------------------------------------------------------------
-// Persistent, software-pipelined row slice step (ROW_IFFT_T_FFT).  Every line walks the
-// (wave, row) items independently; the next item's wave row and transmission row are
-// loaded into registers while the current row is transformed.  MODE = ROW_FFT or ROW_IFFT:
-// the one transform and the scale of k_row's same modes, in place (no transmission row).
+// Persistent, software-pipelined row slice step (ROW_IFFT_T_FFT).  Line l of the grid takes row
+// l % N of the sets l / N, l / N + G, ... (G = lines of the grid / N): the same row of one wave
+// after another, so that a transmission row stays in registers while the waves share it, and at
+// any time G waves are swept front to back.  The next wave's row is loaded into registers while
+// the current one is transformed.  MODE = ROW_FFT or ROW_IFFT: the one transform and the scale
+// of k_row's same modes, in place (no transmission row).
 // --------------------------------------------------------------------------------------
 template <class PL, int IO = BAND_FULL, class SYNC = WaveSync, bool TWREG = true, int MODE = ROW_IFFT_T_FFT>
 __global__ __launch_bounds__(256) void k_row_step_pipe(float2* __restrict__ data, size_t wave_stride,
@@ -840,46 +842,49 @@ __global__ __launch_bounds__(256) void k_row_step_pipe(float2* __restrict__ data
     const int line = tid / L;
     const int t = tid % L;
     float2* ln = lds[line];
-    const int nitems = nsets * N;
-    const int stride = gridDim.x * LINES;
+    // with one line per wave (L = 64) the row is wave-uniform; set, wave and configuration are
+    // the same for all lines of a block (LINES divides N)
+    const int first_line = blockIdx.x * LINES;
+    const int groups = gridDim.x * LINES / N;
+    int row = first_line % N + line;
+    if constexpr (L == 64) row = __builtin_amdgcn_readfirstlane(row);
+    int set = first_line / N;
+    if (set >= nsets) return;
 
     PlanTw<PL, TWREG> tws;
     tws.load(tw, t);
     const SYNC sync{};
 
-    float2 qv[E], qt[E];
-    auto fetch = [&](int item) {
-        // with one line per wave the item is wave-uniform: its wave, configuration and
-        // transmission row then come from scalar loads
-        if constexpr (L == 64) item = __builtin_amdgcn_readfirstlane(item);
-        const int wv = a.wave_map ? cload(a.wave_map + item / N) : item / N, row = item % N;
-        band_load<PL, IO>(qv, data + (size_t)wv * wave_stride + (size_t)row * N, t, a.band_k);
-        if constexpr (!STEP) return;
-        const int cfg = row_config(a, wv);
-        if (a.slice < cload(a.cfg_nslices + cfg)) {
-            const float2* tr = cload(a.cfg_trans + cfg) + (size_t)a.slice * N * N + (size_t)row * N;
-#pragma unroll
-            for (int m = 0; m < E; ++m) qt[m] = gload(tr + t + L * m);
-        } else {  // vacuum below a thinner specimen
-#pragma unroll
-            for (int m = 0; m < E; ++m) qt[m] = make_float2(1.f, 0.f);
-        }
+    auto row_of = [&](int s) {
+        const int wv = a.wave_map ? cload(a.wave_map + s) : s;
+        return data + (size_t)wv * wave_stride + (size_t)row * N;
     };
-    int item = blockIdx.x * LINES + line;
-    if (item < nitems) fetch(item);
-    for (; item < nitems; item += stride) {
-        float2 v[E], tr[E];
+    float2 qv[E], tr[STEP ? E : 1];
+    const float2* cur = nullptr;  // the transmission row in tr
+    bool vacuum = false;          // below a thinner specimen: t = 1, nothing to multiply
+    band_load<PL, IO>(qv, row_of(set), t, a.band_k);
+    for (; set < nsets; set += groups) {
+        if constexpr (STEP) {
+            const int cfg = row_config(a, a.wave_map ? cload(a.wave_map + set) : set);
+            const float2* tp = cload(a.cfg_trans + cfg) + (size_t)a.slice * N * N + (size_t)row * N;
+            vacuum = a.slice >= cload(a.cfg_nslices + cfg);
+            if (!vacuum && tp != cur) {
 #pragma unroll
-        for (int m = 0; m < E; ++m) {
-            v[m] = qv[m];
-            tr[m] = qt[m];
+                for (int m = 0; m < E; ++m) tr[m] = gload(tp + t + L * m);
+                cur = tp;
+            }
         }
-        if (item + stride < nitems) fetch(item + stride);
+        float2 v[E];
+#pragma unroll
+        for (int m = 0; m < E; ++m) v[m] = qv[m];
+        if (set + groups < nsets) band_load<PL, IO>(qv, row_of(set + groups), t, a.band_k);
         if constexpr (STEP) {
             fft_line<PL, true, band_reads(IO)>(v, ln, t, tws, sync);
             sync();
+            if (!vacuum) {
 #pragma unroll
-            for (int m = 0; m < E; ++m) v[m] = cmul(v[m], tr[m]);
+                for (int m = 0; m < E; ++m) v[m] = cmul(v[m], tr[m]);
+            }
             fft_line<PL, false>(v, ln, t, tws, sync);
         } else {
             fft_line<PL, MODE == ROW_IFFT, band_reads(IO)>(v, ln, t, tws, sync);
@@ -887,10 +892,7 @@ __global__ __launch_bounds__(256) void k_row_step_pipe(float2* __restrict__ data
             for (int m = 0; m < E; ++m) v[m] = cscale(v[m], a.scale);
         }
         sync();
-        int it = item;
-        if constexpr (L == 64) it = __builtin_amdgcn_readfirstlane(it);
-        const int wv = a.wave_map ? cload(a.wave_map + it / N) : it / N, row = it % N;
-        band_store<PL, IO>(v, data + (size_t)wv * wave_stride + (size_t)row * N, t, a.band_k);
+        band_store<PL, IO>(v, row_of(set), t, a.band_k);
     }
 }
 

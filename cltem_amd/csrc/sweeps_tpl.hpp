@@ -29,6 +29,17 @@ void row_pass_n(mse_engine* e, int mode, const float2* in, float2* out, int nlin
     using REG = std::true_type;
     using MEM = std::false_type;
     const bool step = mode == mse::ROW_IFFT_T_FFT;
+    if (step && variant < 0) {
+        // Rule: while every line of the grid takes one row at most, the plain kernel (its waves go
+        // straight to the loads); beyond, the persistent one, which keeps a transmission row in
+        // registers over the waves and prefetches.  Plain against persistent, us: 256^2 one wave
+        // 4.3 / 4.9, 32 waves 8.6 / 8.9; 512^2 one 4.7 / 5.3, 8 waves 9.6 / 10.0, 16 waves
+        // 15.4 / 14.1, 64 waves 48 / 35; 768^2 4 waves 11.9 / 12.4, 8 waves 21.5 / 18.9; 1024^2
+        // 2 waves 9.6 / 10.7, 8 waves 27.4 / 24.7.
+        using K = std::integral_constant<int, mse::BAND_STEP>;
+        const int per_cu = resident_per_cu<mse::k_row_step_pipe<P0, K::value, mse::WaveSync, true>>(256, 8);
+        variant = nlines_sets <= e->num_cus * per_cu * (256 / P0::L) / N ? 0 : 4;
+    }
     // one row per line of the grid, out of place or with the non-persistent variants
     auto go = [&](auto plan, auto sync, auto twreg) {
         using PL = decltype(plan);
@@ -65,8 +76,11 @@ void row_pass_n(mse_engine* e, int mode, const float2* in, float2* out, int nlin
         constexpr bool TR = decltype(twreg)::value;
         constexpr int MD = decltype(m)::value, IO = decltype(io)::value;
         constexpr int LINES = 256 / PL::L;
-        const int per_cu = resident_per_cu<mse::k_row_step_pipe<PL, IO, mse::WaveSync, TR, MD>>(256, 4);
-        const int blocks = std::max(1, std::min(e->num_cus * per_cu, (N * nlines_sets + LINES - 1) / LINES));
+        const int per_cu = resident_per_cu<mse::k_row_step_pipe<PL, IO, mse::WaveSync, TR, MD>>(256, 8);
+        // whole groups of N lines; as few as the rounds over the sets need
+        const int most = std::max(1, e->num_cus * per_cu * LINES / N);
+        const int rounds = (nlines_sets + most - 1) / most;
+        const int blocks = (nlines_sets + rounds - 1) / rounds * (N / LINES);
         launch(e, PK_ROW, [&]() {
             mse::k_row_step_pipe<PL, IO, mse::WaveSync, TR, MD><<<blocks, 256, 0, e->stream>>>(
                 out, wave_stride, e->tw.p, args, nlines_sets);
@@ -121,6 +135,7 @@ int col_pass_n(mse_engine* e, int mode, const float2* in, float2* out, int nsets
     using P1 = typename mse::PlanHalfLanes<N>::P;
     using C16 = std::integral_constant<int, 16>;
     using C8 = std::integral_constant<int, 8>;
+    using C4 = std::integral_constant<int, 4>;
     using C32 = std::integral_constant<int, 32>;
     using REG = std::true_type;
     using MEM = std::false_type;
@@ -129,6 +144,22 @@ int col_pass_n(mse_engine* e, int mode, const float2* in, float2* out, int nsets
     const bool band = prop && args0.band_k >= 0;
     if (!hot) variant = 0;
     mse::ColArgs args = args0;
+    if (mode == mse::COL_PROP && in == out && variant < 0) {
+        // Rule: the narrowest tiles while they leave CUs idle, wider ones as the launch grows (a
+        // narrow tile is a shorter chain of loads, transforms and stores, a wide one moves whole
+        // 128-byte lines and shares a line's transfer with no other block).  us per launch on the
+        // band, 4 / 8 / 16 columns (the first two in XCD-aware order): 256^2 one wave
+        // 4.5 / 5.0 / 5.6, 16 waves 6.1 / 6.4 / 6.5, 64 waves 15.7 / 15.2 / 12.3; 512^2 one
+        // 5.7 / 6.4 / 9.8, 8 waves 9.2 / 10.3 / 11.5, 16 waves 17.8 / 17.0 / 16.9, 128 waves
+        // - / 69.8 / 62.8; 768^2 one 8.2 / 10.5 / 26.7, 4 waves 12.3 / 12.2 / 30.5; 1024^2 2 waves
+        // 12.6 / 12.8 / 37.6, 4 waves 22.4 / 20.8 / 41.9, 64 waves 187 / 177 / 407 (16 columns of
+        // the 12- and 16-element plans spill or leave a CU one block of half its waves).
+        const int k = band ? args.band_k : N / 2;
+        const long long items4 = (2 * (k / 4) + 2) * (long long)nsets;
+        variant = items4 <= e->num_cus * (P0::E <= 8 ? 3 : 2)                     ? 5
+                  : N > 512 || (2 * (k / 16) + 2) * (long long)nsets < 3 * e->num_cus ? 12
+                                                                                  : 7;
+    }
     // the tiles of TC columns to visit: with a band, those that hold columns 0..K or N-K..N-1
     auto set_tiles = [&](int TC) {
         args.tile_lo = N / TC;
@@ -174,7 +205,7 @@ int col_pass_n(mse_engine* e, int mode, const float2* in, float2* out, int nsets
             throw Error(MSE_ERR_STATE, "column pass without a kernel");
         });
     };
-    if (variant >= 7 && mode == mse::COL_PROP && in == out) {
+    if ((variant >= 7 || variant == 5) && mode == mse::COL_PROP && in == out) {
         // persistent blocks, at most `cap` per CU; the XCD-aware order takes a multiple of 8
         auto go_pipe = [&](auto plan, auto tc, auto twreg, auto xcd, auto bnd, int cap) {
             using PL = decltype(plan);
@@ -183,7 +214,7 @@ int col_pass_n(mse_engine* e, int mode, const float2* in, float2* out, int nsets
             const int items = set_tiles(TC) * nsets;
             const int per_cu = resident_per_cu<mse::k_col_prop_pipe<PL, TC, BAND, mse::WaveSync, TR, 1, XCD>>(NT, cap / NT);
             int blocks = std::max(1, std::min(e->num_cus * per_cu, items));
-            if (XCD) blocks = blocks >= 8 ? blocks / 8 * 8 : 8;
+            if (XCD) blocks = (blocks + 7) / 8 * 8;
             launch(e, kind, [&]() {
                 mse::k_col_prop_pipe<PL, TC, BAND, mse::WaveSync, TR, 1, XCD><<<blocks, NT, 0, e->stream>>>(
                     out, wave_stride, e->tw.p, args, nsets);
@@ -222,6 +253,7 @@ int col_pass_n(mse_engine* e, int mode, const float2* in, float2* out, int nsets
             if (band ? lean(std::true_type{}) : lean(std::false_type{})) return args.n_tiles;
         }
         switch (variant) {
+            case 5: pipe(P0{}, C4{}, REG{}, std::true_type{}, 2048); break;
             case 12: pipe(P0{}, C8{}, REG{}, std::true_type{}, 2048); break;
             case 13: pipe(P0{}, C16{}, REG{}, std::true_type{}, 2048); break;
             case 10: pipe(P0{}, C8{}, REG{}, std::false_type{}, 1024); break;  // no spills at 1024
@@ -239,8 +271,6 @@ int col_pass_n(mse_engine* e, int mode, const float2* in, float2* out, int nsets
         go(P0{}, C16{}, mse::BlockSync{}, REG{});
     else if (variant == 4)
         go(P0{}, C16{}, mse::WaveSync{}, MEM{});
-    else if (variant == 5)
-        go(P0{}, C8{}, mse::WaveSync{}, MEM{});
     else if (variant == 6) {
         if constexpr (N <= 512)  // 32 columns exceed the 160 KiB LDS above 512 points
             go(P1{}, C32{}, mse::WaveSync{}, REG{});
