@@ -129,7 +129,8 @@ int mse_adjoint_positions(mse_engine* e, const double* dl_di, double* grad_xyz) 
         const int chunk = g.full3d ? 32 : 256;
         for (int s0 = 0; s0 < n; s0 += chunk) {
             const int cs = std::min(chunk, n - s0);
-            dim3 grid(e->res / 16, e->res / 16, cs);
+            const dim3 grid = g.full3d ? dim3(e->res / 16, e->res / 16, cs)
+                                       : dim3(e->res / (16 * mse::kProjPX), e->res / (16 * mse::kProjPY), cs);
             float* o = e->adj_phase.p + (size_t)s0 * N;
             launch(e, PK_POT, [&]() {
                 if (g.full3d) {

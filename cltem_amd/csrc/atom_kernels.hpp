@@ -322,6 +322,7 @@ struct PotArgs {
     // factors), 1 / pixel size and (8 A + a margin of 0.01 A^2)^2 in pixels^2
     double rrx, rry;
     float inv_ps, reach_px2;
+    float inside_px2;  // (8 A - a margin of 0.01 A^2)^2 in pixels^2
 };
 
 // An element's device table as an address biased so that the bucket of r2 sits at byte
@@ -363,13 +364,17 @@ __device__ __forceinline__ float vtab_eval(unsigned long long base, float r2) {
 
 // V(r2) as vtab_eval computes it, for kVtabFloor <= r2 < 2^kOctaveHi, where the offset needs
 // no clamp.
-__device__ __forceinline__ float vtab_eval_in(unsigned long long base, float r2) {
-    const unsigned bits = __float_as_uint(r2);
-    const unsigned off = (bits >> (mse_tab::kMantBits - 4)) & ~15u;
+__device__ __forceinline__ float4 vtab_bucket(unsigned long long base, float r2) {
+    const unsigned off = (__float_as_uint(r2) >> (mse_tab::kMantBits - 4)) & ~15u;
     using gfloat4 = const __attribute__((address_space(1))) float4;
-    const float4 c = *(const float4*)reinterpret_cast<gfloat4*>(base + off);
-    const float m = (float)(bits & ((1u << mse_tab::kMantBits) - 1u));
+    return *(const float4*)reinterpret_cast<gfloat4*>(base + off);
+}
+__device__ __forceinline__ float vtab_cubic(float4 c, float r2) {
+    const float m = (float)(__float_as_uint(r2) & ((1u << mse_tab::kMantBits) - 1u));
     return fmaf(fmaf(fmaf(c.w, m, c.z), m, c.y), m, c.x);
+}
+__device__ __forceinline__ float vtab_eval_in(unsigned long long base, float r2) {
+    return vtab_cubic(vtab_bucket(base, r2), r2);
 }
 
 // V(r2) as vtab_eval computes it, from the LDS copy of an element's buckets
@@ -478,6 +483,12 @@ __device__ __forceinline__ int tile_pixel_y(int j) {
 // through LDS as one sequence, in chunks of 256, with no limit on how many a row holds.  (The
 // tables stay in global memory here: one evaluation per atom and pixel is too little work to
 // repay an LDS copy per block.)
+// VALU issue bounds it: 13 instructions per evaluation where the wave's pixels need no test (11
+// of them the double add of the squared distance, the conversion, the bucket's offset and its
+// cubic, and the double sum), about twice that with the tests, which also put one table read
+// after the other.  Taking the tests out of the pairs that cannot need them, and each wave's list
+// of its own atoms: 768^2, 63 slices 417 -> 372 us; 1024^2, 24 slices 258 -> 238 us; 12 planes of
+// 256^2 29 -> 23 us.
 template <int FORM, bool TAB, int PX = 1, int PY = 1>
 __device__ __forceinline__ void projected_sumz(const double* __restrict__ ax, const double* __restrict__ ay,
                                                const int* __restrict__ aZ, const int* __restrict__ bsp,
@@ -541,6 +552,9 @@ __device__ __forceinline__ void projected_sumz(const double* __restrict__ ax, co
             // bits 16..19: the waves (pixel quadrants of the tile) that may have a pixel
             // within 8 A; the distance to each wave's pixel rectangle, in pixels and in
             // float, is tested against 64.01 A^2, a margin far above the float error.
+            // Bits 20..23: the waves all of whose pixels lie within 8 A (the rectangle's
+            // farthest corner, against 63.99 A^2) and farther than r_min = 1/4 pixel (its
+            // nearest point, against 0.26 pixels), where the potential needs no test.
             // Untilted only (a tilted metric is no lateral distance): all waves otherwise.
             unsigned waves = 15u;
             if (a.untilted) {
@@ -550,62 +564,102 @@ __device__ __forceinline__ void projected_sumz(const double* __restrict__ ax, co
 #pragma unroll
                 for (int w = 0; w < 4; ++w) {
                     const float u0 = (float)((w & 1) * 8 * PX), v0 = (float)((w >> 1) * 8 * PY);
-                    const float du = fmaxf(fmaxf(u0 - u, u - (u0 + (8.f * PX - 1.f))), 0.f);
-                    const float dv = fmaxf(fmaxf(v0 - v, v - (v0 + (8.f * PY - 1.f))), 0.f);
-                    if (du * du + dv * dv <= reach_px2) waves |= 1u << w;
+                    const float u1 = u0 + (8.f * PX - 1.f), v1 = v0 + (8.f * PY - 1.f);
+                    const float du = fmaxf(fmaxf(u0 - u, u - u1), 0.f);
+                    const float dv = fmaxf(fmaxf(v0 - v, v - v1), 0.f);
+                    const float d2 = du * du + dv * dv;
+                    const float fu = fmaxf(u - u0, u1 - u), fv = fmaxf(v - v0, v1 - v);
+                    if (d2 <= reach_px2) waves |= 1u << w;
+                    if (d2 > 0.26f * 0.26f && fu * fu + fv * fv <= a.inside_px2) waves |= 16u << w;
                 }
             }
             sZ[lid] = aZ[c] | (int)(waves << 16);
         }
         __syncthreads();
-        for (int l = 0; l < cnt; ++l) {
-            const int info = __builtin_amdgcn_readfirstlane(sZ[l]);
-            if (!((info >> (16 + wave)) & 1)) continue;
-            const int zs = info & 0xffff;
-            // the element's constants (or table), loaded ahead of the distance arithmetic
-            float pt[TAB ? 1 : kPotProjStride];
-            unsigned long long tz = 0;
-            if constexpr (TAB) {
-                tz = vtab_base(a.vtab + (size_t)(zs - 1) * mse_tab::kBuckets);
-            } else {
-                const float* row = ptab + (size_t)(zs - 1) * kPotProjStride;
+        // the wave's own atoms of each 64 staged: their list is a mask in scalar registers, so
+        // the others cost nothing and the next atom is known without a round trip to LDS
+        for (int l0 = 0; l0 < cnt; l0 += 64) {
+            const int li = l0 + (lid & 63);
+            const int infos = li < cnt ? sZ[li] : 0;
+            unsigned long long todo = __builtin_amdgcn_ballot_w64((infos >> (16 + wave)) & 1);
+            const unsigned long long plain = __builtin_amdgcn_ballot_w64((infos >> (20 + wave)) & 1);
+            while (todo) {
+                const int b = __builtin_ctzll(todo);
+                const int l = l0 + b;
+                todo &= todo - 1;
+                const int zs = __builtin_amdgcn_readlane(infos, b) & 0xffff;
+                // the element's constants (or table), loaded ahead of the distance arithmetic
+                float pt[TAB ? 1 : kPotProjStride];
+                unsigned long long tz = 0;
+                if constexpr (TAB) {
+                    tz = vtab_base(a.vtab + (size_t)(zs - 1) * mse_tab::kBuckets);
+                } else {
+                    const float* row = ptab + (size_t)(zs - 1) * kPotProjStride;
 #pragma unroll
-                for (int q = 0; q < kPotProjStride; ++q) pt[q] = row[q];
-            }
-            const double xl = sx[l], yl = sy[l];
+                    for (int q = 0; q < kPotProjStride; ++q) pt[q] = row[q];
+                }
+                const double xl = sx[l], yl = sy[l];
+                if constexpr (TAB) {
+                    if ((plain >> b) & 1) {
+                        // every pixel of the wave takes part and none is clamped: the pixels'
+                        // table reads are issued together
+                        double rx2[PX], ry2[PY];
 #pragma unroll
-            for (int jy = 0; jy < PY; ++jy) {
-                const double rad_y = im_pos_y[jy] - yl;
+                        for (int i = 0; i < PX; ++i) {
+                            const double d = im_pos_x[i] - xl;
+                            rx2[i] = d * d;
+                        }
 #pragma unroll
-                for (int i = 0; i < PX; ++i) {
-                    const double rad_x = im_pos_x[i] - xl;
-                    double r2;
-                    if (a.untilted) {
-                        // theta = pi/2: z' = O(1e-16) rad and z'/tan(theta) = O(1e-32) rad
-                        // vanish below the rounding of x'^2 + y'^2, which equals this exactly
-                        r2 = rad_x * rad_x + rad_y * rad_y;
-                    } else {
-                        const double z_prime = -0.5 * (rad_x * a.cos_phi + rad_y * a.sin_phi) * a.sin_2theta;
-                        const double zt = z_prime / a.tan_theta;
-                        const double x_prime = rad_x + zt * a.cos_phi;
-                        const double y_prime = rad_y + zt * a.sin_phi;
-                        r2 = z_prime * z_prime + x_prime * x_prime + y_prime * y_prime;
+                        for (int jy = 0; jy < PY; ++jy) {
+                            const double d = im_pos_y[jy] - yl;
+                            ry2[jy] = d * d;
+                        }
+                        float f[PX * PY];
+                        float4 cb[PX * PY];
+#pragma unroll
+                        for (int q = 0; q < PX * PY; ++q) {
+                            f[q] = (float)(rx2[q % PX] + ry2[q / PX]);
+                            cb[q] = vtab_bucket(tz, f[q]);
+                        }
+#pragma unroll
+                        for (int q = 0; q < PX * PY; ++q) sumz[q] += (double)vtab_cubic(cb[q], f[q]);
+                        continue;
                     }
-                    // rad = max(sqrt(r2), r_min) <= 8 with r2 <= 64.0000000001 (the
-                    // reference's test, correctly rounded double sqrt): sqrt(64 + 2^-46) =
-                    // 8 + 2^-50 - 2^-103... rounds to 8 while sqrt of the next double,
-                    // 64 + 2^-45, rounds to 8 + 2^-49, so the test is exactly
-                    // r2 <= 64 + 2^-46.  The potential takes rad in float.
-                    if (r2 <= 0x1.0000000000001p+6) {
-                        if constexpr (TAB) {
-                            // r_min^2 is above the tables' floor (the host enables them only
-                            // then) and r2 <= 64 + 2^-46 is 64 or less in float, far inside
-                            // their top: the lookup needs no clamp
-                            const float f = r2 < r_min2 ? r_minf * r_minf : (float)r2;
-                            sumz[jy * PX + i] += (double)vtab_eval_in(tz, f);
+                }
+#pragma unroll
+                for (int jy = 0; jy < PY; ++jy) {
+                    const double rad_y = im_pos_y[jy] - yl;
+#pragma unroll
+                    for (int i = 0; i < PX; ++i) {
+                        const double rad_x = im_pos_x[i] - xl;
+                        double r2;
+                        if (a.untilted) {
+                            // theta = pi/2: z' = O(1e-16) rad and z'/tan(theta) = O(1e-32) rad
+                            // vanish below the rounding of x'^2 + y'^2, which equals this exactly
+                            r2 = rad_x * rad_x + rad_y * rad_y;
                         } else {
-                            const float rf = r2 < r_min2 ? r_minf : __builtin_amdgcn_sqrtf((float)r2);
-                            sumz[jy * PX + i] += (double)vproj_tab<FORM>(pt, a.i_count, rf);
+                            const double z_prime = -0.5 * (rad_x * a.cos_phi + rad_y * a.sin_phi) * a.sin_2theta;
+                            const double zt = z_prime / a.tan_theta;
+                            const double x_prime = rad_x + zt * a.cos_phi;
+                            const double y_prime = rad_y + zt * a.sin_phi;
+                            r2 = z_prime * z_prime + x_prime * x_prime + y_prime * y_prime;
+                        }
+                        // rad = max(sqrt(r2), r_min) <= 8 with r2 <= 64.0000000001 (the
+                        // reference's test, correctly rounded double sqrt): sqrt(64 + 2^-46) =
+                        // 8 + 2^-50 - 2^-103... rounds to 8 while sqrt of the next double,
+                        // 64 + 2^-45, rounds to 8 + 2^-49, so the test is exactly
+                        // r2 <= 64 + 2^-46.  The potential takes rad in float.
+                        if (r2 <= 0x1.0000000000001p+6) {
+                            if constexpr (TAB) {
+                                // r_min^2 is above the tables' floor (the host enables them only
+                                // then) and r2 <= 64 + 2^-46 is 64 or less in float, far inside
+                                // their top: the lookup needs no clamp
+                                const float f = r2 < r_min2 ? r_minf * r_minf : (float)r2;
+                                sumz[jy * PX + i] += (double)vtab_eval_in(tz, f);
+                            } else {
+                                const float rf = r2 < r_min2 ? r_minf : __builtin_amdgcn_sqrtf((float)r2);
+                                sumz[jy * PX + i] += (double)vproj_tab<FORM>(pt, a.i_count, rf);
+                            }
                         }
                     }
                 }
@@ -658,7 +712,7 @@ __global__ __launch_bounds__(256) void k_potential_projected(
 
 // The phase sigma V of the same slices, reduced to [-pi, pi] as phase_to_t reduces it, so
 // that sincosf of the stored float reproduces the transmission function's exp(i sigma V)
-// before the band limit (used by the adjoint).  Grid (res / 16, res / 16, planes).
+// before the band limit (used by the adjoint).  Grid as k_potential_projected's.
 template <int FORM, bool TAB = false>
 __global__ __launch_bounds__(256) void k_phase_projected(
     float* __restrict__ out, const double* __restrict__ ax, const double* __restrict__ ay,
@@ -666,12 +720,16 @@ __global__ __launch_bounds__(256) void k_phase_projected(
     PotArgs a, int first) {
     __shared__ double sx[256], sy[256];
     __shared__ int sZ[256];
-    double sumz[1];
-    projected_sumz<FORM, TAB, 1, 1>(ax, ay, aZ, bsp, ptab, a, first + (int)blockIdx.z, sx, sy, sZ, sumz);
-    const int xid = tile_pixel_x<1, 1>(0);
-    const int yid = tile_pixel_y<1, 1>(0);
-    out[(size_t)blockIdx.z * a.res * a.res + (size_t)yid * a.res + xid] =
-        (float)reduce_2pi(a.sigma * sumz[0]);
+    double sumz[kProjPX * kProjPY];
+    projected_sumz<FORM, TAB, kProjPX, kProjPY>(ax, ay, aZ, bsp, ptab, a, first + (int)blockIdx.z, sx, sy, sZ, sumz);
+#pragma unroll
+    for (int j = 0; j < kProjPY; ++j) {
+        const int yid = tile_pixel_y<kProjPX, kProjPY>(j);
+#pragma unroll
+        for (int i = 0; i < kProjPX; ++i)
+            out[(size_t)blockIdx.z * a.res * a.res + (size_t)yid * a.res + tile_pixel_x<kProjPX, kProjPY>(i)] =
+                (float)reduce_2pi(a.sigma * sumz[j * kProjPX + i]);
+    }
 }
 
 // transmission_potentials_full_3d: trapezoid over integrals+1 sub-slice points for the

@@ -213,6 +213,7 @@ mse::PotArgs pot_args(mse_engine* e, const ConfigData& c) {
     a.rry = 1.0 / (a.max_y - a.min_y);
     a.inv_ps = (float)(1.0 / a.pixelscale);
     a.reach_px2 = (float)(64.01 / (a.pixelscale * a.pixelscale));
+    a.inside_px2 = (float)(63.99 / (a.pixelscale * a.pixelscale));
     a.load_x = g.load_x;
     a.load_y = g.load_y;
     a.load_z = g.load_z;
