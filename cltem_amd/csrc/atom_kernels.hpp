@@ -306,9 +306,10 @@ struct PotArgs {
     int integrals;
     int per_atom;        // parameters per Z (12 or 10)
     int i_count;
-    // moving STEM frames: when set, blockIdx.z selects a frame whose potential-grid origin is
-    // (frame_xy[2z], frame_xy[2z+1]) and every frame builds the same slice `first`
+    // moving STEM frames: when set, plane blockIdx.z is slice first + z % frame_slices of frame
+    // f = z / frame_slices, whose potential-grid origin is (frame_xy[2f], frame_xy[2f+1])
     const double* frame_xy;
+    int frame_slices;
     // tabulated potentials (potential_table.hpp), kBuckets cubic pieces per element from
     // element 1; read by the kernels instantiated with TAB = true
     const float4* vtab;
@@ -392,13 +393,14 @@ __device__ __forceinline__ float vtab_eval_lds(const float4* __restrict__ lt, in
 }
 
 // The arguments of the plane blockIdx.z of a launch over slices [first, first + gridDim.z),
-// or over frames of slice `first` (frame_xy set); returns the slice.
+// or over frames times slices (frame_xy set); returns the slice.
 __device__ __forceinline__ int plane_args(const PotArgs& a, int first, PotArgs& b) {
     b = a;
     if (a.frame_xy) {
-        b.startx = a.frame_xy[2 * blockIdx.z];
-        b.starty = a.frame_xy[2 * blockIdx.z + 1];
-        return first;
+        const int f = (int)blockIdx.z / a.frame_slices;
+        b.startx = a.frame_xy[2 * f];
+        b.starty = a.frame_xy[2 * f + 1];
+        return first + (int)blockIdx.z % a.frame_slices;
     }
     return first + (int)blockIdx.z;
 }

@@ -40,6 +40,10 @@ namespace mse_rt {
 
 void destroy_stem_graph(mse_engine* e);
 
+// most bytes of transmission functions mse_stem_batch_frames builds at once (one slice of every
+// frame where that takes more)
+constexpr size_t kFrameBytes = size_t(512) << 20;
+
 // Per-device address of `scratch`, looked up once per device with that device current.
 std::mutex g_scratch_mu;
 std::vector<void*> g_scratch_ptr;
@@ -1846,23 +1850,31 @@ int mse_stem_batch_frames(mse_engine* e, int cfg, const double* pos_xy, const do
         e->partials.ensure((size_t)batch * n_det * (e->res / 8));
         e->det_out.ensure((size_t)n_probes * n_det);
         e->frame_xy.ensure(2 * (size_t)batch);
-        e->frame_trans.ensure((size_t)batch * e->N);
-        // the row pass finds wave w's transmission function as plane w of frame_trans: a table
-        // of one "configuration" per wave, each one slice deep, read at slice 0
+        // Transmission functions of several slices of every frame at once, up to half a GiB (and
+        // 65535 planes, the grid's limit): one slice's planes are too little work for the
+        // potential kernel and three band-limit launches.  12 frames of 256^2, 15 slices: 1.74
+        // -> 0.86 ms per 24 probes.
+        const size_t plane_bytes = (size_t)batch * e->N * sizeof(float2);
+        const int most = (int)std::min<size_t>(kFrameBytes / plane_bytes, 65535 / (size_t)batch);
+        const int groups = (ns + std::max(1, most) - 1) / std::max(1, most);
+        const int cs = (ns + groups - 1) / groups;
+        e->frame_trans.ensure((size_t)batch * cs * e->N);
+        // the row pass finds wave w's transmission functions at planes w cs.. of frame_trans: a
+        // table of one "configuration" per wave, each cs slices deep
         e->frame_ptrs.ensure(batch);
         e->frame_ns.ensure(batch);
         e->frame_wcfg.ensure(batch);
         if (!e->h_focus.empty()) e->probe_df.ensure(std::max<size_t>(batch, e->n_waves));
         {
             std::vector<const float2*> ptrs(batch);
-            std::vector<int> ones(batch, 1), ids(batch);
+            std::vector<int> depth(batch, cs), ids(batch);
             for (int w = 0; w < batch; ++w) {
-                ptrs[w] = e->frame_trans.p + (size_t)w * e->N;
+                ptrs[w] = e->frame_trans.p + (size_t)w * cs * e->N;
                 ids[w] = w;
             }
             HIPX(hipMemcpyAsync(e->frame_ptrs.p, ptrs.data(), batch * sizeof(const float2*), hipMemcpyHostToDevice,
                                 e->stream));
-            HIPX(hipMemcpyAsync(e->frame_ns.p, ones.data(), batch * sizeof(int), hipMemcpyHostToDevice, e->stream));
+            HIPX(hipMemcpyAsync(e->frame_ns.p, depth.data(), batch * sizeof(int), hipMemcpyHostToDevice, e->stream));
             HIPX(hipMemcpyAsync(e->frame_wcfg.p, ids.data(), batch * sizeof(int), hipMemcpyHostToDevice, e->stream));
             HIPX(hipMemcpyAsync(e->det_out.p, accum, (size_t)n_probes * n_det * sizeof(double),
                                 hipMemcpyHostToDevice, e->stream));
@@ -1870,11 +1882,11 @@ int mse_stem_batch_frames(mse_engine* e, int cfg, const double* pos_xy, const do
         }
         mse::PotArgs pa = pot_args(e, c);
         pa.frame_xy = e->frame_xy.p;
+        pa.frame_slices = cs;
         mse::RowArgs ra = base_row_args(e);
         ra.cfg_trans = e->frame_ptrs.p;
         ra.cfg_nslices = e->frame_ns.p;
         ra.wave_cfg = e->frame_wcfg.p;
-        ra.slice = 0;
         ra.mix_sets = 0;
         mse::ColArgs ca = base_col_args(e);
         mse::ColArgs da = base_col_args(e);
@@ -1905,8 +1917,13 @@ int mse_stem_batch_frames(mse_engine* e, int cfg, const double* pos_xy, const do
             }
             probes_into_waves(e, nb, probe);
             for (int s = 0; s < ns; ++s) {
-                potential_planes(e, c, g, pa, e->frame_trans.p, nb, s);
-                band_limit_planes(e, e->frame_trans.p, nb);
+                if (s % cs == 0) {
+                    // (the last group may reach past the specimen, by less than a slice per
+                    // group: its planes beyond are not read)
+                    potential_planes(e, c, g, pa, e->frame_trans.p, nb * cs, s);
+                    band_limit_planes(e, e->frame_trans.p, nb * cs);
+                }
+                ra.slice = s % cs;
                 slice_band(e, s == 0, ra, ca);
                 row_pass(e, mse::ROW_IFFT_T_FFT, e->waves.p, e->waves.p, nb, e->N, ra);
                 if (s == ns - 1)

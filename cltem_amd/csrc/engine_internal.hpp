@@ -270,7 +270,7 @@ int col_pass(mse_engine* e, int mode, const float2* in, float2* out, int nsets, 
 // a slice loop), which it clears; else the wave comes from a column pass.
 void slice_band(mse_engine* e, bool first, mse::RowArgs& ra, mse::ColArgs& ca);
 // exp(i sigma V) of `planes` planes into out from the sorted atoms of c: slices
-// first..first+planes-1, or with a.frame_xy set one plane per frame of slice `first`
+// first..first+planes-1, or with a.frame_xy set slices first..first+a.frame_slices-1 of each frame
 void potential_planes(mse_engine* e, const ConfigData& c, const mse_geometry& g, const mse::PotArgs& a,
                       float2* out, int planes, int first);
 // transmission band limit of `planes` planes in place: FFT, |k| <= 2/3 kmax, IFFT
