@@ -170,6 +170,7 @@ struct mse_engine {
     DevBuf<float2> scratch;
     DevBuf<float2> img_tmp;  // CTEM image formation work copy of the waves
     DevBuf<float> ccd_filter;  // sqrt(DQE) and NTF factors per pixel (2 res*res)
+    DevBuf<double> ccd_table;  // the DQE and NTF tables they are interpolated from
     // sort scratch
     DevBuf<double> tmp_xyz;
     DevBuf<int> tmp_Z, tmp_bid, tmp_zid;

@@ -1,7 +1,7 @@
 // CCD response and shot noise of a CTEM image (SimulationCtem::simulateImageDose,
 // microscope/simulationctem.cpp:174-263, with ccd_dqe / ccd_ntf, kernels/ccd_dqe_d.cl and
 // kernels/ccd_ntf_d.cl).  The two filters are radial tables interpolated per pixel on the
-// host in double; each filter is one row pass, one column pass with the filter fused and
+// device in double; each filter is one row pass, one column pass with the filter fused and
 // one row pass.  The Poisson noise uses a seeded counter-based generator (clTEM seeds
 // std::mt19937_64 from the clock, so its noise cannot be reproduced).
 #include "engine_internal.hpp"
@@ -9,25 +9,6 @@
 
 namespace mse_rt {
 namespace {
-
-// ccd_dqe_d / ccd_ntf_d: radius in pixels of the unshifted FFT, linear interpolation of the
-// table at radius / binning, indices clamped to the last entry.
-void radial_filter(int res, const double* table, int n_table, int binning, bool take_sqrt, float* out) {
-    for (int yid = 0; yid < res; ++yid)
-        for (int xid = 0; xid < res; ++xid) {
-            const int midx = xid < res / 2 ? 0 : res;
-            const int midy = yid < res / 2 ? 0 : res;
-            const double xp = xid - midx, yp = yid - midy;
-            const double rad = std::sqrt(xp * xp + yp * yp);
-            const int i0 = (int)std::floor(rad / binning);
-            const int i1 = i0 + 1;
-            const double v0 = table[std::min(i0, n_table - 1)];
-            const double v1 = table[std::min(i1, n_table - 1)];
-            const double interp = rad / binning - std::floor(rad / binning);
-            const double f = interp * v1 + (1 - interp) * v0;
-            out[(size_t)yid * res + xid] = (float)(take_sqrt ? std::sqrt(f) : f);
-        }
-}
 
 void filter_pass(mse_engine* e, float2* z, const float* filter) {
     mse::RowArgs ra = base_row_args(e);
@@ -55,16 +36,18 @@ extern "C" int mse_ccd_image(mse_engine* e, const double* image, const double* d
             REQUIRE(dqe[i] >= 0.0 && std::isfinite(dqe[i]) && std::isfinite(ntf[i]), MSE_ERR_ARG,
                     "DQE must be finite and >= 0, NTF finite");
         const size_t N = e->N;
-        std::vector<float> f(2 * N);
-        radial_filter(e->res, dqe, n_table, binning, true, f.data());
-        radial_filter(e->res, ntf, n_table, binning, false, f.data() + N);
         e->ccd_filter.ensure(2 * N);
+        e->ccd_table.ensure(2 * (size_t)n_table);
         e->img_tmp.ensure(N);
         e->diff_img.ensure(N);
-        HIPX(hipMemcpyAsync(e->ccd_filter.p, f.data(), 2 * N * sizeof(float), hipMemcpyHostToDevice, e->stream));
+        HIPX(hipMemcpyAsync(e->ccd_table.p, dqe, n_table * sizeof(double), hipMemcpyHostToDevice, e->stream));
+        HIPX(hipMemcpyAsync(e->ccd_table.p + n_table, ntf, n_table * sizeof(double), hipMemcpyHostToDevice, e->stream));
+        const unsigned blocks = (unsigned)((N + 255) / 256);
+        launch(e, PK_OTHER, [&]() {
+            mse::k_radial_filters<<<blocks, 256, 0, e->stream>>>(e->ccd_filter.p, e->res, e->ccd_table.p, n_table, binning);
+        });
         HIPX(hipMemcpyAsync(e->diff_img.p, image, N * sizeof(double), hipMemcpyHostToDevice, e->stream));
         float2* z = e->img_tmp.p;
-        const unsigned blocks = (unsigned)((N + 255) / 256);
         launch(e, PK_OTHER, [&]() { mse::k_real_to_complex<<<blocks, 256, 0, e->stream>>>(e->diff_img.p, z, N); });
         filter_pass(e, z, e->ccd_filter.p);  // DQE
         const double n_tot = dose_per_pixel * binning * binning;  // simulationctem.cpp:229
