@@ -21,20 +21,16 @@ struct BinGeom {
     int blocks_x, blocks_y, n_slices;
 };
 
-static __global__ void k_bin_atoms(const double* __restrict__ x, const double* __restrict__ y,
-                            const double* __restrict__ z, int n, BinGeom g, unsigned* __restrict__ key,
-                            unsigned* __restrict__ idx, int* __restrict__ bid_out,
-                            int* __restrict__ zid_out) {
+// bin (block and slice, -1 where out of range) and sort key (slice * blocks + block, or the number
+// of bins) of one atom
+__device__ __forceinline__ unsigned bin_key(double xi, double yi, double zi, const BinGeom& g, int& bid, int& zid) {
 #pragma clang fp contract(off)
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
     const unsigned out_key = (unsigned)(g.n_slices * g.blocks_x * g.blocks_y);
-    const double xi = x[i], yi = y[i], zi = z[i];
     // host filter (simulationgeneral.cpp:206-210): strict against padded limits
     const bool in_x = xi > g.full_x0 && xi < g.full_x1;
     const bool in_y = yi > g.full_y0 && yi < g.full_y1;
     const bool in_z = zi > g.z0 && zi < g.z1;
-    int bid = -1, zid = -1;
+    bid = zid = -1;
     unsigned k = out_key;
     if (in_x && in_y && in_z) {
         const double min_x = g.full_x0, max_x = g.full_x1, min_y = g.full_y0, max_y = g.full_y1;
@@ -52,10 +48,141 @@ static __global__ void k_bin_atoms(const double* __restrict__ x, const double* _
                 k = (unsigned)(zid * g.blocks_x * g.blocks_y + bid);
         }
     }
-    key[i] = k;
+    return k;
+}
+
+static __global__ void k_bin_atoms(const double* __restrict__ x, const double* __restrict__ y,
+                            const double* __restrict__ z, int n, BinGeom g, unsigned* __restrict__ key,
+                            unsigned* __restrict__ idx, int* __restrict__ bid_out,
+                            int* __restrict__ zid_out) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    key[i] = bin_key(x[i], y[i], z[i], g, bid_out[i], zid_out[i]);
     idx[i] = (unsigned)i;
-    bid_out[i] = bid;
-    zid_out[i] = zid;
+}
+
+// Stable counting sort in three launches, for bin counts that fit a block's LDS: the radix sort
+// of the keys, its search for the bins' starts and the gather are a dozen launches whose gaps
+// and round trips are the whole time at these sizes (51,200 atoms in 747 bins: about 95 us of
+// small kernels; these three take about 22 us).
+//
+// k_bin_count: 256 atoms per block; key[i], the atom's rank among the block's earlier atoms of the
+// same bin, and the block's histogram (row blockIdx.x of hist, nkeys wide; out-of-range atoms are
+// not counted).  Dynamic LDS: nkeys counters.
+static __global__ __launch_bounds__(256) void k_bin_count(const double* __restrict__ x, const double* __restrict__ y,
+                                                          const double* __restrict__ z, int n, BinGeom g, int nkeys,
+                                                          unsigned* __restrict__ key, unsigned* __restrict__ rank,
+                                                          int* __restrict__ bid_out, int* __restrict__ zid_out,
+                                                          unsigned* __restrict__ hist) {
+    extern __shared__ unsigned count[];
+    __shared__ uint4 keys4[64];
+    unsigned* keys = reinterpret_cast<unsigned*>(keys4);
+    const int t = threadIdx.x, i = blockIdx.x * 256 + t;
+    for (int k = t; k < nkeys; k += 256) count[k] = 0;
+    unsigned mine = (unsigned)nkeys;
+    if (i < n) {
+        int bid, zid;
+        mine = bin_key(x[i], y[i], z[i], g, bid, zid);
+        key[i] = mine;
+        bid_out[i] = bid;
+        zid_out[i] = zid;
+    }
+    keys[t] = mine;
+    __syncthreads();
+    if (mine < (unsigned)nkeys) atomicAdd(&count[mine], 1u);
+    unsigned before = 0;
+    const int last = (t >> 6) * 16 + 16;  // this wave's own atoms at most
+#pragma unroll 4
+    for (int q = 0; q < last; ++q) {
+        const uint4 k = keys4[q];
+        const int j = 4 * q;
+        before += (k.x == mine && j < t) + (k.y == mine && j + 1 < t) + (k.z == mine && j + 2 < t) +
+                  (k.w == mine && j + 3 < t);
+    }
+    if (i < n) rank[i] = before;
+    __syncthreads();
+    unsigned* row = hist + (size_t)blockIdx.x * nkeys;
+    for (int k = t; k < nkeys; k += 256) row[k] = count[k];
+}
+
+// Each bin's column of hist (rows = atom blocks) to its exclusive prefix over the rows, and the
+// bin's total.  64 bins per block, the rows in 16 segments.
+static __global__ __launch_bounds__(1024) void k_bin_prefix(unsigned* __restrict__ hist, int rows, int nkeys,
+                                                            unsigned* __restrict__ total) {
+    __shared__ unsigned seg_sum[16][64];
+    const int lane = threadIdx.x & 63, seg = threadIdx.x >> 6;
+    const int k = blockIdx.x * 64 + lane;
+    const int per = (rows + 15) / 16, r0 = min(rows, seg * per), r1 = min(rows, r0 + per);
+    unsigned sum = 0;
+    if (k < nkeys) {
+#pragma unroll 8
+        for (int r = r0; r < r1; ++r) sum += hist[(size_t)r * nkeys + k];
+    }
+    seg_sum[seg][lane] = sum;
+    __syncthreads();
+    if (k >= nkeys) return;
+    unsigned run = 0;
+    for (int q = 0; q < seg; ++q) run += seg_sum[q][lane];
+    if (seg == 15) total[k] = run + sum;
+    // 8 rows at a time, their loads together (the stores would order them otherwise)
+    for (int r = r0; r < r1; r += 8) {
+        unsigned c[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) c[q] = r + q < r1 ? hist[(size_t)(r + q) * nkeys + k] : 0u;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            if (r + q < r1) hist[(size_t)(r + q) * nkeys + k] = run;
+            run += c[q];
+        }
+    }
+}
+
+// The bins' starts (every block scans the totals; block 0 writes block_start, nkeys + 1 entries)
+// and each atom to its place: start of its bin + its bin's atoms in earlier blocks + its rank.
+// Dynamic LDS: nkeys + 1 starts.
+static __global__ __launch_bounds__(256) void k_bin_place(
+    const double* __restrict__ x, const double* __restrict__ y, const double* __restrict__ z, const int* __restrict__ Z,
+    int n, int nkeys, const unsigned* __restrict__ key, const unsigned* __restrict__ rank,
+    const unsigned* __restrict__ hist, const unsigned* __restrict__ total, int* __restrict__ block_start,
+    double* __restrict__ sx, double* __restrict__ sy, double* __restrict__ sz, int* __restrict__ sZ,
+    int* __restrict__ orig) {
+    extern __shared__ unsigned start[];
+    __shared__ unsigned part[256];
+    const int t = threadIdx.x;
+    for (int k = t; k < nkeys; k += 256) start[k] = total[k];
+    __syncthreads();
+    // thread t scans bins [t per, (t + 1) per)
+    const int per = (nkeys + 255) / 256, k0 = min(nkeys, t * per), k1 = min(nkeys, k0 + per);
+    unsigned sum = 0;
+    for (int k = k0; k < k1; ++k) sum += start[k];
+    part[t] = sum;
+    __syncthreads();
+    for (int d = 1; d < 256; d *= 2) {
+        const unsigned add = t >= d ? part[t - d] : 0u;
+        __syncthreads();
+        part[t] += add;
+        __syncthreads();
+    }
+    unsigned run = part[t] - sum;
+    for (int k = k0; k < k1; ++k) {
+        const unsigned c = start[k];
+        start[k] = run;
+        run += c;
+    }
+    if (t == 255) start[nkeys] = part[255];
+    __syncthreads();
+    if (blockIdx.x == 0)
+        for (int k = t; k <= nkeys; k += 256) block_start[k] = (int)start[k];
+    const int i = blockIdx.x * 256 + t;
+    if (i >= n) return;
+    const unsigned mine = key[i];
+    if (mine >= (unsigned)nkeys) return;
+    const unsigned p = start[mine] + hist[(size_t)blockIdx.x * nkeys + mine] + rank[i];
+    sx[p] = x[i];
+    sy[p] = y[i];
+    sz[p] = z[i];
+    sZ[p] = Z[i];
+    orig[p] = i;
 }
 
 // block_start[k] = first sorted position with key >= k, for k in [0, nkeys]

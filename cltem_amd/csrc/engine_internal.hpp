@@ -176,6 +176,7 @@ struct mse_engine {
     DevBuf<int> tmp_Z, tmp_bid, tmp_zid;
     DevBuf<unsigned> keys, keys_sorted, idx, idx_sorted;
     DevBuf<unsigned char> cub_tmp;
+    DevBuf<unsigned> bin_hist;  // counting sort: per 256 atoms a histogram of the bins, then the bins' totals
     // kernel variants set by mse_set_kernel_variant, for every wave count; -1: by the sweeps'
     // own rule on the grid size and the wave count
     int row_var = -1, col_var = -1;
