@@ -192,9 +192,9 @@ class Engine:
         Z = np.ascontiguousarray(Z, dtype=np.int32)
         n = len(x)
         g = self.config_geometry(config)
-        bs = np.zeros(g.n_slices * g.blocks_x * g.blocks_y + 1, dtype=np.int32)
-        bid = np.zeros(max(n, 1), dtype=np.int32)
-        zid = np.zeros(max(n, 1), dtype=np.int32)
+        bs = np.empty(g.n_slices * g.blocks_x * g.blocks_y + 1, dtype=np.int32)
+        # without want_ids they stay zeros
+        bid, zid = ((np.empty if want_ids else np.zeros)(max(n, 1), dtype=np.int32) for _ in range(2))
         nr = C.c_int(0)
         nullp = C.POINTER(C.c_int)()
         _check(self.lib.mse_sort_atoms(self.h, config, _dp(x), _dp(y), _dp(z), _ip(Z), n,
@@ -208,7 +208,7 @@ class Engine:
 
     def read_transmission(self, config: int, slice_: int) -> np.ndarray:
         res = self.g.resolution
-        out = np.zeros(2 * res * res, dtype=np.float32)
+        out = np.empty(2 * res * res, dtype=np.float32)
         _check(self.lib.mse_read_transmission(self.h, config, slice_,
                                               out.ctypes.data_as(C.POINTER(C.c_float))))
         return out.view(np.complex64).reshape(res, res)
@@ -274,13 +274,13 @@ class Engine:
 
     def diffraction(self, wave: int = 0) -> np.ndarray:
         res = self.g.resolution
-        out = np.zeros((res, res))
+        out = np.empty((res, res))
         _check(self.lib.mse_diffraction(self.h, wave, _dp(out)))
         return out
 
     def exit_wave(self, wave: int = 0) -> np.ndarray:
         res = self.g.resolution
-        out = np.zeros(2 * res * res)
+        out = np.empty(2 * res * res)
         _check(self.lib.mse_exit_wave(self.h, wave, _dp(out)))
         return out.view(np.complex128).reshape(res, res)
 
@@ -288,7 +288,7 @@ class Engine:
         """CTEM image (objective aperture, aberrations, coherence envelopes) of every wave,
         summed over the waves in FP64; the exit waves are kept."""
         res = self.g.resolution
-        out = np.zeros((res, res)) if accum is None else accum
+        out = np.empty((res, res)) if accum is None else accum
         assert out.shape == (res, res) and out.dtype == np.float64 and out.flags.c_contiguous
         _check(self.lib.mse_ctem_image(self.h, C.byref(imaging), int(accum is not None), _dp(out)))
         return out
@@ -301,14 +301,14 @@ class Engine:
         d = np.ascontiguousarray(dqe, dtype=np.float64)
         n = np.ascontiguousarray(ntf, dtype=np.float64)
         assert img.shape == (res, res) and d.shape == n.shape
-        out = np.zeros((res, res))
+        out = np.empty((res, res))
         _check(self.lib.mse_ccd_image(self.h, _dp(img), _dp(d), _dp(n), len(d), binning, dose_per_pixel,
                                       conversion, C.c_ulonglong(seed), _dp(out)))
         return out
 
     def exit_intensity_sum(self, accum=None) -> np.ndarray:
         res = self.g.resolution
-        out = np.zeros((res, res)) if accum is None else accum
+        out = np.empty((res, res)) if accum is None else accum
         assert out.shape == (res, res) and out.dtype == np.float64 and out.flags.c_contiguous
         _check(self.lib.mse_exit_intensity_sum(self.h, int(accum is not None), _dp(out)))
         return out
@@ -316,7 +316,7 @@ class Engine:
     def diffraction_sum(self, wave_group, n_groups: int, accum=None) -> np.ndarray:
         res = self.g.resolution
         grp = np.ascontiguousarray(wave_group, dtype=np.int32)
-        out = np.zeros((n_groups, res, res)) if accum is None else accum
+        out = np.empty((n_groups, res, res)) if accum is None else accum
         assert out.shape == (n_groups, res, res) and out.dtype == np.float64 and out.flags.c_contiguous
         _check(self.lib.mse_diffraction_sum(self.h, _ip(grp), n_groups, int(accum is not None), _dp(out)))
         return out
@@ -326,7 +326,7 @@ class Engine:
         (within the checkpoint budget) or sqrt(n) checkpoints for adjoint_positions; returns
         |psi_exit|^2, shape (n_waves, res, res)."""
         res = self.g.resolution
-        out = np.zeros((self.n_waves, res, res))
+        out = np.empty((self.n_waves, res, res))
         _check(self.lib.mse_forward_checkpointed(self.h, config, _dp(out)))
         return out
 

@@ -84,9 +84,10 @@ int mse_forward_checkpointed(mse_engine* e, int cfg, double* intensity) {
             ra.scale = (float)(1.0 / e->res);
             ra.dout = e->diff_img.p;
             row_pass(e, mse::ROW_IFFT_INTENSITY, e->waves.p, e->scratch.p, nw, e->N, ra);
-            HIPX(hipMemcpyAsync(intensity, e->diff_img.p, plane * sizeof(double), hipMemcpyDeviceToHost, e->stream));
+            download(e, intensity, e->diff_img.p, plane * sizeof(double));
+        } else {
+            HIPX(hipStreamSynchronize(e->stream));
         }
-        HIPX(hipStreamSynchronize(e->stream));
         e->adj_cfg = cfg;
         e->adj_k = K;
         e->adj_nw = nw;
@@ -118,7 +119,7 @@ int mse_adjoint_positions(mse_engine* e, const double* dl_di, double* grad_xyz) 
 
         // dL/dI, phases phi_s and the gradient accumulator
         e->adj_w.ensure(plane);
-        HIPX(hipMemcpyAsync(e->adj_w.p, dl_di, plane * sizeof(double), hipMemcpyHostToDevice, e->stream));
+        upload(e, e->adj_w.p, dl_di, plane * sizeof(double));
         e->adj_phase.ensure((size_t)std::max(n, 1) * N);
         require_elements(e, c);
         mse::PotArgs pa = pot_args(e, c);
@@ -251,9 +252,9 @@ int mse_adjoint_positions(mse_engine* e, const double* dl_di, double* grad_xyz) 
             }
         }
         if (n_atoms > 0)
-            HIPX(hipMemcpyAsync(grad_xyz, e->adj_grad.p, 3 * (size_t)n_atoms * sizeof(double), hipMemcpyDeviceToHost,
-                                e->stream));
-        HIPX(hipStreamSynchronize(e->stream));
+            download(e, grad_xyz, e->adj_grad.p, 3 * (size_t)n_atoms * sizeof(double));
+        else
+            HIPX(hipStreamSynchronize(e->stream));
     });
 }
 

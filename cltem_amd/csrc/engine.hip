@@ -69,6 +69,128 @@ void* noalloc_scratch(int device) {
     return p;
 }
 
+// Pinned staging memory for copies from and to pageable host memory: at most kStages buffers of
+// kStageBytes in the process, made on first use, shared by all engines and threads and given back
+// when the last engine is destroyed.  A copy takes one buffer for itself until its transfers have
+// finished; while none is free (more threads copying than buffers) a copy goes without.
+constexpr int kStages = 4;
+constexpr size_t kStageBytes = size_t(4) << 20, kStageChunk = size_t(1) << 20;
+constexpr int kStageChunks = (int)(kStageBytes / kStageChunk);
+
+struct Stage {
+    int device = -1;                    // the events' device
+    unsigned char* p = nullptr;
+    hipEvent_t done[kStageChunks] = {}; // the last transfer of each chunk
+    bool used[kStageChunks] = {};
+    bool taken = false;
+};
+std::mutex g_stage_mu;
+Stage g_stages[kStages];
+int g_engines = 0;
+
+void release_stage(Stage& s) {
+    for (auto& ev : s.done)
+        if (ev) (void)hipEventDestroy(ev);
+    if (s.p) (void)hipHostFree(s.p);
+    s = Stage();
+}
+
+// a free buffer whose events belong to `device`; NULL while there is none
+Stage* take_stage(int device) {
+    std::lock_guard<std::mutex> lk(g_stage_mu);
+    Stage* empty = nullptr;
+    for (Stage& s : g_stages) {
+        if (s.taken) continue;
+        if (s.p && s.device == device) {
+            s.taken = true;
+            return &s;
+        }
+        if (!s.p) empty = &s;
+    }
+    if (!empty) return nullptr;
+    bool ok = hipHostMalloc((void**)&empty->p, kStageBytes, hipHostMallocDefault) == hipSuccess;
+    for (auto& ev : empty->done) ok = ok && hipEventCreateWithFlags(&ev, hipEventDisableTiming) == hipSuccess;
+    if (!ok) {
+        (void)hipGetLastError();  // the copy goes without
+        release_stage(*empty);
+        return nullptr;
+    }
+    empty->device = device;
+    empty->taken = true;
+    return empty;
+}
+
+// One copy's hold on a staging buffer; its destructor waits for the buffer's transfers.
+struct StageHold {
+    Stage* s;
+    explicit StageHold(int device) : s(device >= 0 ? take_stage(device) : nullptr) {}  // -1: no buffer
+    ~StageHold() {
+        if (!s) return;
+        for (int i = 0; i < kStageChunks; ++i) {
+            if (s->used[i]) (void)hipEventSynchronize(s->done[i]);
+            s->used[i] = false;
+        }
+        std::lock_guard<std::mutex> lk(g_stage_mu);
+        s->taken = false;
+    }
+    StageHold(const StageHold&) = delete;
+    StageHold& operator=(const StageHold&) = delete;
+};
+
+void download(mse_engine* e, void* dst, const void* src, size_t bytes) {
+    StageHold hold(e->device);
+    Stage* s = hold.s;
+    if (!s) {
+        HIPX(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, e->stream));
+        HIPX(hipStreamSynchronize(e->stream));
+        return;
+    }
+    if (bytes <= kStageChunk) {
+        HIPX(hipMemcpyAsync(s->p, src, bytes, hipMemcpyDeviceToHost, e->stream));
+        HIPX(hipStreamSynchronize(e->stream));
+        std::memcpy(dst, s->p, bytes);
+        return;
+    }
+    // chunk i lands in part i % kStageChunks while the chunks before it are copied out
+    const size_t n = (bytes + kStageChunk - 1) / kStageChunk;
+    for (size_t i = 0; i < n + kStageChunks - 1; ++i) {
+        if (i >= (size_t)kStageChunks - 1) {
+            const size_t j = i - (kStageChunks - 1), at = j * kStageChunk;
+            const int part = (int)(j % kStageChunks);
+            HIPX(hipEventSynchronize(s->done[part]));
+            s->used[part] = false;
+            std::memcpy((unsigned char*)dst + at, s->p + part * kStageChunk, std::min(kStageChunk, bytes - at));
+        }
+        if (i < n) {
+            const size_t at = i * kStageChunk;
+            const int part = (int)(i % kStageChunks);
+            HIPX(hipMemcpyAsync(s->p + part * kStageChunk, (const unsigned char*)src + at, std::min(kStageChunk, bytes - at),
+                                hipMemcpyDeviceToHost, e->stream));
+            HIPX(hipEventRecord(s->done[part], e->stream));
+            s->used[part] = true;
+        }
+    }
+}
+
+void upload(mse_engine* e, void* dst, const void* src, size_t bytes) {
+    StageHold hold(e->device);
+    Stage* s = hold.s;
+    if (!s) {
+        HIPX(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, e->stream));
+        HIPX(hipStreamSynchronize(e->stream));
+        return;
+    }
+    for (size_t at = 0, i = 0; at < bytes; at += kStageChunk, ++i) {
+        const int part = (int)(i % kStageChunks);
+        const size_t len = std::min(kStageChunk, bytes - at);
+        if (s->used[part]) HIPX(hipEventSynchronize(s->done[part]));
+        std::memcpy(s->p + part * kStageChunk, (const unsigned char*)src + at, len);
+        HIPX(hipMemcpyAsync((unsigned char*)dst + at, s->p + part * kStageChunk, len, hipMemcpyHostToDevice, e->stream));
+        HIPX(hipEventRecord(s->done[part], e->stream));
+        s->used[part] = true;
+    }
+}
+
 struct DeviceGuard {
     int prev = -1;
     explicit DeviceGuard(int dev) {
@@ -444,6 +566,8 @@ int mse_create(int device_ordinal, mse_engine** out) {
             throw Error(MSE_ERR_HIP, std::string("hipStreamCreate: ") + hipGetErrorString(st));
         }
         *out = e;
+        std::lock_guard<std::mutex> lk(g_stage_mu);
+        ++g_engines;
     });
 }
 
@@ -461,6 +585,10 @@ int mse_destroy(mse_engine* e) {
         hipStream_t s = e->stream;
         delete e;
         (void)hipStreamDestroy(s);
+        std::lock_guard<std::mutex> lk(g_stage_mu);
+        if (--g_engines == 0)
+            for (Stage& st : g_stages)
+                if (!st.taken) release_stage(st);
     });
     return rc;
 }
@@ -714,8 +842,7 @@ int mse_sort_atoms(mse_engine* e, int cfg, const double* x, const double* y, con
         const long long nkeys = (long long)g.n_slices * nblk;
         REQUIRE(nkeys < (1LL << 30), MSE_ERR_UNSUPPORTED, "too many bins");
         const size_t na = std::max(n, 1);
-        e->tmp_xyz.ensure(3 * na);
-        e->tmp_Z.ensure(na);
+        e->tmp_xyz.ensure(3 * na + (na + 1) / 2);  // x, y, z, then Z
         e->tmp_bid.ensure(na);
         e->tmp_zid.ensure(na);
         e->keys.ensure(na);
@@ -731,11 +858,26 @@ int mse_sort_atoms(mse_engine* e, int cfg, const double* x, const double* y, con
         double* dx = e->tmp_xyz.p;
         double* dy = dx + na;
         double* dzp = dy + na;
+        int* dZ = reinterpret_cast<int*>(dzp + na);
+        // atoms in and bins out through one staging buffer, one transfer each way
+        const size_t in_bytes = (size_t)n * (3 * sizeof(double) + sizeof(int));
+        const size_t out_ints = 2 * (size_t)n + (size_t)nkeys + 1;
+        StageHold hold(std::max(in_bytes, out_ints * sizeof(int)) <= kStageBytes ? e->device : -1);
         if (n > 0) {
-            HIPX(hipMemcpyAsync(dx, x, n * sizeof(double), hipMemcpyHostToDevice, e->stream));
-            HIPX(hipMemcpyAsync(dy, y, n * sizeof(double), hipMemcpyHostToDevice, e->stream));
-            HIPX(hipMemcpyAsync(dzp, z, n * sizeof(double), hipMemcpyHostToDevice, e->stream));
-            HIPX(hipMemcpyAsync(e->tmp_Z.p, Z, n * sizeof(int), hipMemcpyHostToDevice, e->stream));
+            if (hold.s) {
+                unsigned char* h = hold.s->p;
+                const size_t d = (size_t)n * sizeof(double);
+                std::memcpy(h, x, d);
+                std::memcpy(h + d, y, d);
+                std::memcpy(h + 2 * d, z, d);
+                std::memcpy(h + 3 * d, Z, (size_t)n * sizeof(int));
+                HIPX(hipMemcpyAsync(dx, h, in_bytes, hipMemcpyHostToDevice, e->stream));
+            } else {
+                HIPX(hipMemcpyAsync(dx, x, n * sizeof(double), hipMemcpyHostToDevice, e->stream));
+                HIPX(hipMemcpyAsync(dy, y, n * sizeof(double), hipMemcpyHostToDevice, e->stream));
+                HIPX(hipMemcpyAsync(dzp, z, n * sizeof(double), hipMemcpyHostToDevice, e->stream));
+                HIPX(hipMemcpyAsync(dZ, Z, n * sizeof(int), hipMemcpyHostToDevice, e->stream));
+            }
             mse::BinGeom bg{g.full_x[0], g.full_x[1], g.full_y[0], g.full_y[1], g.z_lims[0], g.z_lims[1],
                             g.slice_thickness, g.blocks_x, g.blocks_y, g.n_slices};
             // Rule: the counting sort where a block's LDS holds the bins and the blocks' histograms
@@ -755,11 +897,10 @@ int mse_sort_atoms(mse_engine* e, int cfg, const double* x, const double* y, con
                     mse::k_bin_prefix<<<(unsigned)((nkeys + 63) / 64), 1024, 0, e->stream>>>(e->bin_hist.p, rows, (int)nkeys, total);
                 });
                 launch(e, PK_OTHER, [&]() {
-                    mse::k_bin_place<<<rows, 256, lds, e->stream>>>(dx, dy, dzp, e->tmp_Z.p, n, (int)nkeys, e->keys.p,
+                    mse::k_bin_place<<<rows, 256, lds, e->stream>>>(dx, dy, dzp, dZ, n, (int)nkeys, e->keys.p,
                                                                     e->idx.p, e->bin_hist.p, total, c.block_start.p,
                                                                     c.x.p, c.y.p, c.z.p, c.Z.p, c.orig.p);
                 });
-                HIPX(hipMemcpyAsync(&nr, c.block_start.p + nkeys, sizeof(int), hipMemcpyDeviceToHost, e->stream));
             } else {
                 launch(e, PK_OTHER, [&]() {
                     mse::k_bin_atoms<<<(n + 255) / 256, 256, 0, e->stream>>>(dx, dy, dzp, n, bg, e->keys.p, e->idx.p,
@@ -782,7 +923,7 @@ int mse_sort_atoms(mse_engine* e, int cfg, const double* x, const double* y, con
                 if (nr > 0) {
                     launch(e, PK_OTHER, [&]() {
                         mse::k_gather_atoms<<<(nr + 255) / 256, 256, 0, e->stream>>>(e->idx_sorted.p, nr, dx, dy, dzp,
-                                                                                   e->tmp_Z.p, c.x.p, c.y.p, c.z.p, c.Z.p);
+                                                                                   dZ, c.x.p, c.y.p, c.z.p, c.Z.p);
                     });
                     c.orig.ensure(nr);
                     HIPX(hipMemcpyAsync(c.orig.p, e->idx_sorted.p, nr * sizeof(int), hipMemcpyDeviceToDevice, e->stream));
@@ -793,14 +934,31 @@ int mse_sort_atoms(mse_engine* e, int cfg, const double* x, const double* y, con
             HIPX(hipMemcpyAsync(c.block_start.p, zeros.data(), zeros.size() * sizeof(int), hipMemcpyHostToDevice,
                                 e->stream));
         }
-        if (block_ids && n > 0)
-            HIPX(hipMemcpyAsync(block_ids, e->tmp_bid.p, n * sizeof(int), hipMemcpyDeviceToHost, e->stream));
-        if (z_ids && n > 0)
-            HIPX(hipMemcpyAsync(z_ids, e->tmp_zid.p, n * sizeof(int), hipMemcpyDeviceToHost, e->stream));
-        if (block_start)
-            HIPX(hipMemcpyAsync(block_start, c.block_start.p, (nkeys + 1) * sizeof(int), hipMemcpyDeviceToHost,
-                                e->stream));
-        HIPX(hipStreamSynchronize(e->stream));
+        if (hold.s) {
+            // [bin starts][block ids][slice ids], as far as asked for
+            int* h = reinterpret_cast<int*>(hold.s->p);
+            const size_t first = block_start ? 0 : (size_t)nkeys, starts = (size_t)nkeys + 1 - first;
+            HIPX(hipMemcpyAsync(h, c.block_start.p + first, starts * sizeof(int), hipMemcpyDeviceToHost, e->stream));
+            if (block_ids && n > 0)
+                HIPX(hipMemcpyAsync(h + starts, e->tmp_bid.p, n * sizeof(int), hipMemcpyDeviceToHost, e->stream));
+            if (z_ids && n > 0)
+                HIPX(hipMemcpyAsync(h + starts + n, e->tmp_zid.p, n * sizeof(int), hipMemcpyDeviceToHost, e->stream));
+            HIPX(hipStreamSynchronize(e->stream));
+            nr = h[starts - 1];
+            if (block_start) std::memcpy(block_start, h, starts * sizeof(int));
+            if (block_ids && n > 0) std::memcpy(block_ids, h + starts, n * sizeof(int));
+            if (z_ids && n > 0) std::memcpy(z_ids, h + starts + n, n * sizeof(int));
+        } else {
+            HIPX(hipMemcpyAsync(&nr, c.block_start.p + nkeys, sizeof(int), hipMemcpyDeviceToHost, e->stream));
+            if (block_ids && n > 0)
+                HIPX(hipMemcpyAsync(block_ids, e->tmp_bid.p, n * sizeof(int), hipMemcpyDeviceToHost, e->stream));
+            if (z_ids && n > 0)
+                HIPX(hipMemcpyAsync(z_ids, e->tmp_zid.p, n * sizeof(int), hipMemcpyDeviceToHost, e->stream));
+            if (block_start)
+                HIPX(hipMemcpyAsync(block_start, c.block_start.p, (nkeys + 1) * sizeof(int), hipMemcpyDeviceToHost,
+                                    e->stream));
+            HIPX(hipStreamSynchronize(e->stream));
+        }
         c.n_in_range = nr;
         if (n_in_range) *n_in_range = c.n_in_range;
         c.n_input = n;
@@ -850,9 +1008,7 @@ int mse_read_transmission(mse_engine* e, int cfg, int slice, float* out) {
         ConfigData& c = config(e, cfg);
         REQUIRE(c.trans.p && c.built, MSE_ERR_STATE, "no transmission functions for this configuration");
         REQUIRE(slice >= 0 && slice < cfg_geom(e, c).n_slices, MSE_ERR_ARG, "slice out of range");
-        HIPX(hipMemcpyAsync(out, c.trans.p + (size_t)slice * e->N, e->N * sizeof(float2), hipMemcpyDeviceToHost,
-                            e->stream));
-        HIPX(hipStreamSynchronize(e->stream));
+        download(e, out, c.trans.p + (size_t)slice * e->N, e->N * sizeof(float2));
     });
 }
 
@@ -1637,8 +1793,7 @@ int mse_stem_detect(mse_engine* e, const mse_detector* dets, int n_det, int sqrt
             e->det_tiles = col_pass(e, mse::COL_FFT_DETECT, e->waves.p, e->waves.p, nw, e->N, ca);
             reduce_detectors(e, nw, n_det, sqrt2, e->det_out.p, 0);
         }
-        HIPX(hipMemcpyAsync(out, e->det_out.p, (size_t)nw * n_det * sizeof(double), hipMemcpyDeviceToHost, e->stream));
-        HIPX(hipStreamSynchronize(e->stream));
+        download(e, out, e->det_out.p, (size_t)nw * n_det * sizeof(double));
     });
 }
 
@@ -1688,8 +1843,7 @@ int mse_diffraction(mse_engine* e, int wave, double* out) {
         check_waves(e);
         REQUIRE(wave >= 0 && wave < e->n_waves, MSE_ERR_ARG, "wave index out of range");
         const double* im = diffraction_images(e, wave, 1);  // translated when the beam moved
-        HIPX(hipMemcpyAsync(out, im, e->N * sizeof(double), hipMemcpyDeviceToHost, e->stream));
-        HIPX(hipStreamSynchronize(e->stream));
+        download(e, out, im, e->N * sizeof(double));
     });
 }
 
@@ -1698,17 +1852,13 @@ int mse_exit_wave(mse_engine* e, int wave, double* out) {
         REQUIRE(e && out, MSE_ERR_ARG, "NULL argument");
         check_waves(e);
         REQUIRE(wave >= 0 && wave < e->n_waves, MSE_ERR_ARG, "wave index out of range");
-        e->scratch.ensure(e->N);
+        // widened to double on the device: on one host thread the conversion took 170 us at 256^2
+        e->diff_img.ensure(2 * e->N);
         mse::RowArgs ra = base_row_args(e);
         ra.scale = (float)(1.0 / e->res);
-        row_pass(e, mse::ROW_IFFT, e->waves.p + (size_t)wave * e->N, e->scratch.p, 1, e->N, ra);
-        std::vector<float2> h(e->N);
-        HIPX(hipMemcpyAsync(h.data(), e->scratch.p, e->N * sizeof(float2), hipMemcpyDeviceToHost, e->stream));
-        HIPX(hipStreamSynchronize(e->stream));
-        for (size_t i = 0; i < e->N; ++i) {
-            out[2 * i] = h[i].x;
-            out[2 * i + 1] = h[i].y;
-        }
+        ra.dout = e->diff_img.p;
+        row_pass(e, mse::ROW_IFFT_WIDE, e->waves.p + (size_t)wave * e->N, nullptr, 1, e->N, ra);
+        download(e, out, e->diff_img.p, 2 * e->N * sizeof(double));
     });
 }
 
@@ -1836,9 +1986,7 @@ int mse_stem_batch(mse_engine* e, int cfg, const double* pos_xy, int n_probes, i
                 reduce_detectors(e, nb, n_det, sqrt2, e->det_out.p + (size_t)p0 * n_det, 1);
             }
         }
-        HIPX(hipMemcpyAsync(accum, e->det_out.p, (size_t)n_probes * n_det * sizeof(double), hipMemcpyDeviceToHost,
-                            e->stream));
-        HIPX(hipStreamSynchronize(e->stream));
+        download(e, accum, e->det_out.p, (size_t)n_probes * n_det * sizeof(double));
     });
 }
 
@@ -1961,9 +2109,7 @@ int mse_stem_batch_frames(mse_engine* e, int cfg, const double* pos_xy, const do
             // rel and the frames are reused by the next batch: its uploads must not overtake
             HIPX(hipStreamSynchronize(e->stream));
         }
-        HIPX(hipMemcpyAsync(accum, e->det_out.p, (size_t)n_probes * n_det * sizeof(double), hipMemcpyDeviceToHost,
-                            e->stream));
-        HIPX(hipStreamSynchronize(e->stream));
+        download(e, accum, e->det_out.p, (size_t)n_probes * n_det * sizeof(double));
     });
 }
 
@@ -2134,7 +2280,7 @@ int mse_ctem_image(mse_engine* e, const mse_imaging* im, int accumulate, double*
         e->diff_img.ensure((size_t)nw * e->N);
         e->det_out.ensure(e->N);
         if (accumulate)
-            HIPX(hipMemcpyAsync(e->det_out.p, out, e->N * sizeof(double), hipMemcpyHostToDevice, e->stream));
+            upload(e, e->det_out.p, out, e->N * sizeof(double));
         mse::RowArgs ra = base_row_args(e);
         ra.scale = 1.0f;
         ra.dout = e->diff_img.p;
@@ -2143,8 +2289,7 @@ int mse_ctem_image(mse_engine* e, const mse_imaging* im, int accumulate, double*
             mse::k_sum_waves<<<(unsigned)((e->N + 255) / 256), 256, 0, e->stream>>>(e->diff_img.p, nw, e->N,
                                                                                    e->det_out.p, accumulate);
         });
-        HIPX(hipMemcpyAsync(out, e->det_out.p, e->N * sizeof(double), hipMemcpyDeviceToHost, e->stream));
-        HIPX(hipStreamSynchronize(e->stream));
+        download(e, out, e->det_out.p, e->N * sizeof(double));
     });
 }
 
@@ -2156,7 +2301,7 @@ int mse_exit_intensity_sum(mse_engine* e, int accumulate, double* out) {
         e->diff_img.ensure((size_t)nw * e->N);
         e->det_out.ensure(e->N);
         if (accumulate)
-            HIPX(hipMemcpyAsync(e->det_out.p, out, e->N * sizeof(double), hipMemcpyHostToDevice, e->stream));
+            upload(e, e->det_out.p, out, e->N * sizeof(double));
         mse::RowArgs ra = base_row_args(e);
         ra.scale = (float)(1.0 / e->res);
         ra.dout = e->diff_img.p;
@@ -2165,8 +2310,7 @@ int mse_exit_intensity_sum(mse_engine* e, int accumulate, double* out) {
             mse::k_sum_waves<<<(unsigned)((e->N + 255) / 256), 256, 0, e->stream>>>(e->diff_img.p, nw, e->N,
                                                                                    e->det_out.p, accumulate);
         });
-        HIPX(hipMemcpyAsync(out, e->det_out.p, e->N * sizeof(double), hipMemcpyDeviceToHost, e->stream));
-        HIPX(hipStreamSynchronize(e->stream));
+        download(e, out, e->det_out.p, e->N * sizeof(double));
     });
 }
 
@@ -2183,16 +2327,13 @@ int mse_diffraction_sum(mse_engine* e, const int* wave_group, int n_groups, int 
         e->tmp_bid.ensure(nw);
         HIPX(hipMemcpyAsync(e->tmp_bid.p, wave_group, nw * sizeof(int), hipMemcpyHostToDevice, e->stream));
         if (accumulate)
-            HIPX(hipMemcpyAsync(e->det_out.p, out, (size_t)n_groups * e->N * sizeof(double), hipMemcpyHostToDevice,
-                                e->stream));
+            upload(e, e->det_out.p, out, (size_t)n_groups * e->N * sizeof(double));
         const double* im = diffraction_images(e, 0, nw);  // translated where a beam moved
         launch(e, PK_OTHER, [&]() {
             mse::k_sum_groups<<<(unsigned)((e->N + 255) / 256), 256, 0, e->stream>>>(
                 im, nw, e->N, e->tmp_bid.p, n_groups, e->det_out.p, accumulate);
         });
-        HIPX(hipMemcpyAsync(out, e->det_out.p, (size_t)n_groups * e->N * sizeof(double), hipMemcpyDeviceToHost,
-                            e->stream));
-        HIPX(hipStreamSynchronize(e->stream));
+        download(e, out, e->det_out.p, (size_t)n_groups * e->N * sizeof(double));
     });
 }
 

@@ -173,7 +173,7 @@ struct mse_engine {
     DevBuf<double> ccd_table;  // the DQE and NTF tables they are interpolated from
     // sort scratch
     DevBuf<double> tmp_xyz;
-    DevBuf<int> tmp_Z, tmp_bid, tmp_zid;
+    DevBuf<int> tmp_bid, tmp_zid;
     DevBuf<unsigned> keys, keys_sorted, idx, idx_sorted;
     DevBuf<unsigned char> cub_tmp;
     DevBuf<unsigned> bin_hist;  // counting sort: per 256 atoms a histogram of the bins, then the bins' totals
@@ -251,6 +251,15 @@ inline void launch(mse_engine* e, int kind, F&& f) {
 // variant arguments of row_pass / col_pass: the engine's choice (tuned, else set, else by rule), or
 // the sweeps' rule whatever was tuned or set
 constexpr int kEngineChoice = -1, kRule = -2;
+
+// ---- host copies -----------------------------------------------------------------------------
+// Copies between a caller's pageable memory and the device, through pinned staging memory.  The
+// runtime's own pageable copies stage or pin call by call: 64 KiB to the host takes it 35 us,
+// 512 KiB 230 us and 8 MiB 490 us, where a pinned transfer takes 9, 17 and 156 us and the memcpy
+// (of lines the transfer has put out of the caches) about as long again.
+// Both go by the engine's stream and are complete on return.
+void download(mse_engine* e, void* dst, const void* src, size_t bytes);
+void upload(mse_engine* e, void* dst, const void* src, size_t bytes);
 
 // ---- helpers defined in engine.hip ---------------------------------------------------------
 // potential-kernel arguments for a configuration's geometry

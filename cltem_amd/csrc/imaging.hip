@@ -46,7 +46,7 @@ extern "C" int mse_ccd_image(mse_engine* e, const double* image, const double* d
         launch(e, PK_OTHER, [&]() {
             mse::k_radial_filters<<<blocks, 256, 0, e->stream>>>(e->ccd_filter.p, e->res, e->ccd_table.p, n_table, binning);
         });
-        HIPX(hipMemcpyAsync(e->diff_img.p, image, N * sizeof(double), hipMemcpyHostToDevice, e->stream));
+        upload(e, e->diff_img.p, image, N * sizeof(double));
         float2* z = e->img_tmp.p;
         launch(e, PK_OTHER, [&]() { mse::k_real_to_complex<<<blocks, 256, 0, e->stream>>>(e->diff_img.p, z, N); });
         filter_pass(e, z, e->ccd_filter.p);  // DQE
@@ -55,7 +55,6 @@ extern "C" int mse_ccd_image(mse_engine* e, const double* image, const double* d
         launch(e, PK_OTHER, [&]() { mse::k_shot_noise<<<blocks, 256, 0, e->stream>>>(z, N, n_tot, conversion, key); });
         filter_pass(e, z, e->ccd_filter.p + N);  // NTF
         launch(e, PK_OTHER, [&]() { mse::k_real_part<<<blocks, 256, 0, e->stream>>>(z, e->diff_img.p, N); });
-        HIPX(hipMemcpyAsync(out, e->diff_img.p, N * sizeof(double), hipMemcpyDeviceToHost, e->stream));
-        HIPX(hipStreamSynchronize(e->stream));
+        download(e, out, e->diff_img.p, N * sizeof(double));
     });
 }

@@ -31,10 +31,11 @@ namespace mse {
 enum RowMode : int {
     ROW_IFFT_T_FFT = 0,   // slice step, row half
     ROW_FFT = 2,          // forward x-DFT (transmission band limit, step 1)
-    ROW_IFFT = 3,         // inverse x-DFT (band limit step 3, exit-wave readback)
+    ROW_IFFT = 3,         // inverse x-DFT (band limit step 3)
     ROW_COPY = 4,         // read and write the rows only (bandwidth reference)
     ROW_IFFT_INTENSITY = 5,  // |inverse x-DFT|^2 into a double image per wave (exit intensity)
     ROW_ADJ_SEED = 6,     // adjoint seed: g = 2 w psi for L = sum w |psi|^2, stored as res F_x g
+    ROW_IFFT_WIDE = 1,    // inverse x-DFT, scaled, into a double2 image per wave (exit-wave readback)
     ROW_ADJ = 7,          // adjoint row half: g_t = conj(psi_s) u, then res F_x(conj(t) u)
 };
 
@@ -91,7 +92,7 @@ struct RowArgs {
     const float2* const* cfg_trans;  // per configuration: base of its slices
     const int* cfg_nslices;          // per configuration: its number of slices (t = 1 beyond)
     const int* wave_cfg;             // per wave: configuration
-    double* dout;                    // ROW_IFFT_INTENSITY: res*res doubles per wave
+    double* dout;                    // ROW_IFFT_INTENSITY: res*res doubles per wave (_WIDE: twice that)
     const double* weights;           // ROW_ADJ_SEED: dL/dI, res*res doubles per wave
     const int* wave_map;             // set -> wave index (NULL: identity); skips finished waves
     const float2* aux_in;            // ROW_ADJ: forward state S_s = F_x psi_s (wave_stride per wave)
@@ -257,7 +258,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
         band_store<PL, IO>(v, out + base, t, a.band_k);
         return;
     }
-    if constexpr (MODE == ROW_IFFT_T_FFT || MODE == ROW_IFFT || MODE == ROW_IFFT_INTENSITY) {
+    if constexpr (MODE == ROW_IFFT_T_FFT || MODE == ROW_IFFT || MODE == ROW_IFFT_INTENSITY || MODE == ROW_IFFT_WIDE) {
         fft_line<PL, true, band_reads(IO)>(v, ln, t, tws, sync);
         sync();
     }
@@ -267,6 +268,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
         for (int m = 0; m < E; ++m) {
             const double re = (double)v[m].x * a.scale, im = (double)v[m].y * a.scale;
             d[t + L * m] = re * re + im * im;
+        }
+        return;
+    }
+    if constexpr (MODE == ROW_IFFT_WIDE) {
+        double2* d = reinterpret_cast<double2*>(a.dout) + (size_t)wave * N * N + (size_t)row * N;
+#pragma unroll
+        for (int m = 0; m < E; ++m) {
+            const float2 f = cscale(v[m], a.scale);
+            d[t + L * m] = make_double2((double)f.x, (double)f.y);
         }
         return;
     }

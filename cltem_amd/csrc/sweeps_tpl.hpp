@@ -59,7 +59,7 @@ void row_pass_n(mse_engine* e, int mode, const float2* in, float2* out, int nlin
             MSE_ROW_CASE(ROW_IFFT_T_FFT, BAND_STEP)
             if constexpr (TR && std::is_same<SY, mse::WaveSync>::value && std::is_same<PL, P0>::value) {
                 MSE_ROW_CASE(ROW_FFT, BAND_FULL)
-                MSE_ROW_CASE(ROW_IFFT, BAND_FULL)
+                MSE_ROW_CASE(ROW_IFFT_WIDE, BAND_FULL)
                 MSE_ROW_CASE(ROW_COPY, BAND_FULL)
                 MSE_ROW_CASE(ROW_IFFT_INTENSITY, BAND_FULL)
                 MSE_ROW_CASE(ROW_ADJ_SEED, BAND_FULL)
