@@ -74,10 +74,8 @@ static __global__ __launch_bounds__(256) void k_bin_count(const double* __restri
                                                           unsigned* __restrict__ key, unsigned* __restrict__ rank,
                                                           int* __restrict__ bid_out, int* __restrict__ zid_out,
                                                           unsigned* __restrict__ hist) {
-    extern __shared__ unsigned count[];
-    __shared__ uint4 keys4[64];
-    unsigned* keys = reinterpret_cast<unsigned*>(keys4);
-    const int t = threadIdx.x, i = blockIdx.x * 256 + t;
+    extern __shared__ unsigned count[];  // per bin, one byte of atoms per wave of the block
+    const int t = threadIdx.x, i = blockIdx.x * 256 + t, wave = t >> 6;
     for (int k = t; k < nkeys; k += 256) count[k] = 0;
     unsigned mine = (unsigned)nkeys;
     if (i < n) {
@@ -87,22 +85,29 @@ static __global__ __launch_bounds__(256) void k_bin_count(const double* __restri
         bid_out[i] = bid;
         zid_out[i] = zid;
     }
-    keys[t] = mine;
     __syncthreads();
-    if (mine < (unsigned)nkeys) atomicAdd(&count[mine], 1u);
-    unsigned before = 0;
-    const int last = (t >> 6) * 16 + 16;  // this wave's own atoms at most
-#pragma unroll 4
-    for (int q = 0; q < last; ++q) {
-        const uint4 k = keys4[q];
-        const int j = 4 * q;
-        before += (k.x == mine && j < t) + (k.y == mine && j + 1 < t) + (k.z == mine && j + 2 < t) +
-                  (k.w == mine && j + 3 < t);
+    if (mine < (unsigned)nkeys) atomicAdd(&count[mine], 1u << (8 * wave));
+    // rank among the wave's earlier atoms: one round per bin that the wave holds
+    unsigned r = 0;
+    const unsigned long long below = (1ull << (t & 63)) - 1;
+    unsigned long long todo = __builtin_amdgcn_ballot_w64(mine < (unsigned)nkeys);
+    while (todo) {
+        const unsigned k = (unsigned)__builtin_amdgcn_readlane((int)mine, __builtin_ctzll(todo));
+        const unsigned long long same = __builtin_amdgcn_ballot_w64(mine == k);
+        if (mine == k) r = (unsigned)__popcll(same & below);
+        todo &= ~same;
     }
-    if (i < n) rank[i] = before;
     __syncthreads();
+    if (mine < (unsigned)nkeys) {
+        const unsigned c = count[mine];
+        for (int w = 0; w < wave; ++w) r += (c >> (8 * w)) & 255u;
+        rank[i] = r;
+    }
     unsigned* row = hist + (size_t)blockIdx.x * nkeys;
-    for (int k = t; k < nkeys; k += 256) row[k] = count[k];
+    for (int k = t; k < nkeys; k += 256) {
+        const unsigned c = count[k];
+        row[k] = (c & 255u) + ((c >> 8) & 255u) + ((c >> 16) & 255u) + (c >> 24);
+    }
 }
 
 // Each bin's column of hist (rows = atom blocks) to its exclusive prefix over the rows, and the

@@ -203,7 +203,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
     const int line = tid / L;
     const int t = tid % L;
     const int row = blockIdx.x * LINES + line;
-    const int wave = a.wave_map ? a.wave_map[blockIdx.y] : (int)blockIdx.y;
+    const int wave = a.wave_map ? cload(a.wave_map + blockIdx.y) : (int)blockIdx.y;
     float2* ln = lds[line];
 
     PlanTw<PL, TWREG> tws;
@@ -213,6 +213,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
     const size_t base = (size_t)wave * wave_stride + (size_t)row * N;
     float2 v[E];
     band_load<PL, IO>(v, in + base, t, a.band_k);
+    // the transmission row (and the forward state's row) with the wave's own: its address hangs on
+    // three lookups, and loads after the first transform would wait for all of them there (768^2,
+    // 32 waves: 66 -> 51 us a launch; the adjoint's row half of one wave at 256^2: 6.9 -> 5.7)
+    constexpr bool HAS_T = MODE == ROW_IFFT_T_FFT || MODE == ROW_ADJ;
+    float2 tr[HAS_T ? E : 1], ps[MODE == ROW_ADJ ? E : 1];
+    bool has_t = false;  // below a thinner specimen the slice is vacuum
+    if constexpr (MODE == ROW_ADJ) {
+        const float2* sp = a.aux_in + (size_t)wave * wave_stride + (size_t)row * N;
+#pragma unroll
+        for (int m = 0; m < E; ++m) ps[m] = sp[t + L * m];
+    }
+    if constexpr (HAS_T) {
+        const int cfg = row_config(a, wave);
+        has_t = a.slice < cload(a.cfg_nslices + cfg);
+        if (has_t) {
+            const float2* tp = cload(a.cfg_trans + cfg) + (size_t)a.slice * N * N + (size_t)row * N;
+#pragma unroll
+            for (int m = 0; m < E; ++m) tr[m] = gload(tp + t + L * m);
+        }
+    }
     if constexpr (MODE == ROW_COPY) {
 #pragma unroll
         for (int m = 0; m < E; ++m) out[base + t + L * m] = v[m];
@@ -231,22 +251,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
                 v[m] = make_float2(v[m].x * f, v[m].y * f);  // g = 2 w psi
             }
         } else {
-            float2 ps[E];
-            const float2* sp = a.aux_in + (size_t)wave * wave_stride + (size_t)row * N;
-#pragma unroll
-            for (int m = 0; m < E; ++m) ps[m] = sp[t + L * m];
             fft_line<PL, true>(ps, ln, t, tws, sync);
             sync();
             float2* gt = a.aux_out + (size_t)wave * wave_stride + (size_t)row * N;
-            const int cfg = row_config(a, wave);
-            const float2* tr = a.cfg_trans[cfg] + (size_t)a.slice * N * N + (size_t)row * N;
-            const bool has_t = a.slice < a.cfg_nslices[cfg];
 #pragma unroll
             for (int m = 0; m < E; ++m) {
                 const float2 u = make_float2(v[m].x * inv, v[m].y * inv);
                 const float2 psi = make_float2(ps[m].x * inv, ps[m].y * inv);
                 gt[t + L * m] = cmulc(u, psi);  // conj(psi) u
-                const float2 tv = has_t ? tr[t + L * m] : make_float2(1.f, 0.f);
+                const float2 tv = has_t ? tr[m] : make_float2(1.f, 0.f);
                 v[m] = cmulc(u, tv);  // conj(t) u
             }
         }
@@ -281,11 +294,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
         return;
     }
     if constexpr (MODE == ROW_IFFT_T_FFT) {
-        const int cfg = row_config(a, wave);
-        if (a.slice < a.cfg_nslices[cfg]) {  // below a thinner specimen the slice is vacuum
-            const float2* tr = a.cfg_trans[cfg] + (size_t)a.slice * N * N + (size_t)row * N;
+        if (has_t) {
 #pragma unroll
-            for (int m = 0; m < E; ++m) v[m] = cmul(v[m], tr[t + L * m]);
+            for (int m = 0; m < E; ++m) v[m] = cmul(v[m], tr[m]);
         }
     }
     if constexpr (MODE != ROW_IFFT) {

@@ -32,13 +32,16 @@ void row_pass_n(mse_engine* e, int mode, const float2* in, float2* out, int nlin
     if (step && variant < 0) {
         // Rule: while every line of the grid takes one row at most, the plain kernel (its waves go
         // straight to the loads); beyond, the persistent one, which keeps a transmission row in
-        // registers over the waves and prefetches.  Plain against persistent, us: 256^2 one wave
-        // 4.3 / 4.9, 32 waves 8.6 / 8.9; 512^2 one 4.7 / 5.3, 8 waves 9.6 / 10.0, 16 waves
-        // 15.4 / 14.1, 64 waves 48 / 35; 768^2 4 waves 11.9 / 12.4, 8 waves 21.5 / 18.9; 1024^2
-        // 2 waves 9.6 / 10.7, 8 waves 27.4 / 24.7.
+        // registers over the waves and prefetches.  With 12 elements per lane the plain kernel's
+        // fourth wave per SIMD outweighs both up to some 65,000 rows.  Plain against persistent,
+        // us: 256^2 one wave 4.2 / 4.8, 32 waves 8.4 / 9.0; 384^2 48 waves 22 / 24, 128 waves
+        // 50 / 53; 512^2 one 4.8 / 5.2, 8 waves 9.3 / 10.0, 16 waves 14.9 / 14.0, 64 waves
+        // 45 / 35; 768^2 8 waves 17.6 / 18.9, 64 waves 96 / 99, 128 waves 216 / 194; 1024^2 2
+        // waves 10.4 / 10.8, 8 waves 25.2 / 25.2, 64 waves 208 / 147.
         using K = std::integral_constant<int, mse::BAND_STEP>;
         const int per_cu = resident_per_cu<mse::k_row_step_pipe<P0, K::value, mse::WaveSync, true>>(256, 8);
-        variant = nlines_sets <= e->num_cus * per_cu * (256 / P0::L) / N ? 0 : 4;
+        const bool one_round = nlines_sets <= e->num_cus * per_cu * (256 / P0::L) / N;
+        variant = one_round || (P0::E == 12 && (long long)N * nlines_sets <= 65536) ? 0 : 4;
     }
     // one row per line of the grid, out of place or with the non-persistent variants
     auto go = [&](auto plan, auto sync, auto twreg) {
