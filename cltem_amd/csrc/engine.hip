@@ -1435,9 +1435,8 @@ void potential_planes(mse_engine* e, const ConfigData& c, const mse_geometry& g,
 // with the band's per-row limits as the mask: cmul(v, cmul((s, 0), (1, 0))) = cmul(v, (s, 0))
 // bit for bit, on the persistent column kernels.  Their variant goes by the rule on the grid size
 // and the number of planes, so that transmission functions do not depend on the tuning state: the
-// kernels the rule takes round alike, whatever the number of planes.  (At 768^2 the lean kernel,
-// which has always limited that size's functions: its twiddle products round otherwise, 118
-// against 103 us for 64 planes.)
+// kernels the rule takes round alike, whatever the number of planes.  (At 768^2 the lean kernel
+// with the twiddle rounding that size's functions have always had.)
 void band_limit_planes(mse_engine* e, float2* p, int planes) {
     const bool band = e->band_k >= 0;
     mse::RowArgs ra = base_row_args(e);
@@ -1453,7 +1452,7 @@ void band_limit_planes(mse_engine* e, float2* p, int planes) {
     ca.px = e->band_xy.p;
     ca.py = e->band_xy.p + e->res;
     ca.lim = e->band_lim.p;
-    col_pass(e, mse::COL_PROP, p, p, planes, e->N, ca, PK_COL, e->res == 768 ? 11 : kRule);
+    col_pass(e, mse::COL_PROP, p, p, planes, e->N, ca, PK_COL, e->res == 768 ? kLeanAlt : kRule);
     row_pass(e, mse::ROW_IFFT, p, p, planes, e->N, ra);
 }
 

@@ -251,6 +251,8 @@ inline void launch(mse_engine* e, int kind, F&& f) {
 // variant arguments of row_pass / col_pass: the engine's choice (tuned, else set, else by rule), or
 // the sweeps' rule whatever was tuned or set
 constexpr int kEngineChoice = -1, kRule = -2;
+// column variant 11 with the twiddle rounding of the 768^2 band limit (band_limit_planes)
+constexpr int kLeanAlt = 14;
 
 // ---- host copies -----------------------------------------------------------------------------
 // Copies between a caller's pageable memory and the device, through pinned staging memory.  The
@@ -311,6 +313,7 @@ void sync_wave_prop(mse_engine* e);
 //          9: as 7 with twiddles read at use
 //         10: as 7 with 8-column tiles (512 threads: no register spills at 1024 points)
 constexpr int kRowVariants = 7;
+//         11: lean: one tile per block without prefetch, several blocks per CU, XCD-aware order
 //         12: as 10 (8-column tiles) with XCD-aware item order, up to four blocks per CU
 //         13: as 7 (16-column tiles) with XCD-aware item order
 constexpr int kColVariants = 14;

@@ -340,8 +340,9 @@ struct NoPassTw {
     __device__ __forceinline__ void load(const float2* __restrict__, int) {}
 };
 
-template <class PL, bool IN_REGS = true>
+template <class PL, bool IN_REGS = true, bool ALT = false>
 struct PlanTw {
+    static constexpr bool alt = ALT;  // see cmul_tw
     using T1 = typename std::conditional<IN_REGS, PassTw<PL::N, PL::L, PL::R1, PL::R0>,
                                          PassTwMem<PL::N, PL::L, PL::R1, PL::R0>>::type;
     using T2 = typename std::conditional<IN_REGS, PassTw<PL::N, PL::L, PL::R2, PL::R0 * PL::R1>,
@@ -407,9 +408,20 @@ __device__ __forceinline__ void stockham_first_banded(float2 (&v)[N / L], float2
     }
 }
 
+// The twiddle products with the rounded product of each part written out (as in rot), so that
+// transforms round alike wherever their twiddles come from.  ALT: the other choice in the forward
+// imaginary part, the rounding that the 768^2 band limit of transmission functions has.
+template <bool ALT>
+__device__ __forceinline__ float2 cmul_tw(float2 a, float2 w) {
+    return make_float2(fmaf(a.x, w.x, -(a.y * w.y)), ALT ? fmaf(a.y, w.x, a.x * w.y) : fmaf(a.x, w.y, a.y * w.x));
+}
+__device__ __forceinline__ float2 cmulc_tw(float2 a, float2 w) {
+    return make_float2(fmaf(a.x, w.x, a.y * w.y), fmaf(a.y, w.x, -(a.x * w.y)));
+}
+
 // One Stockham pass.  v holds the line in register layout; line is this line's LDS.
 // P_ = product of radices already done (p); LAST = this pass ends the transform.
-template <int N, int L, int R, int P_, bool INV, bool LAST, class TW, bool PAD2 = false>
+template <int N, int L, int R, int P_, bool INV, bool LAST, bool ALT, class TW, bool PAD2 = false>
 __device__ __forceinline__ void stockham_pass(float2 (&v)[N / L], float2* line, int t,
                                               const TW* tw) {
     constexpr int E = N / L;
@@ -425,7 +437,7 @@ __device__ __forceinline__ void stockham_pass(float2 (&v)[N / L], float2* line, 
 #pragma unroll
             for (int r = 1; r < R; ++r) {
                 const float2 w = tw->get(b, r, k);
-                a[r] = INV ? cmulc(a[r], w) : cmul(a[r], w);
+                a[r] = INV ? cmulc_tw(a[r], w) : cmul_tw<ALT>(a[r], w);
             }
         }
         Dft<R, INV>::run(a);
@@ -461,22 +473,22 @@ __device__ __forceinline__ void fft_line(float2 (&v)[PL::E], float2* line, int t
     if constexpr (BANDED)
         stockham_first_banded<N, L, PL::R0, INV>(v, line, t);
     else
-        stockham_pass<N, L, PL::R0, 1, INV, false, NoTw>(v, line, t, nullptr);
+        stockham_pass<N, L, PL::R0, 1, INV, false, false, NoTw>(v, line, t, nullptr);
     sync();
     line_gather<N, L>(v, line, t);
     sync();
-    stockham_pass<N, L, PL::R1, PL::R0, INV, false, typename TWS::T1, true>(v, line, t, &tw.p1);
+    stockham_pass<N, L, PL::R1, PL::R0, INV, false, TWS::alt, typename TWS::T1, true>(v, line, t, &tw.p1);
     sync();
     line_gather<N, L, true>(v, line, t);
     sync();
     if constexpr (PL::R3 == 1) {
-        stockham_pass<N, L, PL::R2, PL::R0 * PL::R1, INV, true>(v, line, t, &tw.p2);
+        stockham_pass<N, L, PL::R2, PL::R0 * PL::R1, INV, true, TWS::alt>(v, line, t, &tw.p2);
     } else {
-        stockham_pass<N, L, PL::R2, PL::R0 * PL::R1, INV, false, typename TWS::T2>(v, line, t, &tw.p2);
+        stockham_pass<N, L, PL::R2, PL::R0 * PL::R1, INV, false, TWS::alt, typename TWS::T2>(v, line, t, &tw.p2);
         sync();
         line_gather<N, L>(v, line, t);
         sync();
-        stockham_pass<N, L, PL::R3, PL::R0 * PL::R1 * PL::R2, INV, true>(v, line, t, &tw.p3);
+        stockham_pass<N, L, PL::R3, PL::R0 * PL::R1 * PL::R2, INV, true, TWS::alt>(v, line, t, &tw.p3);
     }
 }
 

@@ -415,6 +415,12 @@ __device__ __forceinline__ double wave_sum(double v) {
 // doubles as its FFT exchange buffer.  BAND: the propagation's mask cuts the ky outside the
 // band (a.band_k set), whose outputs are not formed and not transformed back.
 // --------------------------------------------------------------------------------------
+// v px py, the product of the propagator's factors first, as one propagation multiplies (which
+// product of each part is rounded is written out, as in rot: all kernels propagate alike)
+__device__ __forceinline__ float2 prop_mul(float2 v, float2 px, float2 py) {
+    const float2 f = make_float2(fmaf(px.x, py.x, -(px.y * py.y)), fmaf(px.y, py.x, px.x * py.y));
+    return make_float2(fmaf(v.x, f.x, -(v.y * f.y)), fmaf(v.x, f.y, v.y * f.x));
+}
 // first column of tile j of a launch
 template <int TC>
 __device__ __forceinline__ int tile_column(const ColArgs& a, int j) {
@@ -708,7 +714,7 @@ __global__ __launch_bounds__(TC * PL::L) __attribute__((amdgpu_waves_per_eu(WPE)
                 pyy = pyv[m];
             else
                 pyy = per_wave ? gload(pyt + y) : spy[y];
-            const float2 f = cmul(v[m], cmul(pxv, pyy));
+            const float2 f = prop_mul(v[m], pxv, pyy);
             v[m] = ys <= lim ? f : make_float2(0.f, 0.f);
         }
         sync();
@@ -731,10 +737,10 @@ __global__ __launch_bounds__(TC * PL::L) __attribute__((amdgpu_waves_per_eu(WPE)
 }
 
 // --------------------------------------------------------------------------------------
-// Column slice step, one 16-column tile per block with no prefetch, sized for two blocks
-// per CU (at most 64 VGPRs): twiddles and y factors are read from per-block copies in LDS,
-// so that the second block's loads and stores overlap the first one's transforms.  Same
-// arithmetic as k_col<..., COL_PROP>.  Grid (column tiles, nsets).
+// Column slice step, one tile per block with no prefetch, sized for several blocks per CU:
+// twiddles and y factors are read from per-block copies in LDS, so that the other blocks' loads
+// and stores overlap this one's transforms.  Same arithmetic as k_col_prop_pipe.  Grid: tiles x
+// sets in one dimension, rounded up to a multiple of 8; XCD-aware order as there.
 // --------------------------------------------------------------------------------------
 // Twiddle table entries a plan's passes read: pass with radix R after p points reads
 // r k N / (p R) for r < R, k < p.
@@ -751,23 +757,28 @@ constexpr int plan_twiddles() {
     return most + 1;
 }
 
-template <class PL, int TC, bool BAND>
+template <class PL, int TC, bool BAND, bool ALT>
 __device__ __forceinline__ void col_prop_lean(float2* __restrict__ data, size_t wave_stride,
-                                              const float2* __restrict__ tw, const ColArgs& a) {
+                                              const float2* __restrict__ tw, const ColArgs& a, int nsets) {
     constexpr int N = PL::N, L = PL::L, E = PL::E;
     constexpr int NT = TC * L;
     constexpr int CS = LdsLine<N>::col_stride;
     constexpr int NQ = (TC * N / 2) / NT;
-    static_assert(L == 64 && (TC * N / 2) % NT == 0, "one column per wave");
-    constexpr int NTW = plan_twiddles<PL>();
+    static_assert((TC * N / 2) % NT == 0, "tile must split evenly over the block");
+    const int item = (int)((blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8);
+    if (item >= a.n_tiles * nsets) return;
+    // copies of the tables where they leave a CU two blocks; at 1024 points they would not
+    constexpr bool TABLES = N < 1024;
+    constexpr int NTW = TABLES ? plan_twiddles<PL>() : 1;
     __shared__ float2 tile[TC * CS];
     __shared__ float2 stw[NTW];
-    __shared__ float2 spy[N];
+    __shared__ float2 spy[TABLES ? N : 1];
     const int tid = threadIdx.x;
     const int c = tid / L;
     const int t = tid % L;
-    const int wv = a.wave_map ? cload(a.wave_map + blockIdx.y) : (int)blockIdx.y;
-    const int x0 = tile_column<TC>(a, blockIdx.x);
+    const int set = item / a.n_tiles;
+    const int wv = a.wave_map ? cload(a.wave_map + set) : set;
+    const int x0 = tile_column<TC>(a, item % a.n_tiles);
     const int x = x0 + c;
     const float4* in4 = reinterpret_cast<const float4*>(data + (size_t)wv * wave_stride + x0);
     float4 q[NQ];
@@ -783,13 +794,16 @@ __device__ __forceinline__ void col_prop_lean(float2* __restrict__ data, size_t 
         pxt = cload(a.wave_prop + 2 * wv);
         pyt = cload(a.wave_prop + 2 * wv + 1);
     }
-    for (int i = tid; i < N; i += NT) {
-        if (i < NTW) stw[i] = tw[i];
-        spy[i] = pyt[i];
+    if constexpr (TABLES) {
+        for (int i = tid; i < N; i += NT) {
+            if (i < NTW) stw[i] = tw[i];
+            spy[i] = pyt[i];
+        }
     }
     const int xs = (x < N / 2) ? x : N - x;
-    const float2 pxv = cload(pxt + __builtin_amdgcn_readfirstlane(x));
-    const int lim = cload(a.lim + __builtin_amdgcn_readfirstlane(xs));  // the mask is symmetric in kx and ky
+    // the column's factor and mask (symmetric in kx and ky): scalar loads where a wave is one column
+    const float2 pxv = L == 64 ? cload(pxt + __builtin_amdgcn_readfirstlane(x)) : gload(pxt + x);
+    const int lim = L == 64 ? cload(a.lim + __builtin_amdgcn_readfirstlane(xs)) : gload(a.lim + xs);
 #pragma unroll
     for (int k = 0; k < NQ; ++k) {
         const int idx = tid + k * NT;
@@ -798,8 +812,8 @@ __device__ __forceinline__ void col_prop_lean(float2* __restrict__ data, size_t 
         tile[(cc + 1) * CS + lpad(r)] = make_float2(q[k].z, q[k].w);
     }
     __syncthreads();
-    PlanTw<PL, false> tws;
-    tws.load(stw, t);
+    PlanTw<PL, false, ALT> tws;
+    tws.load(TABLES ? stw : tw, t);
     const WaveSync sync{};
     float2* ln = tile + c * CS;
     float2 v[E];
@@ -811,7 +825,7 @@ __device__ __forceinline__ void col_prop_lean(float2* __restrict__ data, size_t 
         if (BAND && band_class<N, L>(m) == BAND_OUT) continue;
         const int y = t + L * m;
         const int ys = (y < N / 2) ? y : N - y;
-        const float2 f = cmul(v[m], cmul(pxv, spy[y]));
+        const float2 f = prop_mul(v[m], pxv, TABLES ? spy[y] : gload(pyt + y));
         v[m] = ys <= lim ? f : make_float2(0.f, 0.f);
     }
     sync();
@@ -830,17 +844,15 @@ __device__ __forceinline__ void col_prop_lean(float2* __restrict__ data, size_t 
     }
 }
 
-// 16-column tiles (512 points): 64 VGPRs, two 1024-thread blocks per CU
-template <class PL, bool BAND>
-__global__ __launch_bounds__(16 * PL::L) __attribute__((amdgpu_waves_per_eu(8), amdgpu_num_vgpr(64))) void k_col_prop_lean(
-    float2* __restrict__ data, size_t wave_stride, const float2* __restrict__ tw, ColArgs a) {
-    col_prop_lean<PL, 16, BAND>(data, wave_stride, tw, a);
+// waves per SIMD the lean kernel is held to: 8 (64 VGPRs) with 8 elements per lane, 4 beyond
+template <class PL>
+constexpr int lean_waves() {
+    return PL::E <= 8 ? 8 : 4;
 }
-// 8-column tiles (four-pass plans, 12 elements per lane): two 512-thread blocks per CU
-template <class PL, bool BAND>
-__global__ __launch_bounds__(8 * PL::L) __attribute__((amdgpu_waves_per_eu(4))) void k_col_prop_lean8(
-    float2* __restrict__ data, size_t wave_stride, const float2* __restrict__ tw, ColArgs a) {
-    col_prop_lean<PL, 8, BAND>(data, wave_stride, tw, a);
+template <class PL, int TC, bool BAND, bool ALT = false>
+__global__ __launch_bounds__(TC * PL::L) __attribute__((amdgpu_waves_per_eu(lean_waves<PL>()))) void k_col_prop_lean(
+    float2* __restrict__ data, size_t wave_stride, const float2* __restrict__ tw, ColArgs a, int nsets) {
+    col_prop_lean<PL, TC, BAND, ALT>(data, wave_stride, tw, a, nsets);
 }
 
 // --------------------------------------------------------------------------------------

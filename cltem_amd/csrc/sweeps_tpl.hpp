@@ -150,18 +150,29 @@ int col_pass_n(mse_engine* e, int mode, const float2* in, float2* out, int nsets
     if (mode == mse::COL_PROP && in == out && variant < 0) {
         // Rule: the narrowest tiles while they leave CUs idle, wider ones as the launch grows (a
         // narrow tile is a shorter chain of loads, transforms and stores, a wide one moves whole
-        // 128-byte lines and shares a line's transfer with no other block).  us per launch on the
-        // band, 4 / 8 / 16 columns (the first two in XCD-aware order): 256^2 one wave
-        // 4.5 / 5.0 / 5.6, 16 waves 6.1 / 6.4 / 6.5, 64 waves 15.7 / 15.2 / 12.3; 512^2 one
-        // 5.7 / 6.4 / 9.8, 8 waves 9.2 / 10.3 / 11.5, 16 waves 17.8 / 17.0 / 16.9, 128 waves
-        // - / 69.8 / 62.8; 768^2 one 8.2 / 10.5 / 26.7, 4 waves 12.3 / 12.2 / 30.5; 1024^2 2 waves
-        // 12.6 / 12.8 / 37.6, 4 waves 22.4 / 20.8 / 41.9, 64 waves 187 / 177 / 407 (16 columns of
-        // the 12- and 16-element plans spill or leave a CU one block of half its waves).
+        // 128-byte lines and shares a line's transfer with no other block); with 12 elements per
+        // lane the lean kernel, whose four waves per SIMD need no prefetch registers (the
+        // persistent one has two).  us per launch on the band, persistent with 4 / 8 / 16 columns
+        // (the first two in XCD-aware order) / lean:
+        //   256^2 one wave 4.5 / 5.0 / 5.6 / 6.1, 16 waves 6.1 / 6.4 / 6.5 / 7.0, 64 15.4 / 15.5 / 12.3 / 13.0
+        //   384^2 one 6.5 / 7.2 / 9.1 / 8.3, 8 waves 8.4 / 8.1 / 9.9 / 9.2, 32 17.6 / 17.3 / 17.4 / 15.8
+        //   512^2 one 5.8 / 6.4 / 9.8 / 8.7, 8 waves 9.2 / 10.3 / 11.5 / 10.7, 64 49 / 38.8 / 38.9 / 44
+        //   768^2 one 8.4 / 10.5 / 27 / 9.0, 4 waves 12.3 / 12.2 / 30 / 11.2, 64 108 / 103 / 235 / 97, 128 255 / 252 / - / 198
+        //   1024^2 one 10.3 / 12.1 / 33 / 11.3, 4 waves 22.4 / 20.8 / 42 / 17.9, 16 48 / 48 / 108 / 52, 64 188 / 176 / 407 / 228
+        // (16 columns of the 12- and 16-element plans spill.)
         const int k = band ? args.band_k : N / 2;
-        const long long items4 = (2 * (k / 4) + 2) * (long long)nsets;
-        variant = items4 <= e->num_cus * (P0::E <= 8 ? 3 : 2)                     ? 5
-                  : N > 512 || (2 * (k / 16) + 2) * (long long)nsets < 3 * e->num_cus ? 12
-                                                                                  : 7;
+        const auto items = [&](int tc) { return (2 * (k / tc) + 2) * (long long)nsets; };
+        const int cus = e->num_cus;
+        if (items(4) <= (P0::E <= 8 ? 3 : N == 384 ? 2 : 1) * cus)
+            variant = 5;
+        else if (N == 384)
+            variant = items(16) <= cus ? 12 : 11;
+        else if (N == 768)
+            variant = 11;
+        else if (N == 1024)
+            variant = items(8) <= 2 * cus ? 11 : 12;
+        else
+            variant = items(16) < 3 * cus ? 12 : 7;
     }
     // the tiles of TC columns to visit: with a band, those that hold columns 0..K or N-K..N-1
     auto set_tiles = [&](int TC) {
@@ -235,25 +246,29 @@ int col_pass_n(mse_engine* e, int mode, const float2* in, float2* out, int nsets
                 return args.n_tiles;
             }
         }
-        if (variant == 11) {  // lean: two blocks per CU
-            auto lean = [&](auto bnd) {
-                constexpr bool BAND = decltype(bnd)::value;
-                if constexpr (P0::L == 64 && N <= 512) {  // 16-column tiles, 64 VGPRs
-                    dim3 grid(set_tiles(16), nsets);
-                    launch(e, kind, [&]() {
-                        mse::k_col_prop_lean<P0, BAND><<<grid, 16 * P0::L, 0, e->stream>>>(out, wave_stride, e->tw.p, args);
-                    });
-                    return true;
-                } else if constexpr (P0::L == 64 && P0::R3 > 1) {  // four-pass plans: 8-column tiles, 128 VGPRs
-                    dim3 grid(set_tiles(8), nsets);
-                    launch(e, kind, [&]() {
-                        mse::k_col_prop_lean8<P0, BAND><<<grid, 8 * P0::L, 0, e->stream>>>(out, wave_stride, e->tw.p, args);
-                    });
-                    return true;
-                }
-                return false;
+        if (variant == 11 || variant == kLeanAlt) {  // lean: one tile per block, several blocks per CU
+            constexpr int TC = N <= 512 ? 16 : 8;
+            const int blocks = (set_tiles(TC) * nsets + 7) / 8 * 8;
+            auto lean = [&](auto bnd, auto alt) {
+                launch(e, kind, [&]() {
+                    mse::k_col_prop_lean<P0, TC, decltype(bnd)::value, decltype(alt)::value>
+                        <<<blocks, TC * P0::L, 0, e->stream>>>(out, wave_stride, e->tw.p, args, nsets);
+                });
             };
-            if (band ? lean(std::true_type{}) : lean(std::false_type{})) return args.n_tiles;
+            if constexpr (N == 768) {
+                if (variant == kLeanAlt) {
+                    if (band)
+                        lean(std::true_type{}, std::true_type{});
+                    else
+                        lean(std::false_type{}, std::true_type{});
+                    return args.n_tiles;
+                }
+            }
+            if (band)
+                lean(std::true_type{}, std::false_type{});
+            else
+                lean(std::false_type{}, std::false_type{});
+            return args.n_tiles;
         }
         switch (variant) {
             case 5: pipe(P0{}, C4{}, REG{}, std::true_type{}, 2048); break;
