@@ -631,6 +631,7 @@ int mse_set_geometry(mse_engine* e, const mse_geometry* g) {
             e->det_key.clear();
         }
         e->adj_ready = false;  // checkpoints belong to the previous geometry
+        ++e->geom_version;
         for (auto& c : e->configs) {  // bins and transmission functions depend on the geometry
             c.sorted = false;
             c.built = false;
@@ -1503,7 +1504,7 @@ void reduce_detectors(mse_engine* e, int nw, int n_det, int sqrt2, double* dev_o
 // memory and are updated (outside the graph) before each replay.
 struct StemGraphKey {
     int res, cfg, nb, n_det, sqrt2, row_var, col_var, n_slices, mix_first, mix_sets;
-    unsigned tune_version;
+    unsigned tune_version, geom_version;
     unsigned long long mix_seed;
     const void *waves, *partials, *det_out, *det_bits, *trans, *probe_pos, *probe_df, *mix_key;
     const void *cfg_ptrs, *cfg_nslices, *wave_cfg, *wave_map, *tw, *px, *py, *wave_prop, *lim, *kx, *ky;
@@ -1549,7 +1550,7 @@ int mse_multislice(mse_engine* e, int first, int count) {
 // device pointer baked into its kernel arguments.
 struct LoopGraphKey {
     int res, nw, first, count, row_var, col_var, num_cus, mix_first, mix_sets;
-    unsigned tune_version;
+    unsigned tune_version, geom_version;
     unsigned long long mix_seed;
     const void *waves, *cfg_ptrs, *cfg_nslices, *wave_cfg, *tw, *px, *py, *wave_prop, *lim, *mix_key;
 };
@@ -1569,6 +1570,7 @@ std::vector<unsigned char> loop_graph_key(mse_engine* e, int first, int count) {
     k.row_var = e->row_var;
     k.col_var = e->col_var;
     k.tune_version = e->tune_version;
+    k.geom_version = e->geom_version;
     k.num_cus = e->num_cus;
     k.waves = e->waves.p;
     k.cfg_ptrs = e->cfg_ptrs.p;
@@ -1914,6 +1916,7 @@ int mse_stem_batch(mse_engine* e, int cfg, const double* pos_xy, int n_probes, i
             k.row_var = e->row_var;
             k.col_var = e->col_var;
             k.tune_version = e->tune_version;
+            k.geom_version = e->geom_version;
             k.n_slices = ns;
             k.waves = e->waves.p;
             k.partials = e->partials.p;

@@ -184,6 +184,8 @@ struct mse_engine {
     // sweeps over a tuned wave count use them, any other count the ones above
     std::vector<std::pair<int, std::pair<int, int>>> tuned;
     unsigned tune_version = 0;     // bumped by every change of variants (captured graphs depend on them)
+    unsigned geom_version = 0;     // bumped by every mse_set_geometry (the band and the probes' optics are
+                                   // baked into captured kernels' arguments)
     hipGraphExec_t stem_exec = nullptr;
     std::vector<unsigned char> stem_key;
     hipGraphExec_t loop_exec = nullptr;   // captured slice loop of mse_multislice_graph
