@@ -54,7 +54,7 @@ enum ColMode : int {
 // Columns a row pass reads and writes (the last four only for limits that band_class covers).
 enum BandIo : int {
     BAND_FULL = 0,    // reads and writes every column
-    BAND_FIRST = 1,   // reads every column, writes the band and zeros outside it
+    BAND_FIRST = 1,   // reads every column up to read_k, writes the band and zeros outside it
     BAND_STEP = 2,    // reads and writes the band (outside it: zero in memory, not touched)
     BAND_WRITE = 3,   // reads every column, writes the band (the rest is left as it was)
     BAND_READ = 4,    // reads the band (the rest is taken as zero), writes every column
@@ -101,6 +101,7 @@ struct RowArgs {
     float scale;                     // ROW_FFT / ROW_IFFT output scale
     int io;                          // BandIo
     int band_k;                      // largest |kx index| of the band (io other than BAND_FULL)
+    int read_k;                      // BAND_FIRST: largest |kx index| that may hold anything but zero
     // mixed static potentials: with mix_sets >= 2 a wave reads configuration mix_first + a
     // set drawn per (mix_key[wave], slice) instead of its own (row_config)
     const unsigned* mix_key;
@@ -140,14 +141,15 @@ struct ColArgs {
     const double* kx;        // k-grid (COL_PROBE)
     const double* ky;
     // COL_PROP*: largest |kx index| that lim keeps, for the sweeps on the band alone (the row
-    // pass before must have left the columns outside it at zero); -1: every column
+    // pass before must have left the columns outside it at zero); COL_PROBE: largest |kx index| of
+    // the columns to write (the rest is left as it was); -1: every column
     int band_k;
     // column tiles of a launch (set by the launcher): tile j < n_tiles starts at column
     // TC j below tile_lo, TC (j + tile_skip) from there
     int n_tiles, tile_lo, tile_skip;
     float scale;             // COL_FFT_*: multiply after the forward DFT
     double det_scale;        // intensity factor applied to |V|^2 in detector sums
-    const unsigned* det_bits;  // ndet bitmasks over the fft-shifted image, res*res bits each
+    const unsigned* det_bits;  // ndet bitmasks over the fft-shifted image, res*res bits each, column-major
     int ndet;
     double* partials;        // [wave][det][tile] partial sums
     double* diff;            // COL_FFT_DIFF: res*res doubles per wave, fft-shifted
@@ -157,12 +159,15 @@ struct ColArgs {
 
 // One line's elements from and to memory (register layout), as IO says.
 template <class PL, int IO>
-__device__ __forceinline__ void band_load(float2 (&v)[PL::E], const float2* src, int t, int k) {
+__device__ __forceinline__ void band_load(float2 (&v)[PL::E], const float2* src, int t, const RowArgs& a) {
     constexpr int N = PL::N, L = PL::L;
+    const int k = IO == BAND_FIRST ? a.read_k : a.band_k;
 #pragma unroll
     for (int m = 0; m < PL::E; ++m) {
         const int x = t + L * m;
-        if (!band_reads(IO) || band_class<N, L>(m) == BAND_IN)
+        if (IO == BAND_FIRST)
+            v[m] = in_band(x, N, k) ? src[x] : make_float2(0.f, 0.f);
+        else if (!band_reads(IO) || band_class<N, L>(m) == BAND_IN)
             v[m] = src[x];
         else if (band_class<N, L>(m) == BAND_EDGE)
             v[m] = in_band(x, N, k) ? src[x] : make_float2(0.f, 0.f);
@@ -212,7 +217,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
 
     const size_t base = (size_t)wave * wave_stride + (size_t)row * N;
     float2 v[E];
-    band_load<PL, IO>(v, in + base, t, a.band_k);
+    band_load<PL, IO>(v, in + base, t, a);
     // the transmission row (and the forward state's row) with the wave's own: its address hangs on
     // three lookups, and loads after the first transform would wait for all of them there (768^2,
     // 32 waves: 66 -> 51 us a launch; the adjoint's row half of one wave at 256^2: 6.9 -> 5.7)
@@ -446,6 +451,15 @@ __global__ __launch_bounds__(TC * PL::L) __attribute__((amdgpu_waves_per_eu(WPE)
     float2* ln = tile + c * CS;
     const size_t wbase = (size_t)wave * wave_stride;
 
+    if constexpr (MODE == COL_PROBE) {
+        // columns outside the aperture are zero: |k| >= |kx| in every rounding step
+        if (fmin(fabs(a.kx[x0]), fabs(a.kx[x0 + TC - 1])) >= a.probe.cond_ap2 + a.probe.smooth_r) {
+            float4* out4 = reinterpret_cast<float4*>(out + wbase + x0);
+            for (int idx = tid; idx < TC * N / 2; idx += NT)
+                out4[((size_t)(idx / (TC / 2)) * N) / 2 + idx % (TC / 2)] = make_float4(0.f, 0.f, 0.f, 0.f);
+            return;
+        }
+    }
     PlanTw<PL, TWREG> tws;
     tws.load(tw, t);
     const SYNC sync{};
@@ -521,14 +535,14 @@ __global__ __launch_bounds__(TC * PL::L) __attribute__((amdgpu_waves_per_eu(WPE)
         const int nw = NT / 64;
         const int wid = tid / 64, lane = tid % 64;
         for (int d = 0; d < a.ndet; ++d) {
-            const unsigned* bits = a.det_bits + (size_t)d * ((size_t)N * N / 32);
+            // the column's own N bits: a wave reads one or two words of them per element
+            const unsigned* bits = a.det_bits + ((size_t)d * N + xs) * (N / 32);
             double acc = 0.0;
 #pragma unroll
             for (int m = 0; m < E; ++m) {
                 if (BAND && band_class<N, L>(m) == BAND_OUT) continue;  // nothing there
                 const int ys = (t + L * m + N / 2) % N;
-                const size_t bit = (size_t)ys * N + xs;
-                if ((bits[bit >> 5] >> (bit & 31)) & 1u) {
+                if ((bits[ys >> 5] >> (ys & 31)) & 1u) {
                     const float i2 = v[m].x * v[m].x + v[m].y * v[m].y;
                     acc += (double)i2;
                 }
@@ -895,7 +909,7 @@ __global__ __launch_bounds__(256) void k_row_step_pipe(float2* __restrict__ data
     float2 qv[E], tr[STEP ? E : 1];
     const float2* cur = nullptr;  // the transmission row in tr
     bool vacuum = false;          // below a thinner specimen: t = 1, nothing to multiply
-    band_load<PL, IO>(qv, row_of(set), t, a.band_k);
+    band_load<PL, IO>(qv, row_of(set), t, a);
     for (; set < nsets; set += groups) {
         if constexpr (STEP) {
             const int cfg = row_config(a, a.wave_map ? cload(a.wave_map + set) : set);
@@ -910,7 +924,7 @@ __global__ __launch_bounds__(256) void k_row_step_pipe(float2* __restrict__ data
         float2 v[E];
 #pragma unroll
         for (int m = 0; m < E; ++m) v[m] = qv[m];
-        if (set + groups < nsets) band_load<PL, IO>(qv, row_of(set + groups), t, a.band_k);
+        if (set + groups < nsets) band_load<PL, IO>(qv, row_of(set + groups), t, a);
         if constexpr (STEP) {
             fft_line<PL, true, band_reads(IO)>(v, ln, t, tws, sync);
             sync();

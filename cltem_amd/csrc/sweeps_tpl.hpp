@@ -178,7 +178,7 @@ int col_pass_n(mse_engine* e, int mode, const float2* in, float2* out, int nsets
     auto set_tiles = [&](int TC) {
         args.tile_lo = N / TC;
         args.tile_skip = 0;
-        if (band) {
+        if (band || (mode == mse::COL_PROBE && args.band_k >= 0)) {
             const int hi = (N - args.band_k) / TC;
             args.tile_lo = args.band_k / TC + 1;
             args.tile_skip = std::max(0, hi - args.tile_lo);
@@ -280,7 +280,11 @@ int col_pass_n(mse_engine* e, int mode, const float2* in, float2* out, int nsets
         }
         return args.n_tiles;
     }
-    if (variant >= 7) variant = 0;
+    // Rule: 8-column tiles where 16-column ones would leave CUs without a block (one wave at 512^2:
+    // detectors 14.4 -> 7.0 us) and for the plans whose 1024-thread blocks spill.  Detector
+    // partials are per tile: FP64 sums in another grouping.
+    if (variant >= 7 || variant == 5 || variant < 0) variant = 0;
+    const bool few = (N / 16) * nsets < e->num_cus, spills = P0::L == 64 && P0::E > 8;
     if (variant == 1)
         go(P1{}, C16{}, mse::WaveSync{}, REG{});
     else if (variant == 2)
@@ -294,7 +298,7 @@ int col_pass_n(mse_engine* e, int mode, const float2* in, float2* out, int nsets
             go(P1{}, C32{}, mse::WaveSync{}, REG{});
         else
             go(P0{}, C16{}, mse::WaveSync{}, REG{});
-    } else if (!hot && P0::L == 64 && P0::E > 8)  // 16-column tiles of 1024 threads spill here
+    } else if (variant == 0 && mode != mse::COL_COPY && mode != mse::COL_PROP && (few || spills))
         go(P0{}, C8{}, mse::WaveSync{}, REG{});
     else
         go(P0{}, C16{}, mse::WaveSync{}, REG{});
