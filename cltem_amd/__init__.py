@@ -374,7 +374,7 @@ class Engine:
     # -- tuning -------------------------------------------------------------------------
     def set_potential_tables(self, enable: bool = True, lds: bool = True):
         """Tabulated potentials (default) or the formulas evaluated directly, from the next build;
-        lds=False keeps the full-3D kernels' table reads in global memory (same values)."""
+        lds=False keeps the builders' table reads in global memory (same values)."""
         _check(self.lib.mse_set_potential_tables(self.h, (1 if lds else 2) if enable else 0))
 
     def set_kernel_variant(self, kernel: int, variant: int):

@@ -126,6 +126,7 @@ int mse_adjoint_positions(mse_engine* e, const double* dl_di, double* grad_xyz) 
         // the phases from the same (tabulated or direct) potentials as the forward build
         pa.vtab = potential_tables(e, c, g);
         const bool tab = pa.vtab != nullptr;
+        const size_t lds = g.full3d ? 0 : projected_lds_tables(e, c, pa);
         // as mse_build_transmission: full 3D 32 slices per launch, projected up to 256
         const int chunk = g.full3d ? 32 : 256;
         for (int s0 = 0; s0 < n; s0 += chunk) {
@@ -145,13 +146,16 @@ int mse_adjoint_positions(mse_engine* e, const double* dl_di, double* grad_xyz) 
                         tab ? mse::k_phase_full3d<2, true><<<grid, 256, 0, e->stream>>>(o, c.x.p, c.y.p, c.z.p, c.Z.p, c.block_start.p, e->params3d.p, pa, s0)
                             : mse::k_phase_full3d<2><<<grid, 256, 0, e->stream>>>(o, c.x.p, c.y.p, c.z.p, c.Z.p, c.block_start.p, e->params3d.p, pa, s0);
                 } else if (e->form == 0)
-                    tab ? mse::k_phase_projected<0, true><<<grid, 256, 0, e->stream>>>(o, c.x.p, c.y.p, c.Z.p, c.block_start.p, e->params_proj.p, pa, s0)
+                    lds ? mse::k_phase_projected<0, true, true><<<grid, 256, lds, e->stream>>>(o, c.x.p, c.y.p, c.Z.p, c.block_start.p, e->params_proj.p, pa, s0)
+                    : tab ? mse::k_phase_projected<0, true><<<grid, 256, 0, e->stream>>>(o, c.x.p, c.y.p, c.Z.p, c.block_start.p, e->params_proj.p, pa, s0)
                         : mse::k_phase_projected<0><<<grid, 256, 0, e->stream>>>(o, c.x.p, c.y.p, c.Z.p, c.block_start.p, e->params_proj.p, pa, s0);
                 else if (e->form == 1)
-                    tab ? mse::k_phase_projected<1, true><<<grid, 256, 0, e->stream>>>(o, c.x.p, c.y.p, c.Z.p, c.block_start.p, e->params_proj.p, pa, s0)
+                    lds ? mse::k_phase_projected<1, true, true><<<grid, 256, lds, e->stream>>>(o, c.x.p, c.y.p, c.Z.p, c.block_start.p, e->params_proj.p, pa, s0)
+                    : tab ? mse::k_phase_projected<1, true><<<grid, 256, 0, e->stream>>>(o, c.x.p, c.y.p, c.Z.p, c.block_start.p, e->params_proj.p, pa, s0)
                         : mse::k_phase_projected<1><<<grid, 256, 0, e->stream>>>(o, c.x.p, c.y.p, c.Z.p, c.block_start.p, e->params_proj.p, pa, s0);
                 else
-                    tab ? mse::k_phase_projected<2, true><<<grid, 256, 0, e->stream>>>(o, c.x.p, c.y.p, c.Z.p, c.block_start.p, e->params_proj.p, pa, s0)
+                    lds ? mse::k_phase_projected<2, true, true><<<grid, 256, lds, e->stream>>>(o, c.x.p, c.y.p, c.Z.p, c.block_start.p, e->params_proj.p, pa, s0)
+                    : tab ? mse::k_phase_projected<2, true><<<grid, 256, 0, e->stream>>>(o, c.x.p, c.y.p, c.Z.p, c.block_start.p, e->params_proj.p, pa, s0)
                         : mse::k_phase_projected<2><<<grid, 256, 0, e->stream>>>(o, c.x.p, c.y.p, c.Z.p, c.block_start.p, e->params_proj.p, pa, s0);
             });
         }

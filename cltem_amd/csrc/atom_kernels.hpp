@@ -456,6 +456,12 @@ struct PotArgs {
     double rrx, rry;
     float inv_ps, reach_px2;
     float inside_px2;  // (8 A - a margin of 0.01 A^2)^2 in pixels^2
+    // the projected kernels: beyond this many pixels^2 an atom needs no test against r_min and no
+    // table below kProjLdsLo.  With LDS = true they copy the buckets from kProjLdsLo to 64 A^2 of
+    // the lds_n elements whose numbers are the bytes of lds_z.
+    float near_px2;
+    int lds_n;
+    unsigned long long lds_z;
 };
 
 // An element's device table as an address biased so that the bucket of r2 sits at byte
@@ -509,6 +515,21 @@ __device__ __forceinline__ float vtab_cubic(float4 c, float r2) {
 __device__ __forceinline__ float vtab_eval_in(unsigned long long base, float r2) {
     return vtab_cubic(vtab_bucket(base, r2), r2);
 }
+
+// The reach of the projected potentials:
+// rad = max(sqrt(r2), r_min) <= 8 with r2 <= 64.0000000001 (the
+// reference's test, correctly rounded double sqrt): sqrt(64 + 2^-46) =
+// 8 + 2^-50 - 2^-103... rounds to 8 while sqrt of the next double,
+// 64 + 2^-45, rounds to 8 + 2^-49, so the test is exactly
+// r2 <= 64 + 2^-46.  The potential takes rad in float.
+constexpr double kProjReach2 = 0x1.0000000000001p+6;
+
+// The projected kernels' LDS copy of the tables: kProjLdsBuckets buckets an element, from
+// r^2 = kProjLdsLo (r = 1/4 A) up to the one of 64 A^2 itself.
+constexpr float kProjLdsLo = 0.0625f;
+constexpr int kProjLdsFirst = (127 - 4) << mse_tab::kSubBits;
+constexpr int kProjLdsBuckets = (10 << mse_tab::kSubBits) + 1;
+constexpr int kProjLdsElements = 5;  // five blocks a CU, as many as the registers allow
 
 // V(r2) as vtab_eval computes it, from the LDS copy of an element's buckets
 // [vb_lo, vb_lo + vb_n), which starts at lt[off + vb_lo]; r2 must lie in those buckets
@@ -614,20 +635,23 @@ __device__ __forceinline__ int tile_pixel_y(int j) {
 
 // Projected potential sums (sumz) of slice `slice` at PX x PY pixels per thread, sumz[j PX + i]
 // for pixel (tile_pixel_x(i), tile_pixel_y(j)).  The atoms of the tile's block rows are staged
-// through LDS as one sequence, in chunks of 256, with no limit on how many a row holds.  (The
-// tables stay in global memory here: one evaluation per atom and pixel is too little work to
-// repay an LDS copy per block.)
-// VALU issue bounds it: 13 instructions per evaluation where the wave's pixels need no test (11
-// of them the double add of the squared distance, the conversion, the bucket's offset and its
-// cubic, and the double sum), about twice that with the tests, which also put one table read
-// after the other.  Taking the tests out of the pairs that cannot need them, and each wave's list
-// of its own atoms: 768^2, 63 slices 417 -> 372 us; 1024^2, 24 slices 258 -> 238 us; 12 planes of
-// 256^2 29 -> 23 us.
-template <int FORM, bool TAB, int PX = 1, int PY = 1>
+// through LDS as one sequence, in chunks of 256, with no limit on how many a row holds.
+// VALU issue bounds it (1 450 instructions a wave, one a cycle and CU): 14 to 16 instructions per
+// evaluation, 11 of them the double add of the squared distance, the conversion, the bucket's
+// address and its cubic, and the double sum.  Taking the tests out of the pairs that cannot need
+// them, and each wave's list of its own atoms: 768^2, 63 slices 417 -> 390 us; 1024^2, 24 slices
+// 258 -> 242 us.  With the tables in global memory their reads, 64 lanes of 16 bytes, kept the
+// vector memory path as busy as the VALU (92 %); LDS = true reads them from a copy the block makes
+// with its first atoms, 5 KB an element, and a wave with pixels beyond 8 A evaluates all of them
+// and drops those: 390 -> 373 us and 242 -> 233 us; 15 frames of 24 slices at 256^2 192 -> 180 us.
+// (That evaluation with the global tables 395 us, the copy with a test per pixel 411 us.  Several
+// slices a block, for one copy and one block range: 388 us, more registers and fewer waves.)
+template <int FORM, bool TAB, bool LDS, int PX = 1, int PY = 1>
 __device__ __forceinline__ void projected_sumz(const double* __restrict__ ax, const double* __restrict__ ay,
                                                const int* __restrict__ aZ, const int* __restrict__ bsp,
                                                const float* __restrict__ ptab, const PotArgs& a, int slice,
-                                               double* sx, double* sy, int* sZ, double (&sumz)[PX * PY]) {
+                                               double* sx, double* sy, int* sZ, float4* lt,
+                                               double (&sumz)[PX * PY]) {
 #pragma clang fp contract(off)
     const int lid = threadIdx.x;
     int starti, endi, startj, endj;
@@ -651,6 +675,7 @@ __device__ __forceinline__ void projected_sumz(const double* __restrict__ ax, co
     const double tile_y0 = a.starty + (int)(blockIdx.y * PY * 16) * a.pixelscale;
     const float inv_ps = a.inv_ps;
     const float reach_px2 = a.reach_px2;
+    bool tables = !LDS;  // the LDS copy is made with the first atoms: empty tiles need none
 #pragma unroll
     for (int i = 0; i < PX * PY; ++i) sumz[i] = 0.0;
     const int nb = a.blocks_x * a.blocks_y;
@@ -686,10 +711,11 @@ __device__ __forceinline__ void projected_sumz(const double* __restrict__ ax, co
             // bits 16..19: the waves (pixel quadrants of the tile) that may have a pixel
             // within 8 A; the distance to each wave's pixel rectangle, in pixels and in
             // float, is tested against 64.01 A^2, a margin far above the float error.
-            // Bits 20..23: the waves all of whose pixels lie within 8 A (the rectangle's
-            // farthest corner, against 63.99 A^2) and farther than r_min = 1/4 pixel (its
-            // nearest point, against 0.26 pixels), where the potential needs no test.
-            // Untilted only (a tilted metric is no lateral distance): all waves otherwise.
+            // Bits 20..23: the waves all of whose pixels are farther than r_min = 1/4 pixel
+            // (their nearest point, against 0.26 pixels) and than kProjLdsLo; bits 24..27:
+            // those of them all of whose pixels lie within 8 A too (the farthest corner,
+            // against 63.99 A^2).  Untilted only (a tilted metric is no lateral distance):
+            // all waves otherwise.  Bits 28..30: the element's slot in LDS.
             unsigned waves = 15u;
             if (a.untilted) {
                 waves = 0;
@@ -704,10 +730,24 @@ __device__ __forceinline__ void projected_sumz(const double* __restrict__ ax, co
                     const float d2 = du * du + dv * dv;
                     const float fu = fmaxf(u - u0, u1 - u), fv = fmaxf(v - v0, v1 - v);
                     if (d2 <= reach_px2) waves |= 1u << w;
-                    if (d2 > 0.26f * 0.26f && fu * fu + fv * fv <= a.inside_px2) waves |= 16u << w;
+                    if (d2 > a.near_px2) waves |= (fu * fu + fv * fv <= a.inside_px2 ? 0x110u : 0x10u) << w;
                 }
             }
-            sZ[lid] = aZ[c] | (int)(waves << 16);
+            const int Z = aZ[c];
+            if constexpr (LDS) {
+#pragma unroll
+                for (int q = 1; q < kProjLdsElements; ++q)
+                    if ((int)((a.lds_z >> (8 * q)) & 255) == Z) waves |= (unsigned)q << 12;
+            }
+            sZ[lid] = (int)((unsigned)Z | waves << 16);
+        }
+        if (!tables) {
+            tables = true;
+            for (int q = 0; q < a.lds_n; ++q) {
+                const float4* from = a.vtab + (size_t)((int)((a.lds_z >> (8 * q)) & 255) - 1) * mse_tab::kBuckets +
+                                     (kProjLdsFirst - ((127 + mse_tab::kOctaveLo) << mse_tab::kSubBits));
+                for (int i = lid; i < kProjLdsBuckets; i += 256) lt[q * kProjLdsBuckets + i] = from[i];
+            }
         }
         __syncthreads();
         // the wave's own atoms of each 64 staged: their list is a mask in scalar registers, so
@@ -716,27 +756,19 @@ __device__ __forceinline__ void projected_sumz(const double* __restrict__ ax, co
             const int li = l0 + (lid & 63);
             const int infos = li < cnt ? sZ[li] : 0;
             unsigned long long todo = __builtin_amdgcn_ballot_w64((infos >> (16 + wave)) & 1);
-            const unsigned long long plain = __builtin_amdgcn_ballot_w64((infos >> (20 + wave)) & 1);
+            const unsigned long long far = __builtin_amdgcn_ballot_w64((infos >> (20 + wave)) & 1);
+            const unsigned long long inside = __builtin_amdgcn_ballot_w64((infos >> (24 + wave)) & 1);
             while (todo) {
                 const int b = __builtin_ctzll(todo);
                 const int l = l0 + b;
                 todo &= todo - 1;
-                const int zs = __builtin_amdgcn_readlane(infos, b) & 0xffff;
-                // the element's constants (or table), loaded ahead of the distance arithmetic
-                float pt[TAB ? 1 : kPotProjStride];
-                unsigned long long tz = 0;
-                if constexpr (TAB) {
-                    tz = vtab_base(a.vtab + (size_t)(zs - 1) * mse_tab::kBuckets);
-                } else {
-                    const float* row = ptab + (size_t)(zs - 1) * kPotProjStride;
-#pragma unroll
-                    for (int q = 0; q < kPotProjStride; ++q) pt[q] = row[q];
-                }
+                const int info = __builtin_amdgcn_readlane(infos, b);
+                const int zs = info & 0xffff;
                 const double xl = sx[l], yl = sy[l];
                 if constexpr (TAB) {
-                    if ((plain >> b) & 1) {
-                        // every pixel of the wave takes part and none is clamped: the pixels'
-                        // table reads are issued together
+                    if ((far >> b) & 1) {
+                        // no pixel of the wave is clamped: the pixels' table reads are issued
+                        // together, those of a pixel beyond 8 A at 64 A^2 and left out of the sum
                         double rx2[PX], ry2[PY];
 #pragma unroll
                         for (int i = 0; i < PX; ++i) {
@@ -748,17 +780,55 @@ __device__ __forceinline__ void projected_sumz(const double* __restrict__ ax, co
                             const double d = im_pos_y[jy] - yl;
                             ry2[jy] = d * d;
                         }
-                        float f[PX * PY];
-                        float4 cb[PX * PY];
+                        auto add = [&](auto all) {
+                            constexpr bool ALL = decltype(all)::value;
+                            float f[PX * PY];
+                            bool in[PX * PY];
+                            float4 cb[PX * PY];
+                            if constexpr (LDS) {
+                                const int off = (int)((unsigned)info >> 28) * kProjLdsBuckets - kProjLdsFirst;
+                                unsigned bk[PX * PY];
 #pragma unroll
-                        for (int q = 0; q < PX * PY; ++q) {
-                            f[q] = (float)(rx2[q % PX] + ry2[q / PX]);
-                            cb[q] = vtab_bucket(tz, f[q]);
-                        }
+                                for (int q = 0; q < PX * PY; ++q) {
+                                    const double r2 = rx2[q % PX] + ry2[q / PX];
+                                    in[q] = ALL || r2 <= kProjReach2;
+                                    f[q] = ALL ? (float)r2 : fminf((float)r2, 64.f);
+                                    asm("v_lshrrev_b32 %0, %1, %2" : "=v"(bk[q]) : "i"(mse_tab::kMantBits), "v"(__float_as_uint(f[q])));
+                                }
 #pragma unroll
-                        for (int q = 0; q < PX * PY; ++q) sumz[q] += (double)vtab_cubic(cb[q], f[q]);
+                                for (int q = 0; q < PX * PY; ++q) cb[q] = lt[(int)bk[q] + off];
+                            } else {
+                                const unsigned long long tz = vtab_base(a.vtab + (size_t)(zs - 1) * mse_tab::kBuckets);
+#pragma unroll
+                                for (int q = 0; q < PX * PY; ++q) {
+                                    const double r2 = rx2[q % PX] + ry2[q / PX];
+                                    in[q] = ALL || r2 <= kProjReach2;
+                                    f[q] = ALL ? (float)r2 : fminf((float)r2, 64.f);
+                                    cb[q] = vtab_bucket(tz, f[q]);
+                                }
+                            }
+#pragma unroll
+                            for (int q = 0; q < PX * PY; ++q) {
+                                const float v = vtab_cubic(cb[q], f[q]);
+                                sumz[q] += (double)(in[q] ? v : 0.f);
+                            }
+                        };
+                        if ((inside >> b) & 1)
+                            add(std::true_type{});
+                        else
+                            add(std::false_type{});
                         continue;
                     }
+                }
+                // the element's constants (or table), loaded ahead of the distance arithmetic
+                float pt[TAB ? 1 : kPotProjStride];
+                unsigned long long tz = 0;
+                if constexpr (TAB) {
+                    tz = vtab_base(a.vtab + (size_t)(zs - 1) * mse_tab::kBuckets);
+                } else {
+                    const float* row = ptab + (size_t)(zs - 1) * kPotProjStride;
+#pragma unroll
+                    for (int q = 0; q < kPotProjStride; ++q) pt[q] = row[q];
                 }
 #pragma unroll
                 for (int jy = 0; jy < PY; ++jy) {
@@ -778,12 +848,7 @@ __device__ __forceinline__ void projected_sumz(const double* __restrict__ ax, co
                             const double y_prime = rad_y + zt * a.sin_phi;
                             r2 = z_prime * z_prime + x_prime * x_prime + y_prime * y_prime;
                         }
-                        // rad = max(sqrt(r2), r_min) <= 8 with r2 <= 64.0000000001 (the
-                        // reference's test, correctly rounded double sqrt): sqrt(64 + 2^-46) =
-                        // 8 + 2^-50 - 2^-103... rounds to 8 while sqrt of the next double,
-                        // 64 + 2^-45, rounds to 8 + 2^-49, so the test is exactly
-                        // r2 <= 64 + 2^-46.  The potential takes rad in float.
-                        if (r2 <= 0x1.0000000000001p+6) {
+                        if (r2 <= kProjReach2) {
                             if constexpr (TAB) {
                                 // r_min^2 is above the tables' floor (the host enables them only
                                 // then) and r2 <= 64 + 2^-46 is 64 or less in float, far inside
@@ -820,18 +885,19 @@ __device__ __forceinline__ void fill_lds_tables(const PotArgs& a, float4* lt) {
 // slice (relative to first).  Grid (res / (16 kProjPX), res / (16 kProjPY), planes):
 // (16 kProjPX)x(16 kProjPY) pixel tiles, 16x16 pixels per wave.
 constexpr int kProjPX = 2, kProjPY = 2;
-template <int FORM, bool TAB = false>
+template <int FORM, bool TAB = false, bool LDS = false>
 __global__ __launch_bounds__(256) void k_potential_projected(
     float2* __restrict__ out, const double* __restrict__ ax, const double* __restrict__ ay,
     const int* __restrict__ aZ, const int* __restrict__ bsp, const float* __restrict__ ptab,
     PotArgs a, int first) {
     __shared__ double sx[256], sy[256];
     __shared__ int sZ[256];
+    extern __shared__ float4 lt[];
     PotArgs b;
     const int slice = plane_args(a, first, b);
     // kProjPX x kProjPY pixels per thread: the atom's staging, loads and wave test serve them all
     double sumz[kProjPX * kProjPY];
-    projected_sumz<FORM, TAB, kProjPX, kProjPY>(ax, ay, aZ, bsp, ptab, b, slice, sx, sy, sZ, sumz);
+    projected_sumz<FORM, TAB, LDS, kProjPX, kProjPY>(ax, ay, aZ, bsp, ptab, b, slice, sx, sy, sZ, lt, sumz);
 #pragma unroll
     for (int j = 0; j < kProjPY; ++j) {
         const int yid = tile_pixel_y<kProjPX, kProjPY>(j);
@@ -847,15 +913,16 @@ __global__ __launch_bounds__(256) void k_potential_projected(
 // The phase sigma V of the same slices, reduced to [-pi, pi] as phase_to_t reduces it, so
 // that sincosf of the stored float reproduces the transmission function's exp(i sigma V)
 // before the band limit (used by the adjoint).  Grid as k_potential_projected's.
-template <int FORM, bool TAB = false>
+template <int FORM, bool TAB = false, bool LDS = false>
 __global__ __launch_bounds__(256) void k_phase_projected(
     float* __restrict__ out, const double* __restrict__ ax, const double* __restrict__ ay,
     const int* __restrict__ aZ, const int* __restrict__ bsp, const float* __restrict__ ptab,
     PotArgs a, int first) {
     __shared__ double sx[256], sy[256];
     __shared__ int sZ[256];
+    extern __shared__ float4 lt[];
     double sumz[kProjPX * kProjPY];
-    projected_sumz<FORM, TAB, kProjPX, kProjPY>(ax, ay, aZ, bsp, ptab, a, first + (int)blockIdx.z, sx, sy, sZ, sumz);
+    projected_sumz<FORM, TAB, LDS, kProjPX, kProjPY>(ax, ay, aZ, bsp, ptab, a, first + (int)blockIdx.z, sx, sy, sZ, lt, sumz);
 #pragma unroll
     for (int j = 0; j < kProjPY; ++j) {
         const int yid = tile_pixel_y<kProjPX, kProjPY>(j);

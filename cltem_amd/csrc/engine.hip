@@ -344,6 +344,9 @@ mse::PotArgs pot_args(mse_engine* e, const ConfigData& c) {
     a.inv_ps = (float)(1.0 / a.pixelscale);
     a.reach_px2 = (float)(64.01 / (a.pixelscale * a.pixelscale));
     a.inside_px2 = (float)(63.99 / (a.pixelscale * a.pixelscale));
+    a.near_px2 = 0.26f * 0.26f;
+    a.lds_n = 0;
+    a.lds_z = 0;
     a.load_x = g.load_x;
     a.load_y = g.load_y;
     a.load_z = g.load_z;
@@ -1369,8 +1372,7 @@ const float4* potential_tables(mse_engine* e, const ConfigData& c, const mse_geo
 // the configuration and the buckets an untilted slice reaches, from r_min^2 as the kernels
 // round it (at least the tables' floor) to 64 + ((load_z + 2) dz)^2.  Returns the bytes of
 // LDS it takes, or 0 where the global tables are used instead: a tilted beam, or tables over
-// 32 KB.  (The projected kernels, one evaluation per atom and pixel, read the global tables:
-// an LDS copy per block costs them more than it saves.)
+// 32 KB.
 static size_t lds_tables(mse_engine* e, const ConfigData& c, const mse_geometry& g, mse::PotArgs& a) {
     if (!g.full3d || a.shift_x != 0.0 || a.shift_y != 0.0) return 0;
     const float r_min = (float)(0.25 * a.pixelscale);
@@ -1413,6 +1415,27 @@ static size_t lds_tables(mse_engine* e, const ConfigData& c, const mse_geometry&
     return bytes;
 }
 
+// The projected kernels' LDS copy (PotArgs::lds_n, lds_z, near_px2): the bytes of LDS it takes, or 0
+// where the global tables are used instead: a tilted beam, whose distances the copy need not hold,
+// or more than kProjLdsElements elements, whose copies would leave fewer blocks a CU than the registers do (six: 496 us against
+// 467 from global memory for 27 slices of 1024^2; three: 457 against 467).
+size_t projected_lds_tables(mse_engine* e, const ConfigData& c, mse::PotArgs& a) {
+    if (!e->vtab_lds || !a.vtab || !a.untilted) return 0;
+    int n = 0;
+    unsigned long long zs = 0;
+    for (int Z = 1; Z < (int)c.has_Z.size(); ++Z) {
+        if (!c.has_Z[Z]) continue;
+        if (Z > e->max_Z || Z > 255 || n == mse::kProjLdsElements) return 0;
+        zs |= (unsigned long long)Z << (8 * n++);
+    }
+    if (n == 0) return 0;
+    a.lds_n = n;
+    a.lds_z = zs;
+    // 0.255 A: the margin to kProjLdsLo covers the float arithmetic of the waves' test
+    a.near_px2 = std::max(a.near_px2, (float)(0.255 * 0.255 / (a.pixelscale * a.pixelscale)));
+    return (size_t)n * mse::kProjLdsBuckets * sizeof(float4);
+}
+
 void potential_planes(mse_engine* e, const ConfigData& c, const mse_geometry& g, const mse::PotArgs& args,
                       float2* out, int planes, int first) {
     require_elements(e, c);
@@ -1422,7 +1445,7 @@ void potential_planes(mse_engine* e, const ConfigData& c, const mse_geometry& g,
     mse::PotArgs a = args;
     a.vtab = potential_tables(e, c, g);
     const bool tab = a.vtab != nullptr;
-    const size_t lds = tab && e->vtab_lds ? lds_tables(e, c, g, a) : 0;
+    const size_t lds = !tab ? 0 : !g.full3d ? projected_lds_tables(e, c, a) : e->vtab_lds ? lds_tables(e, c, g, a) : 0;
     launch(e, PK_POT, [&]() {
         if (g.full3d && lds) {
             if (e->form == 0)
@@ -1443,13 +1466,16 @@ void potential_planes(mse_engine* e, const ConfigData& c, const mse_geometry& g,
                     : mse::k_potential_full3d<2><<<grid, 256, 0, e->stream>>>(out, c.x.p, c.y.p, c.z.p, c.Z.p, c.block_start.p, e->params3d.p, a, first);
         } else {
             if (e->form == 0)
-                tab ? mse::k_potential_projected<0, true><<<grid_proj, 256, 0, e->stream>>>(out, c.x.p, c.y.p, c.Z.p, c.block_start.p, e->params_proj.p, a, first)
+                lds ? mse::k_potential_projected<0, true, true><<<grid_proj, 256, lds, e->stream>>>(out, c.x.p, c.y.p, c.Z.p, c.block_start.p, e->params_proj.p, a, first)
+                : tab ? mse::k_potential_projected<0, true><<<grid_proj, 256, 0, e->stream>>>(out, c.x.p, c.y.p, c.Z.p, c.block_start.p, e->params_proj.p, a, first)
                     : mse::k_potential_projected<0><<<grid_proj, 256, 0, e->stream>>>(out, c.x.p, c.y.p, c.Z.p, c.block_start.p, e->params_proj.p, a, first);
             else if (e->form == 1)
-                tab ? mse::k_potential_projected<1, true><<<grid_proj, 256, 0, e->stream>>>(out, c.x.p, c.y.p, c.Z.p, c.block_start.p, e->params_proj.p, a, first)
+                lds ? mse::k_potential_projected<1, true, true><<<grid_proj, 256, lds, e->stream>>>(out, c.x.p, c.y.p, c.Z.p, c.block_start.p, e->params_proj.p, a, first)
+                : tab ? mse::k_potential_projected<1, true><<<grid_proj, 256, 0, e->stream>>>(out, c.x.p, c.y.p, c.Z.p, c.block_start.p, e->params_proj.p, a, first)
                     : mse::k_potential_projected<1><<<grid_proj, 256, 0, e->stream>>>(out, c.x.p, c.y.p, c.Z.p, c.block_start.p, e->params_proj.p, a, first);
             else
-                tab ? mse::k_potential_projected<2, true><<<grid_proj, 256, 0, e->stream>>>(out, c.x.p, c.y.p, c.Z.p, c.block_start.p, e->params_proj.p, a, first)
+                lds ? mse::k_potential_projected<2, true, true><<<grid_proj, 256, lds, e->stream>>>(out, c.x.p, c.y.p, c.Z.p, c.block_start.p, e->params_proj.p, a, first)
+                : tab ? mse::k_potential_projected<2, true><<<grid_proj, 256, 0, e->stream>>>(out, c.x.p, c.y.p, c.Z.p, c.block_start.p, e->params_proj.p, a, first)
                     : mse::k_potential_projected<2><<<grid_proj, 256, 0, e->stream>>>(out, c.x.p, c.y.p, c.Z.p, c.block_start.p, e->params_proj.p, a, first);
         }
     });

@@ -309,8 +309,9 @@ int mse_stem_batch_frames(mse_engine* e, int config, const double* pos_xy, const
  *      (kernels/transmission_potentials_projected_d.cl:71-181,
  *      kernels/transmission_potentials_full_3d_d.cl:57-134).  Geometries whose distances leave
  *      that range (pixels below 0.004 A, full-3D depth reach above 13.8 A) evaluate the
- *      formulas directly.  The full-3D kernels of an untilted beam copy the buckets a slice
- *      reaches into LDS when they take at most 32 KB; enable = 2 keeps every read in global
+ *      formulas directly.  The kernels of an untilted beam copy the buckets they read into LDS,
+ *      full 3D when those of a slice take at most 32 KB, projected for at most five elements;
+ *      enable = 2 keeps every read in global
  *      memory (same values; for tests), enable = 0 always evaluates the formulas directly.
  *      The next mse_build_transmission uses the choice.  No clTEM counterpart. ---- */
 int mse_set_potential_tables(mse_engine* e, int enable);
