@@ -240,6 +240,20 @@ int tuned_variant(const mse_engine* e, int nsets, bool column) {
     return column ? e->col_var : e->row_var;
 }
 
+// Whether the column passes write through to memory (store_through).  The row passes, whose lanes
+// write whole lines, always do; a tile of 8 columns writes half lines, which cost more once the
+// waves come from memory rather than from the L2s and the cache behind them.  us per slice (row and
+// column pass, captured loop) with neither / the rows / both written through:
+//   256^2 one wave 8.7 / 8.7 / 8.7, 16 waves 15.3 / 13.1 / 11.9, 32 24.9 / 20.6 / 14.9, 128 41.6 / 40.7 / 40.7
+//   384^2 one 12.4 / 12.2 / 12.6, 16 waves 29.8 / 24.6 / 20.3, 48 47.0 / 47.1 / 43.8
+//   512^2 one 11.4 / 11.2 / 11.3, 8 waves 26.1 / 22.2 / 18.0, 64 75.0 / 74.4 / 73.2
+//   768^2 one 17.0 / 16.1 / 16.4, 4 waves 30.6 / 24.9 / 22.5, 16 59.4 / 58.8 / 58.2, 24 80.7 / 79.5 / 80.1, 96 304 / 303 / 336
+//   1024^2 one 21.7 / 19.7 / 19.9, 2 waves 30.0 / 24.8 / 22.8, 4 37.9 / 34.9 / 35.9, 8 54.5 / 53.0 / 53.0, 32 154 / 154 / 161
+static bool columns_through(int res, int nsets) {
+    const long long mib = 8 * (long long)res * res * nsets >> 20;
+    return res <= 512 || mib <= (res == 768 ? 80 : 24);
+}
+
 void row_pass(mse_engine* e, int mode, const float2* in, float2* out, int nlines_sets,
               size_t wave_stride, const mse::RowArgs& args, int variant) {
     if (variant == kEngineChoice) variant = tuned_variant(e, nlines_sets, false);
@@ -255,8 +269,10 @@ void row_pass(mse_engine* e, int mode, const float2* in, float2* out, int nlines
 
 // returns the number of column tiles of the launch (detector partials per wave)
 int col_pass(mse_engine* e, int mode, const float2* in, float2* out, int nsets, size_t wave_stride,
-             const mse::ColArgs& args, int kind, int variant) {
+             const mse::ColArgs& args0, int kind, int variant) {
     if (variant == kEngineChoice) variant = tuned_variant(e, nsets, true);
+    mse::ColArgs args = args0;
+    args.through = columns_through(e->res, nsets);
     switch (e->res) {
         case 256: return col_pass_n<256>(e, mode, in, out, nsets, wave_stride, args, kind, variant);
         case 384: return col_pass_n<384>(e, mode, in, out, nsets, wave_stride, args, kind, variant);

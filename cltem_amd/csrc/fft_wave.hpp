@@ -31,6 +31,41 @@ __device__ __forceinline__ float2 cmulc(float2 a, float2 b) {
 }
 __device__ __forceinline__ float2 cscale(float2 a, float s) { return make_float2(a.x * s, a.y * s); }
 
+// ---- stores of planes that the next kernel reads -----------------------------------
+// Written through to memory (sc1, the agent scope) instead of left dirty in the writing XCD's L2.
+// The passes read each plane across the direction they wrote it in, from other XCDs, and a line
+// that another XCD's L2 holds dirty comes slower than one from the memory side: 8 x 1 MB read and
+// written on other XCDs than the launch before 6.7 us a launch, 3.5 written through; 8 x 2 MB 11.8
+// and 5.7; 8 x 6 MB, more than the L2s hold, 14.8 both ways.
+__device__ __forceinline__ void store_through(float2* p, float2 v) {
+    unsigned long long b;
+    __builtin_memcpy(&b, &v, sizeof(b));
+    __hip_atomic_store(reinterpret_cast<unsigned long long*>(p), b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// 16-byte stores at byte offsets from a pointer that is the same in every lane of the wave
+template <bool THROUGH>
+struct ColumnOut {
+    __amdgpu_buffer_rsrc_t rsrc;
+    __device__ __forceinline__ explicit ColumnOut(float2* p) {
+        const unsigned long long u = reinterpret_cast<unsigned long long>(p);
+        const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)u), hi = __builtin_amdgcn_readfirstlane((unsigned)(u >> 32));
+        rsrc = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>((unsigned long long)hi << 32 | lo), 0,
+                                                 0xffffffff, 0x00027000);
+    }
+    __device__ __forceinline__ void store(unsigned off, float4 v) const {
+        using u4 = unsigned __attribute__((ext_vector_type(4)));
+        u4 b;
+        __builtin_memcpy(&b, &v, sizeof(b));
+        __builtin_amdgcn_raw_buffer_store_b128(b, rsrc, off, 0, 16);
+    }
+};
+template <>
+struct ColumnOut<false> {
+    char* p;
+    __device__ __forceinline__ explicit ColumnOut(float2* q) : p(reinterpret_cast<char*>(q)) {}
+    __device__ __forceinline__ void store(unsigned off, float4 v) const { *reinterpret_cast<float4*>(p + off) = v; }
+};
+
 // ---- compile-time trigonometry for the small-DFT internal twiddles -----------------
 constexpr double kTwoPi = 6.283185307179586476925286766559;
 constexpr double ct_cos_series(double x) {

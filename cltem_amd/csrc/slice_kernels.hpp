@@ -140,6 +140,7 @@ struct ColArgs {
     const float* filter;     // COL_FILTER: res*res real factors, row-major [ky][kx] (unshifted)
     const double* kx;        // k-grid (COL_PROBE)
     const double* ky;
+    int through;  // store the waves written through to memory (the launch's rule)
     // COL_PROP*: largest |kx index| that lim keeps, for the sweeps on the band alone (the row
     // pass before must have left the columns outside it at zero); COL_PROBE: largest |kx index| of
     // the columns to write (the rest is left as it was); -1: every column
@@ -182,14 +183,14 @@ __device__ __forceinline__ void band_store(const float2 (&v)[PL::E], float2* dst
     for (int m = 0; m < PL::E; ++m) {
         const int x = t + L * m;
         if (IO == BAND_FULL || IO == BAND_READ || band_class<N, L>(m) == BAND_IN) {
-            dst[x] = v[m];
+            store_through(dst + x, v[m]);
         } else if (band_class<N, L>(m) == BAND_EDGE) {
             if (in_band(x, N, k))
-                dst[x] = v[m];
+                store_through(dst + x, v[m]);
             else if (IO == BAND_FIRST)
-                dst[x] = make_float2(0.f, 0.f);
+                store_through(dst + x, make_float2(0.f, 0.f));
         } else if (IO == BAND_FIRST) {
-            dst[x] = make_float2(0.f, 0.f);
+            store_through(dst + x, make_float2(0.f, 0.f));
         }
     }
 }
@@ -240,7 +241,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
     }
     if constexpr (MODE == ROW_COPY) {
 #pragma unroll
-        for (int m = 0; m < E; ++m) out[base + t + L * m] = v[m];
+        for (int m = 0; m < E; ++m) store_through(out + base + t + L * m, v[m]);
         return;
     }
     if constexpr (MODE == ROW_ADJ_SEED || MODE == ROW_ADJ) {
@@ -263,7 +264,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
             for (int m = 0; m < E; ++m) {
                 const float2 u = make_float2(v[m].x * inv, v[m].y * inv);
                 const float2 psi = make_float2(ps[m].x * inv, ps[m].y * inv);
-                gt[t + L * m] = cmulc(u, psi);  // conj(psi) u
+                store_through(gt + t + L * m, cmulc(u, psi));  // conj(psi) u
                 const float2 tv = has_t ? tr[m] : make_float2(1.f, 0.f);
                 v[m] = cmulc(u, tv);  // conj(t) u
             }
@@ -454,9 +455,9 @@ __global__ __launch_bounds__(TC * PL::L) __attribute__((amdgpu_waves_per_eu(WPE)
     if constexpr (MODE == COL_PROBE) {
         // columns outside the aperture are zero: |k| >= |kx| in every rounding step
         if (fmin(fabs(a.kx[x0]), fabs(a.kx[x0 + TC - 1])) >= a.probe.cond_ap2 + a.probe.smooth_r) {
-            float4* out4 = reinterpret_cast<float4*>(out + wbase + x0);
+            const ColumnOut<true> out4(out + wbase + x0);
             for (int idx = tid; idx < TC * N / 2; idx += NT)
-                out4[((size_t)(idx / (TC / 2)) * N) / 2 + idx % (TC / 2)] = make_float4(0.f, 0.f, 0.f, 0.f);
+                out4.store((idx / (TC / 2)) * N * 8 + idx % (TC / 2) * 16, make_float4(0.f, 0.f, 0.f, 0.f));
             return;
         }
     }
@@ -483,12 +484,12 @@ __global__ __launch_bounds__(TC * PL::L) __attribute__((amdgpu_waves_per_eu(WPE)
         }
         __syncthreads();
         if constexpr (MODE == COL_COPY) {
-            float4* out4 = reinterpret_cast<float4*>(out + wbase + x0);
+            const ColumnOut<true> out4(out + wbase + x0);
 #pragma unroll 4
             for (int idx = tid; idx < TC * N / 2; idx += NT) {
                 const int r = idx / (TC / 2), cc = 2 * (idx % (TC / 2));
                 const float2 a0 = tile[cc * CS + lpad(r)], a1 = tile[(cc + 1) * CS + lpad(r)];
-                out4[((size_t)r * N) / 2 + cc / 2] = make_float4(a0.x, a0.y, a1.x, a1.y);
+                out4.store(r * N * 8 + cc * 8, make_float4(a0.x, a0.y, a1.x, a1.y));
             }
             return;
         }
@@ -576,13 +577,16 @@ __global__ __launch_bounds__(TC * PL::L) __attribute__((amdgpu_waves_per_eu(WPE)
 #pragma unroll
         for (int m = 0; m < E; ++m) ln[lpad(t + L * m)] = v[m];
         __syncthreads();
-        float4* out4 = reinterpret_cast<float4*>(out + wbase + x0);
+        auto put = [&](auto through) {
+            const ColumnOut<decltype(through)::value> out4(out + wbase + x0);
 #pragma unroll 4
-        for (int idx = tid; idx < TC * N / 2; idx += NT) {
-            const int r = idx / (TC / 2), cc = 2 * (idx % (TC / 2));
-            const float2 a0 = tile[cc * CS + lpad(r)], a1 = tile[(cc + 1) * CS + lpad(r)];
-            out4[((size_t)r * N) / 2 + cc / 2] = make_float4(a0.x, a0.y, a1.x, a1.y);
-        }
+            for (int idx = tid; idx < TC * N / 2; idx += NT) {
+                const int r = idx / (TC / 2), cc = 2 * (idx % (TC / 2));
+                const float2 a0 = tile[cc * CS + lpad(r)], a1 = tile[(cc + 1) * CS + lpad(r)];
+                out4.store(r * N * 8 + cc * 8, make_float4(a0.x, a0.y, a1.x, a1.y));
+            }
+        };
+        a.through ? put(std::true_type{}) : put(std::false_type{});
     }
 }
 
@@ -635,13 +639,19 @@ __global__ __launch_bounds__(TC * PL::L) __attribute__((amdgpu_waves_per_eu(WPE)
     auto store = [&](int item) {
         const int wv = a.wave_map ? cload(a.wave_map + item / ntiles) : item / ntiles;
         const int xx = tile_column<TC>(a, item % ntiles);
-        float4* out4 = reinterpret_cast<float4*>(data + (size_t)wv * wave_stride + xx);
+        auto put = [&](auto through) {
+            const ColumnOut<decltype(through)::value> out4(data + (size_t)wv * wave_stride + xx);
 #pragma unroll
-        for (int k = 0; k < NQ; ++k) {
-            const int idx = tid + k * NT;
-            const int r = idx / (TC / 2), cc = 2 * (idx % (TC / 2));
-            out4[((size_t)r * N) / 2 + cc / 2] = o[k];
-        }
+            for (int k = 0; k < NQ; ++k) {
+                const int idx = tid + k * NT;
+                const int r = idx / (TC / 2), cc = 2 * (idx % (TC / 2));
+                out4.store(r * N * 8 + cc * 8, o[k]);
+            }
+        };
+        if constexpr (N < 1024)  // (at 1024^2 it runs where waves are not written through, or is one wave)
+            a.through ? put(std::true_type{}) : put(std::false_type{});
+        else
+            put(std::false_type{});
     };
     // With one propagator for every wave the y factors are the same in every tile: a lane
     // keeps its E of them in registers when E <= 8, larger plans read them from an LDS copy
@@ -848,14 +858,17 @@ __device__ __forceinline__ void col_prop_lean(float2* __restrict__ data, size_t 
 #pragma unroll
     for (int m = 0; m < E; ++m) ln[lpad(t + L * m)] = v[m];
     __syncthreads();
-    float4* out4 = reinterpret_cast<float4*>(data + (size_t)wv * wave_stride + x0);
+    auto put = [&](auto through) {
+        const ColumnOut<decltype(through)::value> out4(data + (size_t)wv * wave_stride + x0);
 #pragma unroll
-    for (int k = 0; k < NQ; ++k) {
-        const int idx = tid + k * NT;
-        const int r = idx / (TC / 2), cc = 2 * (idx % (TC / 2));
-        const float2 a0 = tile[cc * CS + lpad(r)], a1 = tile[(cc + 1) * CS + lpad(r)];
-        out4[((size_t)r * N) / 2 + cc / 2] = make_float4(a0.x, a0.y, a1.x, a1.y);
-    }
+        for (int k = 0; k < NQ; ++k) {
+            const int idx = tid + k * NT;
+            const int r = idx / (TC / 2), cc = 2 * (idx % (TC / 2));
+            const float2 a0 = tile[cc * CS + lpad(r)], a1 = tile[(cc + 1) * CS + lpad(r)];
+            out4.store(r * N * 8 + cc * 8, make_float4(a0.x, a0.y, a1.x, a1.y));
+        }
+    };
+    a.through ? put(std::true_type{}) : put(std::false_type{});
 }
 
 // waves per SIMD the lean kernel is held to: 8 (64 VGPRs) with 8 elements per lane, 4 beyond
