@@ -159,11 +159,16 @@ int col_pass_n(mse_engine* e, int mode, const float2* in, float2* out, int nsets
         //   512^2 one 5.8 / 6.4 / 9.8 / 8.7, 8 waves 9.2 / 10.3 / 11.5 / 10.7, 64 49 / 38.8 / 38.9 / 44
         //   768^2 one 8.4 / 10.5 / 27 / 9.0, 4 waves 12.3 / 12.2 / 30 / 11.2, 64 108 / 103 / 235 / 97, 128 255 / 252 / - / 198
         //   1024^2 one 10.3 / 12.1 / 33 / 11.3, 4 waves 22.4 / 20.8 / 42 / 17.9, 16 48 / 48 / 108 / 52, 64 188 / 176 / 407 / 228
-        // (16 columns of the 12- and 16-element plans spill.)
+        // (16 columns of the 12- and 16-element plans spill.)  In a loop, where the row pass comes
+        // between and the waves are written through (us per slice, 4 / 8 / 16 columns / lean):
+        //   256^2 16 waves 11.8 / 11.7 / 11.7 / 12.8, 32 16.6 / 15.0 / 16.0 / 18.7, 64 29.2 / 25.8 / 23.2 / 27.7
+        //   384^2 4 waves 13.3 / 13.7 / 15.6 / 14.9, 8 17.1 / 15.8 / 17.4 / 17.0, 16 23.5 / 20.4 / 20.8 / 20.6
+        //   512^2 8 waves 18.1 / 18.5 / 19.7 / 19.4, 16 32.7 / 29.0 / 29.2 / 28.6, 64 89.8 / 74.2 / 72.8 / 74.1
+        //   768^2 one 16.4 / 18.6 / 36 / 17.5, 4 waves 25.1 / 23.5 / 43 / 22.4; 1024^2 8 waves 53.2 / 53.0 / 101 / 52.7
         const int k = band ? args.band_k : N / 2;
         const auto items = [&](int tc) { return (2 * (k / tc) + 2) * (long long)nsets; };
         const int cus = e->num_cus;
-        if (items(4) <= (P0::E <= 8 ? 3 : N == 384 ? 2 : 1) * cus)
+        if (2 * items(4) <= (P0::E <= 8 ? 6 : N == 384 ? 3 : 2) * cus)
             variant = 5;
         else if (N == 384)
             variant = items(16) <= cus ? 12 : 11;
