@@ -112,6 +112,10 @@ __device__ __forceinline__ float vtab_slope_in(unsigned long long base, float r2
 // derivative of the tabulated forward, with its clamp r2 < r_min^2 and its cutoff), else the
 // derivative of the formulas.  grad has 3 doubles (x, y, z) per input atom, indexed through
 // orig.
+// VALU issue bounds it.  The block ranges per pixel (as a mask of the pixel groups, once a wave), the
+// tilted metric with its divide (tilted beams alone) and a division per pixel for its coordinates
+// were most of it: 2000 atoms at 256^2 72 -> 50 us (a whole
+// gradient at 384^2 2.05 -> 1.92 ms).
 template <int FORM, bool TAB = false>
 __global__ __launch_bounds__(256) void k_atom_grad_projected(
     const double* __restrict__ ax, const double* __restrict__ ay, const int* __restrict__ aZ,
@@ -156,17 +160,39 @@ __global__ __launch_bounds__(256) void k_atom_grad_projected(
     const double dzx = -0.5 * a.cos_phi * a.sin_2theta, dzy = -0.5 * a.sin_phi * a.sin_2theta;
     const double dxx = 1.0 + dzx / a.tan_theta * a.cos_phi, dxy = dzy / a.tan_theta * a.cos_phi;
     const double dyx = dzx / a.tan_theta * a.sin_phi, dyy = 1.0 + dzy / a.tan_theta * a.sin_phi;
+    // the 16x16 pixel groups whose block range holds the atom's block, a bit each (res <= 1024: 64
+    // groups across, lane l looks at group (l, l)); the ends in x hang on the column alone
+    unsigned long long groups_x, groups_y;
+    {
+        const int l = threadIdx.x & 63;
+        int starti, endi, startj, endj;
+        tile_block_range(a, l, l, starti, endi, startj, endj);
+        groups_x = __builtin_amdgcn_ballot_w64(bidx >= starti && bidx <= endi);
+        groups_y = __builtin_amdgcn_ballot_w64(bidy >= startj && bidy <= endj);
+    }
     double gx = 0.0, gy = 0.0;
+    const int step_y = 256 / max(wx, 1), step_x = 256 - step_y * wx;
+    int py = threadIdx.x / max(wx, 1), px = threadIdx.x - py * wx;  // pixel threadIdx.x + 256 i of the window
     for (int q = threadIdx.x; q < npix; q += 256) {
-        const int xid = x0 + q % wx;
-        const int yid = y0 + q / wx;
+        const int xid = x0 + px;
+        const int yid = y0 + py;
+        px += step_x;
+        py += step_y;
+        if (px >= wx) {
+            px -= wx;
+            ++py;
+        }
         const double rad_x = (a.startx + xid * a.pixelscale) - xa;
         const double rad_y = (a.starty + yid * a.pixelscale) - ya;
-        const double z_prime = -0.5 * (rad_x * a.cos_phi + rad_y * a.sin_phi) * a.sin_2theta;
-        const double zt = z_prime / a.tan_theta;
-        const double x_prime = rad_x + zt * a.cos_phi;
-        const double y_prime = rad_y + zt * a.sin_phi;
-        const double r2 = z_prime * z_prime + x_prime * x_prime + y_prime * y_prime;
+        // untilted, z' and its terms vanish below the rounding (projected_sumz)
+        double z_prime = 0.0, x_prime = rad_x, y_prime = rad_y, r2 = rad_x * rad_x + rad_y * rad_y;
+        if (!a.untilted) {
+            z_prime = -0.5 * (rad_x * a.cos_phi + rad_y * a.sin_phi) * a.sin_2theta;
+            const double zt = z_prime / a.tan_theta;
+            x_prime = rad_x + zt * a.cos_phi;
+            y_prime = rad_y + zt * a.sin_phi;
+            r2 = z_prime * z_prime + x_prime * x_prime + y_prime * y_prime;
+        }
         double rad = 0.0;
         if constexpr (TAB) {
             // clamped to V(r_min) (constant) or outside the cutoff r2 <= 64 + 2^-46
@@ -176,9 +202,7 @@ __global__ __launch_bounds__(256) void k_atom_grad_projected(
             rad = sqrt(r2);
             if (rad < r_min || rad > 8.0) continue;  // clamped (constant) or outside the cutoff
         }
-        int starti, endi, startj, endj;
-        tile_block_range(a, xid >> 4, yid >> 4, starti, endi, startj, endj);
-        if (bidx < starti || bidx > endi || bidy < startj || bidy > endj) continue;
+        if (!((groups_x >> (xid >> 4)) & (groups_y >> (yid >> 4)) & 1)) continue;
         const size_t p = (size_t)yid * a.res + xid;
         float s, c;
         sincosf(phase[p], &s, &c);
@@ -191,8 +215,11 @@ __global__ __launch_bounds__(256) void k_atom_grad_projected(
         else
             dv_r = (double)dvproj<FORM>(pz, a.i_count, (float)rad) / rad;
         const double f = a.sigma * dl_dphi * dv_r;
-        const double dr_drx = z_prime * dzx + x_prime * dxx + y_prime * dyx;  // times rad
-        const double dr_dry = z_prime * dzy + x_prime * dxy + y_prime * dyy;
+        double dr_drx = x_prime, dr_dry = y_prime;  // times rad
+        if (!a.untilted) {
+            dr_drx = z_prime * dzx + x_prime * dxx + y_prime * dyx;
+            dr_dry = z_prime * dzy + x_prime * dxy + y_prime * dyy;
+        }
         gx -= f * dr_drx;  // d rad_x / d x_a = -1
         gy -= f * dr_dry;
     }
