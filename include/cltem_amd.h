@@ -294,11 +294,12 @@ int mse_stem_batch(mse_engine* e, int config, const double* pos_xy, int n_probes
  * position is taken relative to that origin (simulationcbed.cpp:54-59) and its potential grid
  * starts there plus the configuration's reference offset (mse_set_reference_offset).  clTEM
  * regenerates every transmission function for each pixel job (initialiseSimulation,
- * microscope/simulationgeneral.cpp:345-358); here, slice by slice, the transmission functions
+ * microscope/simulationgeneral.cpp:345-358); here, some slices at a time, the transmission functions
  * of the batch's frames are built from the sorted atoms of `config` (its transmission
  * functions need not be built), band limited, and each multiplies its own wave.  The engine
- * geometry (grid, field size, optics) is the moving-frame geometry.  Device memory: one
- * transmission plane per wave of the batch.  Eager launches only. */
+ * geometry (grid, field size, optics) is the moving-frame geometry.  Device memory:
+ * one transmission plane per wave of the batch and slice, for as many slices as 512 MiB hold
+ * (one at least).  Eager launches only. */
 int mse_stem_batch_frames(mse_engine* e, int config, const double* pos_xy, const double* frame_xy,
                           int n_probes, int batch, const mse_probe* probe, const mse_detector* dets,
                           int n_det, int sqrt2, double* accum);
@@ -322,16 +323,16 @@ int mse_potential_table(int form, int full3d, const double* params, int n_params
 
 /* ---- tuning: kernel variants of the slice sweeps.  kernel 0 = row pass (variants 0..6):
  *      0 wave-level LDS sync, 1 half lanes per line, 2 block barriers, 3 twiddles read at
- *      use, 4 persistent with the next row prefetched (default), 5 as 4 with half lanes,
+ *      use, 4 persistent with the next row prefetched, 5 as 4 with half lanes,
  *      6 as 4 with twiddles read at use.
  *      kernel 1 = column pass (variants 0..13): 0 16-column tiles, 1 half lanes, 2 8-column
- *      tiles, 3 block barriers, 4/5 twiddles read at use (16/8 columns), 6 32-column tiles,
- *      7 persistent with the next tile prefetched (default), 8 as 7 with half lanes, 9 as 7
- *      with twiddles read at use, 10 as 7 with 8-column tiles, 11 one tile per block at two
- *      blocks per CU, twiddles and propagator rows from LDS (16-column tiles at 512 points,
- *      8-column tiles for the four-pass 768-point plan; every other size, 384 included,
- *      runs variant 7), 12 / 13 as 10 / 7 with the persistent blocks of each XCD taking
- *      consecutive tiles, so that 8-column tiles sharing 128-byte lines meet in one L2.
+ *      tiles, 3 block barriers, 4 twiddles read at use, 5 as 12 with 4-column tiles, 6 32-column
+ *      tiles, 7 persistent with the next tile prefetched, 8 as 7 with half lanes, 9 as 7
+ *      with twiddles read at use, 10 as 7 with 8-column tiles, 11 one tile per block at several
+ *      blocks per CU, twiddles and propagator rows from LDS (16-column tiles up to 512 points,
+ *      8-column tiles beyond), 12 / 13 as 10 / 7 with the blocks of each XCD taking
+ *      consecutive tiles, so that narrow tiles sharing 128-byte lines meet in one L2.
+ *      Without a choice, the grid size and the number of waves decide.
  *      mse_autotune times every variant of both sweeps on n_waves waves of `config`
  *      (reps launches each; times in microseconds per launch) and selects the fastest: sweeps
  *      over that number of waves use it from then on, sweeps over any other number of waves keep
