@@ -144,7 +144,7 @@ constexpr bool rot_x_im(int R, int J, int s2, bool inv) {
 // ---- small DFTs in registers --------------------------------------------------------
 // run<Z>: bit r of Z says that input a[r] is zero (its register is not read).  The sums and
 // differences with those inputs are left out; x + 0 and 0 - x are exact, so every output equals
-// that of run<0> on stored zeros (up to the sign of a zero).
+// that of run<0> on stored zeros (up to the sign of a zero).  SPLIT3: see Dft<3>.
 template <int R, bool INV>
 struct Dft;
 
@@ -166,7 +166,7 @@ __device__ __forceinline__ float2 csub_z(float2 a, float2 b) {
 
 template <bool INV>
 struct Dft<2, INV> {
-    template <int Z = 0>
+    template <int Z = 0, bool SPLIT3 = false>
     static __device__ __forceinline__ void run(float2* a) {
         constexpr bool z0 = Z & 1, z1 = Z & 2;
         const float2 t = a[0], u = a[1];
@@ -175,27 +175,38 @@ struct Dft<2, INV> {
     }
 };
 
+// t - s (-d.y, d.x) with the products rounded before the difference
+__device__ __forceinline__ float2 sub_split(float2 t, float s, float2 d) {
+#pragma clang fp contract(off)
+    const float2 p = make_float2(-s * d.y, s * d.x);
+    return make_float2(t.x - p.x, t.y - p.y);
+}
+
+// Which products enter a fused multiply-add is written out, as in rot: left to the compiler, it
+// depended on where the kernel's loads stood.  Both outputs t2 +- i s d take theirs fused; SPLIT3:
+// the second one's is rounded, the rounding that the inverse transforms of the adjoint's row pass
+// and the forward ones of most of k_col's modes have always had.
 template <bool INV>
 struct Dft<3, INV> {
-    template <int Z = 0>
+    template <int Z = 0, bool SPLIT3 = false>
     static __device__ __forceinline__ void run(float2* a) {
         constexpr bool z0 = Z & 1, z1 = Z & 2, z2 = Z & 4;
         constexpr float s3 = 0.86602540378443864676f;
+        constexpr float s = INV ? s3 : -s3;
         const float2 a0 = z0 ? make_float2(0.f, 0.f) : a[0];
         float2 t1 = cadd_z<z1, z2>(a[1], a[2]);
         float2 t2 = make_float2(a0.x - 0.5f * t1.x, a0.y - 0.5f * t1.y);
         float2 d = csub_z<z1, z2>(a[1], a[2]);
-        // forward: y1 = t2 - i s3 d, y2 = t2 + i s3 d
-        float2 isd = INV ? make_float2(-s3 * d.y, s3 * d.x) : make_float2(s3 * d.y, -s3 * d.x);
+        // y1 = t2 + i s d, y2 = t2 - i s d
         a[0] = cadd_z<z0, z1 && z2>(a0, t1);
-        a[1] = cadd(t2, isd);
-        a[2] = csub(t2, isd);
+        a[1] = make_float2(fmaf(-s, d.y, t2.x), fmaf(s, d.x, t2.y));
+        a[2] = SPLIT3 ? sub_split(t2, s, d) : make_float2(fmaf(s, d.y, t2.x), fmaf(-s, d.x, t2.y));
     }
 };
 
 template <bool INV>
 struct Dft<4, INV> {
-    template <int Z = 0>
+    template <int Z = 0, bool SPLIT3 = false>
     static __device__ __forceinline__ void run(float2* a) {
         constexpr bool z0 = Z & 1, z1 = Z & 2, z2 = Z & 4, z3 = Z & 8;
         float2 t0 = cadd_z<z0, z2>(a[0], a[2]), t1 = csub_z<z0, z2>(a[0], a[2]);
@@ -225,13 +236,13 @@ struct DftComposite {
         for (int r1 = 0; r1 < R1; ++r1) z |= (inner_zero(Z, r1) == (1 << R2) - 1) << r1;
         return z;
     }
-    template <int r1, int Z>
+    template <int r1, int Z, bool SPLIT3>
     static __device__ __forceinline__ void inner(const float2* a, float2* b) {
         if constexpr (((outer_zero(Z) >> r1) & 1) == 0) {
             float2 tmp[R2];
 #pragma unroll
             for (int r2 = 0; r2 < R2; ++r2) tmp[r2] = a[r1 + R1 * r2];
-            Dft<R2, INV>::template run<inner_zero(Z, r1)>(tmp);
+            Dft<R2, INV>::template run<inner_zero(Z, r1), SPLIT3>(tmp);
             twid<r1, 0>(tmp, b);
         }
     }
@@ -243,23 +254,23 @@ struct DftComposite {
             twid<r1, s2 + 1>(tmp, b);
         }
     }
-    template <int r1, int Z>
+    template <int r1, int Z, bool SPLIT3>
     static __device__ __forceinline__ void all_inner(const float2* a, float2* b) {
         if constexpr (r1 < R1) {
-            inner<r1, Z>(a, b);
-            all_inner<r1 + 1, Z>(a, b);
+            inner<r1, Z, SPLIT3>(a, b);
+            all_inner<r1 + 1, Z, SPLIT3>(a, b);
         }
     }
-    template <int Z = 0>
+    template <int Z = 0, bool SPLIT3 = false>
     static __device__ __forceinline__ void run(float2* a) {
         float2 b[R];
-        all_inner<0, Z>(a, b);
+        all_inner<0, Z, SPLIT3>(a, b);
 #pragma unroll
         for (int s2 = 0; s2 < R2; ++s2) {
             float2 tmp[R1];
 #pragma unroll
             for (int r1 = 0; r1 < R1; ++r1) tmp[r1] = b[r1 * R2 + s2];
-            Dft<R1, INV>::template run<outer_zero(Z)>(tmp);
+            Dft<R1, INV>::template run<outer_zero(Z), SPLIT3>(tmp);
 #pragma unroll
             for (int s1 = 0; s1 < R1; ++s1) a[R2 * s1 + s2] = tmp[s1];
         }
@@ -427,7 +438,7 @@ constexpr int band_zero_mask(int b) {
 
 // First pass of a band-limited line: as stockham_pass with p = 1, with the elements outside the
 // band taken as zero (their registers are not read).
-template <int N, int L, int R, bool INV, int b = 0>
+template <int N, int L, int R, bool INV, bool SPLIT3, int b = 0>
 __device__ __forceinline__ void stockham_first_banded(float2 (&v)[N / L], float2* line, int t) {
     constexpr int NB = (N / L) / R;
     if constexpr (b < NB) {
@@ -435,11 +446,11 @@ __device__ __forceinline__ void stockham_first_banded(float2 (&v)[N / L], float2
         float2 a[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) a[r] = (Z >> r) & 1 ? make_float2(0.f, 0.f) : v[b + r * NB];
-        Dft<R, INV>::template run<Z>(a);
+        Dft<R, INV>::template run<Z, SPLIT3>(a);
         const int j = (t + L * b) * R;
 #pragma unroll
         for (int r = 0; r < R; ++r) line[lpad(j + r)] = a[r];
-        stockham_first_banded<N, L, R, INV, b + 1>(v, line, t);
+        stockham_first_banded<N, L, R, INV, SPLIT3, b + 1>(v, line, t);
     }
 }
 
@@ -456,7 +467,7 @@ __device__ __forceinline__ float2 cmulc_tw(float2 a, float2 w) {
 
 // One Stockham pass.  v holds the line in register layout; line is this line's LDS.
 // P_ = product of radices already done (p); LAST = this pass ends the transform.
-template <int N, int L, int R, int P_, bool INV, bool LAST, bool ALT, class TW, bool PAD2 = false>
+template <int N, int L, int R, int P_, bool INV, bool LAST, bool ALT, bool SPLIT3, class TW, bool PAD2 = false>
 __device__ __forceinline__ void stockham_pass(float2 (&v)[N / L], float2* line, int t,
                                               const TW* tw) {
     constexpr int E = N / L;
@@ -475,7 +486,7 @@ __device__ __forceinline__ void stockham_pass(float2 (&v)[N / L], float2* line, 
                 a[r] = INV ? cmulc_tw(a[r], w) : cmul_tw<ALT>(a[r], w);
             }
         }
-        Dft<R, INV>::run(a);
+        Dft<R, INV>::template run<0, SPLIT3>(a);
         if constexpr (LAST) {
 #pragma unroll
             for (int r = 0; r < R; ++r) v[b + r * NB] = a[r];
@@ -501,29 +512,29 @@ struct NoTw {
 // Full transform of one line in register layout.  sync() must order LDS writes before
 // reads and reads before the next pass's writes for every lane sharing the LDS line.
 // BANDED: the input is band limited (elements of class BAND_OUT are zero and not read).
-template <class PL, bool INV, bool BANDED = false, class TWS, class Sync>
+template <class PL, bool INV, bool BANDED = false, bool SPLIT3 = false, class TWS, class Sync>
 __device__ __forceinline__ void fft_line(float2 (&v)[PL::E], float2* line, int t, const TWS& tw,
                                          Sync sync) {
     constexpr int N = PL::N, L = PL::L;
     if constexpr (BANDED)
-        stockham_first_banded<N, L, PL::R0, INV>(v, line, t);
+        stockham_first_banded<N, L, PL::R0, INV, SPLIT3>(v, line, t);
     else
-        stockham_pass<N, L, PL::R0, 1, INV, false, false, NoTw>(v, line, t, nullptr);
+        stockham_pass<N, L, PL::R0, 1, INV, false, false, SPLIT3, NoTw>(v, line, t, nullptr);
     sync();
     line_gather<N, L>(v, line, t);
     sync();
-    stockham_pass<N, L, PL::R1, PL::R0, INV, false, TWS::alt, typename TWS::T1, true>(v, line, t, &tw.p1);
+    stockham_pass<N, L, PL::R1, PL::R0, INV, false, TWS::alt, SPLIT3, typename TWS::T1, true>(v, line, t, &tw.p1);
     sync();
     line_gather<N, L, true>(v, line, t);
     sync();
     if constexpr (PL::R3 == 1) {
-        stockham_pass<N, L, PL::R2, PL::R0 * PL::R1, INV, true, TWS::alt>(v, line, t, &tw.p2);
+        stockham_pass<N, L, PL::R2, PL::R0 * PL::R1, INV, true, TWS::alt, SPLIT3>(v, line, t, &tw.p2);
     } else {
-        stockham_pass<N, L, PL::R2, PL::R0 * PL::R1, INV, false, TWS::alt, typename TWS::T2>(v, line, t, &tw.p2);
+        stockham_pass<N, L, PL::R2, PL::R0 * PL::R1, INV, false, TWS::alt, SPLIT3, typename TWS::T2>(v, line, t, &tw.p2);
         sync();
         line_gather<N, L>(v, line, t);
         sync();
-        stockham_pass<N, L, PL::R3, PL::R0 * PL::R1 * PL::R2, INV, true, TWS::alt>(v, line, t, &tw.p3);
+        stockham_pass<N, L, PL::R3, PL::R0 * PL::R1 * PL::R2, INV, true, TWS::alt, SPLIT3>(v, line, t, &tw.p3);
     }
 }
 

@@ -246,7 +246,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
     }
     if constexpr (MODE == ROW_ADJ_SEED || MODE == ROW_ADJ) {
         // u = F_x^-1 v / res (real space)
-        fft_line<PL, true, band_reads(IO)>(v, ln, t, tws, sync);
+        fft_line<PL, true, band_reads(IO), MODE == ROW_ADJ>(v, ln, t, tws, sync);
         sync();
         const float inv = 1.0f / N;
         if constexpr (MODE == ROW_ADJ_SEED) {
@@ -257,7 +257,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
                 v[m] = make_float2(v[m].x * f, v[m].y * f);  // g = 2 w psi
             }
         } else {
-            fft_line<PL, true>(ps, ln, t, tws, sync);
+            fft_line<PL, true, false, true>(ps, ln, t, tws, sync);
             sync();
             float2* gt = a.aux_out + (size_t)wave * wave_stride + (size_t)row * N;
 #pragma unroll
@@ -495,7 +495,9 @@ __global__ __launch_bounds__(TC * PL::L) __attribute__((amdgpu_waves_per_eu(WPE)
         }
         line_gather<N, L>(v, ln, t);
         sync();
-        fft_line<PL, false>(v, ln, t, tws, sync);
+        // the forward transforms' rounding that these modes have always had (see Dft<3>)
+        constexpr bool SPLIT3 = MODE == COL_PROP || MODE == COL_PROP_DETECT || MODE == COL_PROP_CONJ || MODE == COL_FFT_DIFF;
+        fft_line<PL, false, false, SPLIT3>(v, ln, t, tws, sync);
     }
 
     if constexpr (MODE == COL_PROP || MODE == COL_PROP_DETECT || MODE == COL_PROP_CONJ) {
