@@ -69,126 +69,15 @@ void* noalloc_scratch(int device) {
     return p;
 }
 
-// Pinned staging memory for copies from and to pageable host memory: at most kStages buffers of
-// kStageBytes in the process, made on first use, shared by all engines and threads and given back
-// when the last engine is destroyed.  A copy takes one buffer for itself until its transfers have
-// finished; while none is free (more threads copying than buffers) a copy goes without.
-constexpr int kStages = 4;
-constexpr size_t kStageBytes = size_t(4) << 20, kStageChunk = size_t(1) << 20;
-constexpr int kStageChunks = (int)(kStageBytes / kStageChunk);
-
-struct Stage {
-    int device = -1;                    // the events' device
-    unsigned char* p = nullptr;
-    hipEvent_t done[kStageChunks] = {}; // the last transfer of each chunk
-    bool used[kStageChunks] = {};
-    bool taken = false;
-};
-std::mutex g_stage_mu;
-Stage g_stages[kStages];
-int g_engines = 0;
-
-void release_stage(Stage& s) {
-    for (auto& ev : s.done)
-        if (ev) (void)hipEventDestroy(ev);
-    if (s.p) (void)hipHostFree(s.p);
-    s = Stage();
-}
-
-// a free buffer whose events belong to `device`; NULL while there is none
-Stage* take_stage(int device) {
-    std::lock_guard<std::mutex> lk(g_stage_mu);
-    Stage* empty = nullptr;
-    for (Stage& s : g_stages) {
-        if (s.taken) continue;
-        if (s.p && s.device == device) {
-            s.taken = true;
-            return &s;
-        }
-        if (!s.p) empty = &s;
-    }
-    if (!empty) return nullptr;
-    bool ok = hipHostMalloc((void**)&empty->p, kStageBytes, hipHostMallocDefault) == hipSuccess;
-    for (auto& ev : empty->done) ok = ok && hipEventCreateWithFlags(&ev, hipEventDisableTiming) == hipSuccess;
-    if (!ok) {
-        (void)hipGetLastError();  // the copy goes without
-        release_stage(*empty);
-        return nullptr;
-    }
-    empty->device = device;
-    empty->taken = true;
-    return empty;
-}
-
-// One copy's hold on a staging buffer; its destructor waits for the buffer's transfers.
-struct StageHold {
-    Stage* s;
-    explicit StageHold(int device) : s(device >= 0 ? take_stage(device) : nullptr) {}  // -1: no buffer
-    ~StageHold() {
-        if (!s) return;
-        for (int i = 0; i < kStageChunks; ++i) {
-            if (s->used[i]) (void)hipEventSynchronize(s->done[i]);
-            s->used[i] = false;
-        }
-        std::lock_guard<std::mutex> lk(g_stage_mu);
-        s->taken = false;
-    }
-    StageHold(const StageHold&) = delete;
-    StageHold& operator=(const StageHold&) = delete;
-};
+// staging memory of the host copies, one pool for the process
+StagePool<HipStaging> g_stages;
 
 void download(mse_engine* e, void* dst, const void* src, size_t bytes) {
-    StageHold hold(e->device);
-    Stage* s = hold.s;
-    if (!s) {
-        HIPX(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, e->stream));
-        HIPX(hipStreamSynchronize(e->stream));
-        return;
-    }
-    if (bytes <= kStageChunk) {
-        HIPX(hipMemcpyAsync(s->p, src, bytes, hipMemcpyDeviceToHost, e->stream));
-        HIPX(hipStreamSynchronize(e->stream));
-        std::memcpy(dst, s->p, bytes);
-        return;
-    }
-    // chunk i lands in part i % kStageChunks while the chunks before it are copied out
-    const size_t n = (bytes + kStageChunk - 1) / kStageChunk;
-    for (size_t i = 0; i < n + kStageChunks - 1; ++i) {
-        if (i >= (size_t)kStageChunks - 1) {
-            const size_t j = i - (kStageChunks - 1), at = j * kStageChunk;
-            const int part = (int)(j % kStageChunks);
-            HIPX(hipEventSynchronize(s->done[part]));
-            s->used[part] = false;
-            std::memcpy((unsigned char*)dst + at, s->p + part * kStageChunk, std::min(kStageChunk, bytes - at));
-        }
-        if (i < n) {
-            const size_t at = i * kStageChunk;
-            const int part = (int)(i % kStageChunks);
-            HIPX(hipMemcpyAsync(s->p + part * kStageChunk, (const unsigned char*)src + at, std::min(kStageChunk, bytes - at),
-                                hipMemcpyDeviceToHost, e->stream));
-            HIPX(hipEventRecord(s->done[part], e->stream));
-            s->used[part] = true;
-        }
-    }
+    staged_download(g_stages, e->lane, dst, src, bytes);
 }
 
 void upload(mse_engine* e, void* dst, const void* src, size_t bytes) {
-    StageHold hold(e->device);
-    Stage* s = hold.s;
-    if (!s) {
-        HIPX(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, e->stream));
-        HIPX(hipStreamSynchronize(e->stream));
-        return;
-    }
-    for (size_t at = 0, i = 0; at < bytes; at += kStageChunk, ++i) {
-        const int part = (int)(i % kStageChunks);
-        const size_t len = std::min(kStageChunk, bytes - at);
-        if (s->used[part]) HIPX(hipEventSynchronize(s->done[part]));
-        std::memcpy(s->p + part * kStageChunk, (const unsigned char*)src + at, len);
-        HIPX(hipMemcpyAsync((unsigned char*)dst + at, s->p + part * kStageChunk, len, hipMemcpyHostToDevice, e->stream));
-        HIPX(hipEventRecord(s->done[part], e->stream));
-        s->used[part] = true;
-    }
+    staged_upload(g_stages, e->lane, dst, src, bytes);
 }
 
 struct DeviceGuard {
@@ -593,9 +482,10 @@ int mse_create(int device_ordinal, mse_engine** out) {
             delete e;
             throw Error(MSE_ERR_HIP, std::string("hipStreamCreate: ") + hipGetErrorString(st));
         }
+        e->lane.device = e->device;
+        e->lane.stream = e->stream;
+        g_stages.engine_made();
         *out = e;
-        std::lock_guard<std::mutex> lk(g_stage_mu);
-        ++g_engines;
     });
 }
 
@@ -613,10 +503,7 @@ int mse_destroy(mse_engine* e) {
         hipStream_t s = e->stream;
         delete e;
         (void)hipStreamDestroy(s);
-        std::lock_guard<std::mutex> lk(g_stage_mu);
-        if (--g_engines == 0)
-            for (Stage& st : g_stages)
-                if (!st.taken) release_stage(st);
+        g_stages.engine_gone();
     });
     return rc;
 }
@@ -891,7 +778,7 @@ int mse_sort_atoms(mse_engine* e, int cfg, const double* x, const double* y, con
         // atoms in and bins out through one staging buffer, one transfer each way
         const size_t in_bytes = (size_t)n * (3 * sizeof(double) + sizeof(int));
         const size_t out_ints = 2 * (size_t)n + (size_t)nkeys + 1;
-        StageHold hold(std::max(in_bytes, out_ints * sizeof(int)) <= kStageBytes ? e->device : -1);
+        StageHold<HipStaging> hold(g_stages, e->lane, std::max(in_bytes, out_ints * sizeof(int)) <= kStageBytes);
         if (n > 0) {
             if (hold.s) {
                 unsigned char* h = hold.s->p;
@@ -900,7 +787,7 @@ int mse_sort_atoms(mse_engine* e, int cfg, const double* x, const double* y, con
                 std::memcpy(h + d, y, d);
                 std::memcpy(h + 2 * d, z, d);
                 std::memcpy(h + 3 * d, Z, (size_t)n * sizeof(int));
-                HIPX(hipMemcpyAsync(dx, h, in_bytes, hipMemcpyHostToDevice, e->stream));
+                hold.to_device(dx, 0, in_bytes);
             } else {
                 HIPX(hipMemcpyAsync(dx, x, n * sizeof(double), hipMemcpyHostToDevice, e->stream));
                 HIPX(hipMemcpyAsync(dy, y, n * sizeof(double), hipMemcpyHostToDevice, e->stream));
@@ -967,12 +854,10 @@ int mse_sort_atoms(mse_engine* e, int cfg, const double* x, const double* y, con
             // [bin starts][block ids][slice ids], as far as asked for
             int* h = reinterpret_cast<int*>(hold.s->p);
             const size_t first = block_start ? 0 : (size_t)nkeys, starts = (size_t)nkeys + 1 - first;
-            HIPX(hipMemcpyAsync(h, c.block_start.p + first, starts * sizeof(int), hipMemcpyDeviceToHost, e->stream));
-            if (block_ids && n > 0)
-                HIPX(hipMemcpyAsync(h + starts, e->tmp_bid.p, n * sizeof(int), hipMemcpyDeviceToHost, e->stream));
-            if (z_ids && n > 0)
-                HIPX(hipMemcpyAsync(h + starts + n, e->tmp_zid.p, n * sizeof(int), hipMemcpyDeviceToHost, e->stream));
-            HIPX(hipStreamSynchronize(e->stream));
+            hold.to_host(0, c.block_start.p + first, starts * sizeof(int));
+            if (block_ids && n > 0) hold.to_host(starts * sizeof(int), e->tmp_bid.p, n * sizeof(int));
+            if (z_ids && n > 0) hold.to_host((starts + n) * sizeof(int), e->tmp_zid.p, n * sizeof(int));
+            hold.sync();
             nr = h[starts - 1];
             if (block_start) std::memcpy(block_start, h, starts * sizeof(int));
             if (block_ids && n > 0) std::memcpy(block_ids, h + starts, n * sizeof(int));

@@ -21,6 +21,7 @@
 #include "../../include/cltem_amd.h"
 #include "fft_wave.hpp"
 #include "slice_kernels.hpp"
+#include "staging.hpp"
 
 
 
@@ -48,6 +49,36 @@ struct Error : std::runtime_error {
     do {                                      \
         if (!(cond)) throw Error(code, msg);  \
     } while (0)
+
+// HIP's calls for the staging memory of host copies (staging.hpp)
+struct HipStaging {
+    using Stream = hipStream_t;
+    using Event = hipEvent_t;
+    static bool pin(unsigned char** p, size_t bytes) {
+        if (hipHostMalloc((void**)p, bytes, hipHostMallocDefault) == hipSuccess) return true;
+        (void)hipGetLastError();
+        *p = nullptr;
+        return false;
+    }
+    static void unpin(unsigned char* p) { (void)hipHostFree(p); }
+    static bool make_event(hipEvent_t* ev) {
+        if (hipEventCreateWithFlags(ev, hipEventDisableTiming) == hipSuccess) return true;
+        (void)hipGetLastError();
+        *ev = nullptr;
+        return false;
+    }
+    static void drop_event(hipEvent_t ev) { (void)hipEventDestroy(ev); }
+    static void to_host(void* dst, const void* src, size_t bytes, hipStream_t st) {
+        HIPX(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st));
+    }
+    static void to_device(void* dst, const void* src, size_t bytes, hipStream_t st) {
+        HIPX(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st));
+    }
+    static void record(hipEvent_t ev, hipStream_t st) { HIPX(hipEventRecord(ev, st)); }
+    static void wait(hipEvent_t ev) { HIPX(hipEventSynchronize(ev)); }
+    static void sync(hipStream_t st) { HIPX(hipStreamSynchronize(st)); }
+    static bool try_sync(hipStream_t st) { return hipStreamSynchronize(st) == hipSuccess; }
+};
 
 template <typename T>
 struct DevBuf {
@@ -115,6 +146,7 @@ using namespace mse_rt;
 struct mse_engine {
     int device = 0;
     hipStream_t stream = nullptr;
+    mse_rt::StageLane<mse_rt::HipStaging> lane;  // the stream's host copies
     bool have_geom = false;
     mse_geometry g{};
     int res = 0;
