@@ -482,7 +482,6 @@ int mse_create(int device_ordinal, mse_engine** out) {
             delete e;
             throw Error(MSE_ERR_HIP, std::string("hipStreamCreate: ") + hipGetErrorString(st));
         }
-        e->lane.device = e->device;
         e->lane.stream = e->stream;
         g_stages.engine_made();
         *out = e;

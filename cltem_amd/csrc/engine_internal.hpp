@@ -54,8 +54,9 @@ struct Error : std::runtime_error {
 struct HipStaging {
     using Stream = hipStream_t;
     using Event = hipEvent_t;
+    // for the copies of every device
     static bool pin(unsigned char** p, size_t bytes) {
-        if (hipHostMalloc((void**)p, bytes, hipHostMallocDefault) == hipSuccess) return true;
+        if (hipHostMalloc((void**)p, bytes, hipHostMallocPortable) == hipSuccess) return true;
         (void)hipGetLastError();
         *p = nullptr;
         return false;

@@ -12,44 +12,49 @@ constexpr int kStages = 4;
 constexpr size_t kStageBytes = size_t(4) << 20, kStageChunk = size_t(1) << 20;
 constexpr int kStageChunks = (int)(kStageBytes / kStageChunk);
 
-// The stream whose copies are staged, and its device.
+// The stream whose copies are staged: an engine's.  Its events belong to its device, the buffers to
+// none, so that every device's engines share them.
 template <class RT>
 struct StageLane {
-    int device = 0;
     typename RT::Stream stream{};
+    typename RT::Event done[kStageChunks] = {};  // the last transfer of each chunk of the buffer in hand
+    StageLane() = default;
+    StageLane(const StageLane&) = delete;
+    StageLane& operator=(const StageLane&) = delete;
+    ~StageLane() {
+        for (auto ev : done)
+            if (ev) RT::drop_event(ev);
+    }
+    // the events, made on first use (on the current device)
+    bool ready() {
+        for (auto& ev : done)
+            if (!ev && !RT::make_event(&ev)) return false;
+        return true;
+    }
 };
 
 // At most kStages buffers of kStageBytes, made on first use, shared by all engines and threads of
-// the process and given back when the last engine is destroyed.
+// the process, whatever their devices, and given back when the last engine is destroyed.
 template <class RT>
 struct StagePool {
     struct Stage {
-        int device = -1;                           // the events' device
         unsigned char* p = nullptr;
-        typename RT::Event done[kStageChunks] = {};  // the last transfer of each chunk
         bool taken = false;
     };
 
-    // a free buffer whose events belong to `device`; NULL while there is none
-    Stage* take(int device) {
+    // a free buffer; NULL while there is none
+    Stage* take() {
         std::lock_guard<std::mutex> lk(mu);
         Stage* empty = nullptr;
         for (Stage& s : stages) {
             if (s.taken) continue;
-            if (s.p && s.device == device) {
+            if (s.p) {
                 s.taken = true;
                 return &s;
             }
-            if (!s.p) empty = &s;
+            empty = &s;
         }
-        if (!empty) return nullptr;
-        bool ok = RT::pin(&empty->p, kStageBytes);
-        for (auto& ev : empty->done) ok = ok && RT::make_event(&ev);
-        if (!ok) {  // the copy goes without
-            release(*empty);
-            return nullptr;
-        }
-        empty->device = device;
+        if (!empty || !RT::pin(&empty->p, kStageBytes)) return nullptr;  // the copy goes without
         empty->taken = true;
         return empty;
     }
@@ -70,8 +75,6 @@ struct StagePool {
 
 private:
     static void release(Stage& s) {
-        for (auto& ev : s.done)
-            if (ev) RT::drop_event(ev);
         if (s.p) RT::unpin(s.p);
         s = Stage();
     }
@@ -92,7 +95,7 @@ struct StageHold {
     bool in_flight = false;  // a transfer may be using the buffer
 
     StageHold(StagePool<RT>& pool, StageLane<RT>& lane, bool wanted = true)
-        : pool(pool), lane(lane), s(wanted ? pool.take(lane.device) : nullptr) {}
+        : pool(pool), lane(lane), s(wanted && lane.ready() ? pool.take() : nullptr) {}
     ~StageHold() {
         if (s && (!in_flight || RT::try_sync(lane.stream))) pool.give_back(s);
     }
@@ -107,8 +110,8 @@ struct StageHold {
         in_flight = true;
         RT::to_host(s->p + at, src, bytes, lane.stream);
     }
-    void record(int part) { RT::record(s->done[part], lane.stream); }
-    void wait(int part) { RT::wait(s->done[part]); }
+    void record(int part) { RT::record(lane.done[part], lane.stream); }
+    void wait(int part) { RT::wait(lane.done[part]); }
     void sync() {
         RT::sync(lane.stream);
         in_flight = false;

@@ -102,6 +102,30 @@ int main() {
 }
 """
 
+# engines on more devices than the pool has buffers, in turn: every one's copies are staged, with
+# events of its own device
+DEVICES = r"""
+int main() {
+    StagePool<Fake> pool;
+    constexpr int devices = 2 * kStages + 1;
+    for (int round = 0; round < 3; ++round)
+        for (int d = 0; d < devices; ++d) {
+            Fake::device = d;
+            static FakeStream st[devices];
+            static StageLane<Fake> lane[devices];
+            st[d].device = d;
+            lane[d].stream = &st[d];
+            const Bytes a = pattern(2 * kStageChunk + 3, d + round);
+            Bytes dev(a.size()), back(a.size());
+            staged_upload(pool, lane[d], dev.data(), a.data(), a.size());
+            staged_download(pool, lane[d], back.data(), dev.data(), a.size());
+            CHECK(back == a);
+            CHECK(Fake::direct == 0);
+        }
+    CHECK(Fake::pinned <= kStages);
+}
+"""
+
 
 def run(tmp_path, body):
     src = tmp_path / "t.cpp"
@@ -112,6 +136,6 @@ def run(tmp_path, body):
     assert r.returncode == 0, r.stdout + r.stderr
 
 
-@pytest.mark.parametrize("body", [COPIES, IN_FLIGHT], ids=["copies", "in_flight"])
+@pytest.mark.parametrize("body", [COPIES, IN_FLIGHT, DEVICES], ids=["copies", "in_flight", "devices"])
 def test_staging(tmp_path, body):
     run(tmp_path, body)
