@@ -378,6 +378,8 @@ class Engine:
         _check(self.lib.mse_set_potential_tables(self.h, (1 if lds else 2) if enable else 0))
 
     def set_kernel_variant(self, kernel: int, variant: int):
+        """Forces a variant of the row (kernel 0) or column pass (1) for every number of waves; -1: the
+        choice by grid size and number of waves again."""
         _check(self.lib.mse_set_kernel_variant(self.h, kernel, variant))
 
     def autotune(self, config: int = 0, n_waves: int = 64, reps: int = 5):

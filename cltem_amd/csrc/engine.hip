@@ -2297,8 +2297,8 @@ int mse_set_kernel_variant(mse_engine* e, int kernel, int variant) {
     return run_guarded("mse_set_kernel_variant", e, [&]() {
         REQUIRE(e, MSE_ERR_ARG, "engine is NULL");
         REQUIRE(kernel == 0 || kernel == 1, MSE_ERR_ARG, "kernel must be 0 (row) or 1 (column)");
-        REQUIRE(variant >= 0 && variant < (kernel == 0 ? kRowVariants : kColVariants), MSE_ERR_ARG,
-                "variant out of range");
+        REQUIRE(variant >= -1 && variant < (kernel == 0 ? kRowVariants : kColVariants), MSE_ERR_ARG,
+                "variant out of range");  // -1: the rule
         if (kernel == 0)
             e->row_var = variant;
         else

@@ -336,8 +336,10 @@ int mse_potential_table(int form, int full3d, const double* params, int n_params
  *      mse_autotune times every variant of both sweeps on n_waves waves of `config`
  *      (reps launches each; times in microseconds per launch) and selects the fastest: sweeps
  *      over that number of waves use it from then on, sweeps over any other number of waves keep
- *      the variants chosen by grid size and wave count.  It leaves the waves' contents undefined.  mse_set_kernel_variant
- *      forces a variant for every number of waves. ---- */
+ *      the variants chosen by grid size and wave count.  It leaves the waves' contents undefined.
+ *      mse_set_kernel_variant forces a variant for every number of waves; variant -1 takes that
+ *      back, the grid size and the number of waves decide again.  Either forgets what
+ *      mse_autotune found. ---- */
 int mse_set_kernel_variant(mse_engine* e, int kernel, int variant);
 int mse_autotune(mse_engine* e, int config, int n_waves, int reps, double* row_us, double* col_us,
                  int* best_row, int* best_col);

@@ -25,3 +25,13 @@ def engine():
     e = cltem_amd.Engine(0)
     yield e
     e.close()
+
+
+@pytest.fixture(autouse=True)
+def kernels_by_rule(request):
+    """Each test finds the session's engine with no kernel variant forced or tuned by another."""
+    yield
+    if "engine" in request.fixturenames:
+        e = request.getfixturevalue("engine")
+        for kernel in (0, 1):
+            e.set_kernel_variant(kernel, -1)
