@@ -21,6 +21,7 @@
 #include "../../include/cltem_amd.h"
 #include "atom_kernels.hpp"
 #include "engine_internal.hpp"
+#include "frame_plan.hpp"
 #include "potential_table.hpp"
 
 namespace mse_geom {
@@ -1980,29 +1981,31 @@ int mse_stem_batch_frames(mse_engine* e, int cfg, const double* pos_xy, const do
         e->partials.ensure((size_t)batch * n_det * (e->res / 8));
         e->det_out.ensure((size_t)n_probes * n_det);
         e->frame_xy.ensure(2 * (size_t)batch);
-        // Transmission functions of several slices of every frame at once, up to half a GiB (and
-        // 65535 planes, the grid's limit): one slice's planes are too little work for the
-        // potential kernel and three band-limit launches.  12 frames of 256^2, 15 slices: 1.74
-        // -> 0.86 ms per 24 probes.
-        const size_t plane_bytes = (size_t)batch * e->N * sizeof(float2);
-        const int most = (int)std::min<size_t>(kFrameBytes / plane_bytes, 65535 / (size_t)batch);
-        const int groups = (ns + std::max(1, most) - 1) / std::max(1, most);
-        const int cs = (ns + groups - 1) / groups;
-        e->frame_trans.ensure((size_t)batch * cs * e->N);
-        // the row pass finds wave w's transmission functions at planes w cs.. of frame_trans: a
-        // table of one "configuration" per wave, each cs slices deep
-        e->frame_ptrs.ensure(batch);
+        e->frame_ptrs.ensure(2 * (size_t)batch);
         e->frame_ns.ensure(batch);
         e->frame_wcfg.ensure(batch);
         if (!e->h_focus.empty()) e->probe_df.ensure(std::max<size_t>(batch, e->n_waves));
+        // Transmission functions of several slices of every frame at once, up to half a GiB (and
+        // 65535 planes, the grid's limit): one slice's planes are too little work for the
+        // potential kernel and three band-limit launches.  12 frames of 256^2, 15 slices: 1.74
+        // -> 1.06 ms per 24 probes.
+        const size_t plane_bytes = (size_t)batch * e->N * sizeof(float2);
+        const int most = (int)std::min<size_t>(kFrameBytes / plane_bytes, 65535 / (size_t)batch);
+        const int cs = frame_slices(ns, most);
+        e->frame_trans.ensure((size_t)batch * cs * e->N);
+        // the row pass finds wave w's transmission functions at planes w cs.. of frame_trans: a
+        // table of one "configuration" per wave, each cs slices deep; a second table for the last
+        // group, whose frames lie as many planes apart as it has slices
+        const int tail = (ns - 1) % cs + 1;
         {
-            std::vector<const float2*> ptrs(batch);
+            std::vector<const float2*> ptrs(2 * (size_t)batch);
             std::vector<int> depth(batch, cs), ids(batch);
             for (int w = 0; w < batch; ++w) {
                 ptrs[w] = e->frame_trans.p + (size_t)w * cs * e->N;
+                ptrs[batch + w] = e->frame_trans.p + (size_t)w * tail * e->N;
                 ids[w] = w;
             }
-            HIPX(hipMemcpyAsync(e->frame_ptrs.p, ptrs.data(), batch * sizeof(const float2*), hipMemcpyHostToDevice,
+            HIPX(hipMemcpyAsync(e->frame_ptrs.p, ptrs.data(), ptrs.size() * sizeof(const float2*), hipMemcpyHostToDevice,
                                 e->stream));
             HIPX(hipMemcpyAsync(e->frame_ns.p, depth.data(), batch * sizeof(int), hipMemcpyHostToDevice, e->stream));
             HIPX(hipMemcpyAsync(e->frame_wcfg.p, ids.data(), batch * sizeof(int), hipMemcpyHostToDevice, e->stream));
@@ -2012,9 +2015,7 @@ int mse_stem_batch_frames(mse_engine* e, int cfg, const double* pos_xy, const do
         }
         mse::PotArgs pa = pot_args(e, c);
         pa.frame_xy = e->frame_xy.p;
-        pa.frame_slices = cs;
         mse::RowArgs ra = base_row_args(e);
-        ra.cfg_trans = e->frame_ptrs.p;
         ra.cfg_nslices = e->frame_ns.p;
         ra.wave_cfg = e->frame_wcfg.p;
         ra.mix_sets = 0;
@@ -2048,10 +2049,11 @@ int mse_stem_batch_frames(mse_engine* e, int cfg, const double* pos_xy, const do
             ra.read_k = probes_into_waves(e, nb, probe, true);
             for (int s = 0; s < ns; ++s) {
                 if (s % cs == 0) {
-                    // (the last group may reach past the specimen, by less than a slice per
-                    // group: its planes beyond are not read)
-                    potential_planes(e, c, g, pa, e->frame_trans.p, nb * cs, s);
-                    band_limit_planes(e, e->frame_trans.p, nb * cs);
+                    const int here = frame_group(ns, cs, s);
+                    pa.frame_slices = here;
+                    ra.cfg_trans = e->frame_ptrs.p + (here == cs ? 0 : batch);
+                    potential_planes(e, c, g, pa, e->frame_trans.p, nb * here, s);
+                    band_limit_planes(e, e->frame_trans.p, nb * here);
                 }
                 ra.slice = s % cs;
                 slice_band(e, s == 0, ra, ca);
