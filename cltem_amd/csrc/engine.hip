@@ -1991,8 +1991,8 @@ int mse_stem_batch_frames(mse_engine* e, int cfg, const double* pos_xy, const do
         // -> 1.06 ms per 24 probes.
         const size_t plane_bytes = (size_t)batch * e->N * sizeof(float2);
         const int most = (int)std::min<size_t>(kFrameBytes / plane_bytes, 65535 / (size_t)batch);
-        const int cs = frame_slices(ns, most);
-        e->frame_trans.ensure((size_t)batch * cs * e->N);
+        const int cs = frame_slices_that_fit(ns, most, [&](int slices) { return e->frame_trans.try_ensure((size_t)batch * slices * e->N); });
+        if (cs == 0) throw Error(MSE_ERR_HIP, "hipMalloc: no memory for one slice's transmission functions of the batch's frames");
         // the row pass finds wave w's transmission functions at planes w cs.. of frame_trans: a
         // table of one "configuration" per wave, each cs slices deep; a second table for the last
         // group, whose frames lie as many planes apart as it has slices

@@ -100,18 +100,27 @@ struct DevBuf {
         n = 0;
     }
     void ensure(size_t count) {
-        if (count <= n && p) return;
+        const hipError_t rc = allocate(count);
+        if (rc != hipSuccess) throw Error(MSE_ERR_HIP, std::string("hipMalloc: ") + hipGetErrorString(rc));
+    }
+    // false: no memory for it; the buffer is then empty
+    bool try_ensure(size_t count) { return allocate(count) == hipSuccess; }
+
+private:
+    hipError_t allocate(size_t count) {
+        if (count <= n && p) return hipSuccess;
         release();
-        if (count == 0) return;
+        if (count == 0) return hipSuccess;
         const hipError_t rc = hipMalloc((void**)&p, count * sizeof(T));
         if (rc != hipSuccess) {
             // a failed allocation also leaves its code as the runtime's last error, which the
-            // launch check of the next kernel would report: clear it, the error is thrown here
+            // launch check of the next kernel would report: clear it, the caller has it
             (void)hipGetLastError();
             p = nullptr;
-            throw Error(MSE_ERR_HIP, std::string("hipMalloc: ") + hipGetErrorString(rc));
+            return rc;
         }
         n = count;
+        return hipSuccess;
     }
 };
 

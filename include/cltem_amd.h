@@ -299,7 +299,7 @@ int mse_stem_batch(mse_engine* e, int config, const double* pos_xy, int n_probes
  * functions need not be built), band limited, and each multiplies its own wave.  The engine
  * geometry (grid, field size, optics) is the moving-frame geometry.  Device memory:
  * one transmission plane per wave of the batch and slice, for as many slices as 512 MiB hold
- * (one at least).  Eager launches only. */
+ * (one at least; fewer where the device has no room for them).  Eager launches only. */
 int mse_stem_batch_frames(mse_engine* e, int config, const double* pos_xy, const double* frame_xy,
                           int n_probes, int batch, const mse_probe* probe, const mse_detector* dets,
                           int n_det, int sqrt2, double* accum);

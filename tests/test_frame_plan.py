@@ -37,8 +37,32 @@ int main() {
 }
 """
 
+# memory that runs out: fewer slices at a time, down to one; never more than there is room for, and
+# no smaller groups than halving finds
+NO_MEMORY = r"""
+int main() {
+    for (int ns = 1; ns <= 200; ++ns)
+        for (int most = 0; most <= 70; ++most)
+            for (int room = 0; room <= 70; ++room) {
+                int tried = 0, last = 1 << 30;
+                const int cs = frame_slices_that_fit(ns, most, [&](int slices) {
+                    CHECK(slices >= 1 && slices < last);
+                    last = slices;
+                    ++tried;
+                    return slices <= room;
+                });
+                if (room == 0) {
+                    CHECK(cs == 0 && last == 1);
+                } else {
+                    CHECK(cs >= 1 && cs <= room && cs == last);
+                    if (frame_slices(ns, most) <= room) CHECK(tried == 1);
+                }
+            }
+}
+"""
 
-@pytest.mark.parametrize("body", [GROUPS], ids=["groups"])
+
+@pytest.mark.parametrize("body", [GROUPS, NO_MEMORY], ids=["groups", "no_memory"])
 def test_frame_plan(tmp_path, body):
     src = tmp_path / "t.cpp"
     src.write_text(COMMON + body)
