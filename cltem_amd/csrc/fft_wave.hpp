@@ -22,12 +22,16 @@ namespace mse {
 
 __device__ __forceinline__ float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
 __device__ __forceinline__ float2 csub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }
+// Of the two products of each part one is rounded and the other enters the fused multiply-add.  Which
+// one is written out in these and in all products of the sweeps: the compiler's own choice depends on
+// the expressions around it, on negated operands, say, or on where a kernel's loads stand.
+// cmul(a, b) and cmul(b, a) round the imaginary part differently.
 __device__ __forceinline__ float2 cmul(float2 a, float2 b) {
-    return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+    return make_float2(fmaf(a.x, b.x, -(a.y * b.y)), fmaf(a.x, b.y, a.y * b.x));
 }
 // a * conj(b)
 __device__ __forceinline__ float2 cmulc(float2 a, float2 b) {
-    return make_float2(a.x * b.x + a.y * b.y, a.y * b.x - a.x * b.y);
+    return make_float2(fmaf(a.x, b.x, a.y * b.y), fmaf(a.y, b.x, -(a.x * b.y)));
 }
 __device__ __forceinline__ float2 cscale(float2 a, float s) { return make_float2(a.x * s, a.y * s); }
 
@@ -99,12 +103,10 @@ constexpr double ct_sin2pi(int J, int R) {
     return ct_sin_series(a);
 }
 
-// multiply by W_R^J = exp(-+ 2 pi i J / R) (forward: minus, inverse: plus).  Of the two products
-// of each component one is rounded and the other enters the fused multiply-add.  Which one is
-// written out (XR: the product with a.x is rounded in the real part, XI: in the imaginary part):
-// the compiler's own choice depends on the expressions around it (on negated operands, say), and
-// written out a transform with zero inputs left out rounds exactly as the full one, and every
-// kernel's transform as every other's.
+// multiply by W_R^J = exp(-+ 2 pi i J / R) (forward: minus, inverse: plus).  XR: the product with
+// a.x is the rounded one in the real part (see cmul), XI: in the imaginary part.  Written out, a
+// transform with zero inputs left out rounds exactly as the full one, and every kernel's transform as
+// every other's of the same SPLIT3 (Dft<3>) and ALT (cmul_tw).
 template <int R, int J, bool INV, bool XR, bool XI>
 __device__ __forceinline__ float2 rot(float2 a) {
     constexpr int j = ((J % R) + R) % R;
@@ -182,8 +184,7 @@ __device__ __forceinline__ float2 sub_split(float2 t, float s, float2 d) {
     return make_float2(t.x - p.x, t.y - p.y);
 }
 
-// Which products enter a fused multiply-add is written out, as in rot: left to the compiler, it
-// depended on where the kernel's loads stood.  Both outputs t2 +- i s d take theirs fused; SPLIT3:
+// Both outputs t2 +- i s d take theirs fused; SPLIT3:
 // the second one's is rounded, the rounding that the inverse transforms of the adjoint's row pass
 // and the forward ones of most of k_col's modes have always had.
 template <bool INV>
@@ -195,7 +196,7 @@ struct Dft<3, INV> {
         constexpr float s = INV ? s3 : -s3;
         const float2 a0 = z0 ? make_float2(0.f, 0.f) : a[0];
         float2 t1 = cadd_z<z1, z2>(a[1], a[2]);
-        float2 t2 = make_float2(a0.x - 0.5f * t1.x, a0.y - 0.5f * t1.y);
+        float2 t2 = make_float2(fmaf(-0.5f, t1.x, a0.x), fmaf(-0.5f, t1.y, a0.y));
         float2 d = csub_z<z1, z2>(a[1], a[2]);
         // y1 = t2 + i s d, y2 = t2 - i s d
         a[0] = cadd_z<z0, z1 && z2>(a0, t1);
@@ -454,9 +455,8 @@ __device__ __forceinline__ void stockham_first_banded(float2 (&v)[N / L], float2
     }
 }
 
-// The twiddle products with the rounded product of each part written out (as in rot), so that
-// transforms round alike wherever their twiddles come from.  ALT: the other choice in the forward
-// imaginary part, the rounding that the 768^2 band limit of transmission functions has.
+// The twiddle products: as cmul and cmulc, wherever the twiddles come from.  ALT: the other choice in
+// the forward imaginary part, the rounding that the 768^2 band limit of transmission functions has.
 template <bool ALT>
 __device__ __forceinline__ float2 cmul_tw(float2 a, float2 w) {
     return make_float2(fmaf(a.x, w.x, -(a.y * w.y)), ALT ? fmaf(a.y, w.x, a.x * w.y) : fmaf(a.x, w.y, a.y * w.x));

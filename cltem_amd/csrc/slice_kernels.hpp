@@ -302,7 +302,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
     if constexpr (MODE == ROW_IFFT_T_FFT) {
         if (has_t) {
 #pragma unroll
-            for (int m = 0; m < E; ++m) v[m] = cmul(v[m], tr[m]);
+            for (int m = 0; m < E; ++m) v[m] = cmul(tr[m], v[m]);
         }
     }
     if constexpr (MODE != ROW_IFFT) {
@@ -421,12 +421,10 @@ __device__ __forceinline__ double wave_sum(double v) {
 // doubles as its FFT exchange buffer.  BAND: the propagation's mask cuts the ky outside the
 // band (a.band_k set), whose outputs are not formed and not transformed back.
 // --------------------------------------------------------------------------------------
-// v px py, the product of the propagator's factors first, as one propagation multiplies (which
-// product of each part is rounded is written out, as in rot: all kernels propagate alike)
-__device__ __forceinline__ float2 prop_mul(float2 v, float2 px, float2 py) {
-    const float2 f = make_float2(fmaf(px.x, py.x, -(px.y * py.y)), fmaf(px.y, py.x, px.x * py.y));
-    return make_float2(fmaf(v.x, f.x, -(v.y * f.y)), fmaf(v.x, f.y, v.y * f.x));
-}
+// v px py, the product of the propagator's factors first, as one propagation multiplies: the
+// persistent and the lean kernels' rounding.  (k_col's propagation takes cmul(px, py) and, at 384^2 and
+// 768^2, Dft<3>'s SPLIT3: it rounds otherwise.)
+__device__ __forceinline__ float2 prop_mul(float2 v, float2 px, float2 py) { return cmul(v, cmul(py, px)); }
 // first column of tile j of a launch
 template <int TC>
 __device__ __forceinline__ int tile_column(const ColArgs& a, int j) {
@@ -517,9 +515,8 @@ __global__ __launch_bounds__(TC * PL::L) __attribute__((amdgpu_waves_per_eu(WPE)
             }
             const int y = t + L * m;
             const bool keep = xs <= a.lim[y];
-            float2 f = cmul(pxv, pyt[y]);
-            if constexpr (MODE == COL_PROP_CONJ) f.y = -f.y;
-            v[m] = keep ? cmul(v[m], f) : make_float2(0.f, 0.f);
+            const float2 f = cmul(pxv, pyt[y]);
+            v[m] = !keep ? make_float2(0.f, 0.f) : MODE == COL_PROP_CONJ ? cmulc(v[m], f) : cmul(v[m], f);
         }
     } else if constexpr (MODE == COL_FFT_DETECT || MODE == COL_FFT_DIFF) {
 #pragma unroll
@@ -546,7 +543,7 @@ __global__ __launch_bounds__(TC * PL::L) __attribute__((amdgpu_waves_per_eu(WPE)
                 if (BAND && band_class<N, L>(m) == BAND_OUT) continue;  // nothing there
                 const int ys = (t + L * m + N / 2) % N;
                 if ((bits[ys >> 5] >> (ys & 31)) & 1u) {
-                    const float i2 = v[m].x * v[m].x + v[m].y * v[m].y;
+                    const float i2 = fmaf(v[m].x, v[m].x, v[m].y * v[m].y);
                     acc += (double)i2;
                 }
             }
@@ -945,7 +942,7 @@ __global__ __launch_bounds__(256) void k_row_step_pipe(float2* __restrict__ data
             sync();
             if (!vacuum) {
 #pragma unroll
-                for (int m = 0; m < E; ++m) v[m] = cmul(v[m], tr[m]);
+                for (int m = 0; m < E; ++m) v[m] = cmul(tr[m], v[m]);
             }
             fft_line<PL, false>(v, ln, t, tws, sync);
         } else {
