@@ -876,9 +876,10 @@ int mse_sort_atoms(mse_engine* e, int cfg, const double* x, const double* y, con
         c.n_in_range = nr;
         if (n_in_range) *n_in_range = c.n_in_range;
         c.n_input = n;
-        c.has_Z.assign((size_t)std::max(e->max_Z, 0) + 1, 0);
-        for (int i = 0; i < n; ++i)
-            if (Z[i] >= 1 && Z[i] < (int)c.has_Z.size()) c.has_Z[Z[i]] = 1;
+        // (before mse_set_parameterisation any number is binned; require_elements refuses it later)
+        const int most_Z = std::max(e->max_Z, 255);
+        c.has_Z.assign((size_t)most_Z + 1, 0);
+        for (int i = 0; i < n; ++i) c.has_Z[Z[i] >= 1 && Z[i] <= most_Z ? Z[i] : 0] = 1;
         ++c.version;
         c.sorted = true;
     });
@@ -1238,6 +1239,8 @@ void require_elements(const mse_engine* e, const ConfigData& c) {
     // the potential kernels read per-element rows of the parameterisation (and its tables)
     // by atomic number: a configuration sorted under a larger parameterisation must not reach
     // past the current one
+    REQUIRE(c.has_Z.empty() || !c.has_Z[0], MSE_ERR_STATE,
+            "the configuration holds atomic numbers that no parameterisation has (it was sorted before one was set)");
     for (size_t Z = (size_t)std::max(e->max_Z, 0) + 1; Z < c.has_Z.size(); ++Z)
         REQUIRE(!c.has_Z[Z], MSE_ERR_STATE,
                 "the configuration holds atomic numbers beyond the current parameterisation "

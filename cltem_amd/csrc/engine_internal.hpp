@@ -133,7 +133,7 @@ struct ConfigData {
     unsigned version = 0;   // bumped whenever the atoms or transmission functions change
     double ref_off[2] = {0.0, 0.0};  // potential grid origin shift (source-size incoherence)
     int n_in_range = 0;
-    std::vector<unsigned char> has_Z;  // atomic numbers present in the last sort (index Z)
+    std::vector<unsigned char> has_Z;  // atomic numbers present in the last sort (index Z; 0: some that is none)
     bool sorted = false;
     DevBuf<float2> trans;  // n_slices * N
     bool built = false;     // trans holds the transmission functions of the current geometry
