@@ -56,7 +56,7 @@ struct HipStaging {
     using Event = hipEvent_t;
     // for the copies of every device
     static bool pin(unsigned char** p, size_t bytes) {
-        if (hipHostMalloc((void**)p, bytes, hipHostMallocPortable) == hipSuccess) return true;
+        if (hipHostMalloc((void**)p, bytes, hipHostMallocPortable | hipHostMallocCoherent) == hipSuccess) return true;
         (void)hipGetLastError();
         *p = nullptr;
         return false;
